@@ -43,7 +43,7 @@ void* workspace(monte_ctx* c, int slot, size_t bytes) {
 namespace {
 
 constexpr int kSlotFwd = 0, kSlotAdj = 1, kSlotMc = 2, kSlotConst = 3, kSlotStageA = 4, kSlotStageB = 5,
-              kSlotTuneA = 6, kSlotTuneB = 7, kSlotVolT = 8, kSlotQuad = 9,
+              kSlotTuneA = 6, kSlotTuneB = 7, kSlotVolT = 8,
               kSlotPlan = 10, kSlotE2E = 11, kSlotRay = 12, kSlotE2ERay = 13;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -203,13 +203,11 @@ int run_backproject_padded(monte_ctx* c, const monte_geom& g, const float* pad, 
     MONTE_HIP(c, launch_fill(vol, 0.f, vol_elems(g), c->stream));
     accumulate = 1;  // ROI columns added onto zeros
   }
-  float4* quads = (float4*)workspace(c, kSlotQuad, padded_elems(g) * sizeof(float4));
-  if (!quads) return fail(c, MONTE_ERR_NOMEM, "tap quad allocation failed");
-  MONTE_HIP(c, launch_tap_quads(pad, quads, g.n_views, grid.rows, grid.pitch, c->stream));
+  const BpReach reach = compute_bp_reach(g, grid);
   const int chunk = c->tuning.bp_view_chunk > 0 ? c->tuning.bp_view_chunk : g.n_views;
   for (int v0 = 0; v0 < g.n_views; v0 += chunk) {
     const int n = std::min(chunk, g.n_views - v0);
-    MONTE_HIP(c, launch_backproject(quads, views, v0, n, grid, vol, (accumulate || v0 > 0) ? 1 : 0, c->tuning,
+    MONTE_HIP(c, launch_backproject(pad, views, v0, n, grid, reach, vol, (accumulate || v0 > 0) ? 1 : 0, c->tuning,
                                     c->stream));
   }
   return MONTE_OK;
@@ -673,8 +671,8 @@ monte_tuning default_tuning() {
   t.mc_batch = 64;
   t.mc_blocks_per_cu = 6;
   t.bp_zchunk = 16;
-  t.bp_tile_x = 8;   // fastest at 325^3 / 512^2 / 360 views
-  t.bp_tile_y = 32;
+  t.bp_tile_x = 16;  // square tiles have the smallest patches on the detector
+  t.bp_tile_y = 16;
   t.bp_view_chunk = 0;
   t.pj_zchunk = 0;
   t.mc_ray_brick = 4;  // 2.45 Woodcock steps per history at 325^3 / 512^2 (7.56 with the global majorant)
@@ -1284,12 +1282,13 @@ int monte_autotune(monte_ctx* c, int what, const monte_geom* g, const monte_phan
     const float* taps;
     const BpView* views;
     if ((rc = ensure_constants(c, tg, &taps, &views))) return rc;
-    const int nviews = std::min(g->n_views, 360);  // L2 reuse across views shapes the best tile
-    float4* quads = (float4*)workspace(c, kSlotQuad, padded_elems(tg) * sizeof(float4));
+    const int nviews = g->n_views;  // the whole scan: orbits of four views need it
+    float* pad = (float*)workspace(c, kSlotFwd, padded_elems(tg) * sizeof(float));
     float* vol = (float*)workspace(c, kSlotTuneB, vol_elems(tg) * sizeof(float));
-    if (!quads || !vol) return fail(c, MONTE_ERR_NOMEM, "tuning buffers");
-    MONTE_HIP(c, launch_fill((float*)quads, 0.f, 4 * padded_elems(tg), c->stream));
+    if (!pad || !vol) return fail(c, MONTE_ERR_NOMEM, "tuning buffers");
+    MONTE_HIP(c, launch_fill(pad, 0.f, padded_elems(tg), c->stream));
     const BpGrid grid = compute_bp_grid(tg);
+    const BpReach reach = compute_bp_reach(tg, grid);
     hipEvent_t e0, e1;
     MONTE_HIP(c, hipEventCreate(&e0));
     MONTE_HIP(c, hipEventCreate(&e1));
@@ -1302,9 +1301,9 @@ int monte_autotune(monte_ctx* c, int what, const monte_geom* g, const monte_phan
         t.bp_zchunk = zc;
         t.bp_tile_x = tx;
         t.bp_tile_y = 256 / tx;
-        MONTE_HIP(c, launch_backproject(quads, views, 0, nviews, grid, vol, 0, t, c->stream));  // warm
+        MONTE_HIP(c, launch_backproject(pad, views, 0, nviews, grid, reach, vol, 0, t, c->stream));  // warm
         MONTE_HIP(c, hipEventRecord(e0, c->stream));
-        MONTE_HIP(c, launch_backproject(quads, views, 0, nviews, grid, vol, 0, t, c->stream));
+        MONTE_HIP(c, launch_backproject(pad, views, 0, nviews, grid, reach, vol, 0, t, c->stream));
         MONTE_HIP(c, hipEventRecord(e1, c->stream));
         MONTE_HIP(c, hipEventSynchronize(e1));
         float ms = 0.f;
@@ -1383,9 +1382,7 @@ int monte_fdk_graph(monte_ctx* c, const monte_geom* g, const float* proj, float*
   if ((rc = ensure_constants(c, *g, &taps, &views))) return rc;
   float* pad = (float*)workspace(c, kSlotFwd, padded_elems(*g) * sizeof(float));
   if (!pad) return fail(c, MONTE_ERR_NOMEM, "filtered stack allocation failed");
-  if (!workspace(c, kSlotQuad, padded_elems(*g) * sizeof(float4))) return fail(c, MONTE_ERR_NOMEM, "tap quad allocation failed");
   key.push_back((double)(uintptr_t)pad);
-  key.push_back((double)(uintptr_t)c->ws[kSlotQuad]);
   key.push_back((double)(uintptr_t)c->ws[kSlotConst]);
   if (key != c->graph_key || !c->graph_exec) {
     if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
@@ -1456,7 +1453,6 @@ int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, c
   const uint32_t *plan_offs, *plan_list;
   if ((rc = ensure_projector_plan(c, *g, views, grid, &plan_offs, &plan_list))) return rc;
   if (!workspace(c, kSlotFwd, padded_elems(*g) * sizeof(float)) ||
-      !workspace(c, kSlotQuad, padded_elems(*g) * sizeof(float4)) ||
       !workspace(c, kSlotAdj, padded_elems(*g) * sizeof(float)) ||
       !workspace(c, kSlotVolT, vol_elems(*g) * sizeof(float)))
     return fail(c, MONTE_ERR_NOMEM, "end-to-end workspace allocation failed");
@@ -1468,7 +1464,7 @@ int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, c
     std::vector<double> key = mkey;
     const void* ptrs[] = {b.primary, b.scatter, b.lineint, b.vol, b.vol_ref, b.residual, b.grad, b.loss};
     for (const void* p : ptrs) key.push_back((double)(uintptr_t)p);
-    for (int slot : {kSlotFwd, kSlotQuad, kSlotAdj, kSlotVolT, kSlotPlan, kSlotConst, kSlotE2E, kSlotE2ERay})
+    for (int slot : {kSlotFwd, kSlotAdj, kSlotVolT, kSlotPlan, kSlotConst, kSlotE2E, kSlotE2ERay})
       key.push_back((double)(uintptr_t)c->ws[slot]);
     const monte_tuning& t = c->tuning;
     for (double v : {(double)t.bp_zchunk, (double)t.bp_tile_x, (double)t.bp_view_chunk, (double)t.pj_zchunk})

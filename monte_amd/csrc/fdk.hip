@@ -8,12 +8,16 @@
 //   filter:  one block per (view, 16 detector columns); the weighted input
 //            tile is transposed through LDS and every thread keeps a 4 x NB
 //            register tile of outputs, so each LDS tap feeds 4 FMAs.
-//   backprojection: one thread per voxel column (x,y) and ZC voxels along z.
-//            Along a column u, the distance weight and the v-slope are
-//            constant, so per voxel-update only v moves (one FMA) before a
-//            4-tap bilinear gather from the zero-padded filtered view.  Tiles
-//            are ordered so each XCD owns a contiguous z-slab (its L2 then
-//            holds only the detector rows that slab projects to).
+//   backprojection: one thread per voxel column (x,y), or per orbit of columns
+//            that a part of a turn maps onto each other, and ZC voxels along z.
+//            Along a column u, the distance weight and the v-slope are constant,
+//            so per voxel-update only v moves (one integer add) before the four
+//            bilinear taps are read from the view's patch in LDS.  Tiles are
+//            ordered so each XCD owns a contiguous z-slab (its L2 then holds
+//            only the detector rows that slab projects to).
+#include <algorithm>
+#include <cmath>
+
 #include "internal.h"
 
 namespace monte {
@@ -386,6 +390,21 @@ __device__ inline int xcd_tile(int b, int nblocks) {
 }
 
 
+// 1 / U and wn / dd to about an ulp: a hardware estimate and Newton steps, a
+// third of the instructions of the correctly rounded divisions.
+__device__ inline double recip64(double u) {
+  double y = __builtin_amdgcn_rcp(u);
+  y = fma(y, fma(-u, y, 1.0), y);
+  return fma(y, fma(-u, y, 1.0), y);
+}
+
+// floor as an integer in one instruction (v_floor + v_cvt otherwise)
+__device__ inline int floor_i(float f) {
+  int r;
+  asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(f));
+  return r;
+}
+
 // Per-column quantities of one view, shared by the backprojector and its
 // transpose so both evaluate bit-identical weights.
 struct ColumnCore {
@@ -397,10 +416,12 @@ struct ColumnCore {
   float dsv;    // sv increment per voxel step along z
 };
 
+// STANDARD: the view's distance weight has no signed term (BpView's g and h are 0).
+template <bool STANDARD = false>
 __device__ inline ColumnCore column_core(const BpView& c, double X, double Y, float Xf, float Yf, const BpGrid& g) {
   ColumnCore r;
   const double U = fma(c.cx, X, fma(c.cy, Y, c.c0));
-  const double inv = 1.0 / U;
+  const double inv = recip64(U);
   double su = fma(c.suk * fma(c.ax, X, c.ay * Y), inv, c.su0);
   r.ok = su >= g.lo_u && su <= g.hi_u;
   su = fmin(fmax(su, g.lo_u), g.hi_u);
@@ -410,60 +431,66 @@ __device__ inline ColumnCore column_core(const BpView& c, double X, double Y, fl
   r.kv = c.svk * inv;
   r.dsv = (float)(r.kv * g.gsz);
   // sign test in unfused FP64 (as recon/bp3d20_325.cpp:145,151 evaluates it)
-  const double gp = xadd(xmul(X, c.gx), xmul(Y, c.gy));
-  const float hp = fabsf(fmaf(c.hx, Xf, c.hy * Yf));
-  const float dd = fmaf(c.dx, Xf, fmaf(c.dy, Yf, c.d0)) - (gp < 0.0 ? -hp : hp);
-  const float q = c.wn / dd;
+  float dd = fmaf(c.dx, Xf, fmaf(c.dy, Yf, c.d0));
+  if (!STANDARD) {
+    const double gp = xadd(xmul(X, c.gx), xmul(Y, c.gy));
+    const float hp = fabsf(fmaf(c.hx, Xf, c.hy * Yf));
+    dd -= gp < 0.0 ? -hp : hp;
+  }
+  float rd = __builtin_amdgcn_rcpf(dd);
+  rd = fmaf(rd, fmaf(-dd, rd, 1.0f), rd);
+  const float q = c.wn * rd;
   r.w = c.fac * q * q;
   return r;
 }
 
-// v coordinate at a 16-aligned base voxel: integer part and FP32 fraction.
-struct ChunkBase {
-  int ivb;
-  float fvb;
-  float flo, fhi;  // v window relative to ivb
-};
-
-// The v coordinate of voxel z is formed from a base taken at the 16-aligned z
-// at or below it (zb), whatever the thread's z-chunk, so every chunking and
-// tile shape evaluates the same floating-point expression for each voxel and
-// the volume is bitwise independent of the launch tuning.
+// The v coordinate of voxel z is formed from a base taken in the middle of its
+// 16-aligned group, whatever the thread's z-chunk, so every chunking and tile
+// shape evaluates the same floating-point expression for each voxel and the
+// volume is bitwise independent of the launch tuning.
 constexpr int kZBase = 16;
+constexpr int kZMid = kZBase / 2;  // the base voxel of a group of 16: dsv's rounding is multiplied by 8 at most
 
 __device__ inline double base_z(const BpGrid& g, int zb) {
   // recon/bp3d20_325.cpp:109 forms the coordinate as start - index * step, unfused
   return xadd(g.gz0, xmul((double)zb, g.gsz));
 }
 
-__device__ inline ChunkBase chunk_base(const ColumnCore& cc, const BpView& c, double Zb, const BpGrid& g) {
-  ChunkBase b;
+// The v coordinates of a group's voxels in the column's view: row ivb of the
+// base voxel, and in fixed point of kVBits fraction bits, relative to that row,
+// the base voxel's coordinate, the step per voxel and the window.  Integers add
+// without rounding, so a coordinate is within 2^-(kVBits + 1) rows x 9 of the
+// FP64 line; as FP32 multiply-adds of the step they were 2^-21 off (|f| up to 16).
+// Voxels of a tile that fits in LDS (at most 62 rows, 16 voxels) step by less
+// than 4.1 rows, so a group stays within +-33 rows of its base.
+constexpr int kVBits = 25;
+struct GroupV {
+  int ivb;
+  int f, d;        // base coordinate and step
+  int flo, fhi;    // window, clamped to +-63 rows
+};
+
+__device__ inline GroupV group_v(const ColumnCore& cc, const BpView& c, double Zb, const BpGrid& g) {
+  constexpr double one = (double)(1 << kVBits);
+  GroupV b;
   double sv = fma(cc.kv, Zb, c.sv0);
-  sv = fmin(fmax(sv, -1.0e6), 1.0e6);
+  // (a group whose base lies 40 rows outside the window lies outside as a whole)
+  sv = fmin(fmax(sv, g.lo_v - 40.0), g.hi_v + 40.0);
   const double fv0 = floor(sv);
   b.ivb = (int)fv0;
-  b.fvb = (float)(sv - fv0);
-  b.flo = (float)(g.lo_v - fv0);
-  b.fhi = (float)(g.hi_v - fv0);
+  b.f = (int)rint((sv - fv0) * one);
+  b.d = (int)rint(cc.kv * g.gsz * one);
+  b.flo = (int)(fmin(fmax(g.lo_v - fv0, -63.0), 63.0) * one);
+  b.fhi = (int)(fmin(fmax(g.hi_v - fv0, -63.0), 63.0) * one);
   return b;
 }
 
-// Sample position of voxel zb + j, as the byte offset of its tap quad in the
-// view (`off0` is that of row ivb, column iu; rows are `prow` bytes apart) and
-// the row fraction; false when the sample lies outside the v window.  The
-// clamped coordinate equals the unclamped one exactly when it is inside, so
-// one compare gives the window test.  |floor(f)| < 2^23 (sv is clamped to
-// +-1e6 and the window is a few thousand rows) and prow < 2^23, so a 24-bit
-// multiply forms the row step; the sum is taken mod 2^32 and the true offset
-// lies inside the view.
-__device__ inline bool chunk_tap(const ColumnCore& cc, const ChunkBase& b, int j, uint32_t off0, uint32_t prow,
-                                 uint32_t& off, float& fv) {
-  const float f = fmaf((float)j, cc.dsv, b.fvb);
-  const float fc = fminf(fmaxf(f, b.flo), b.fhi);
-  const float fl = floorf(fc);
-  fv = fc - fl;
-  off = off0 + (uint32_t)__mul24((int)fl, (int)prow);
-  return fc == f;
+// Whether voxel z's sample lies in the v window, edges included.  Decided on the
+// FP64 line: in the bp3d20 preset samples fall on an edge exactly (rational
+// geometry), and the reference's FP64 comparison decides whether they count.
+__device__ inline bool in_window(const ColumnCore& cc, const BpView& c, const BpGrid& g, int z) {
+  const double sv = fma(cc.kv, base_z(g, z), c.sv0);
+  return sv >= g.lo_v && sv <= g.hi_v;
 }
 
 __device__ inline bool in_mask(const BpGrid& g, int x, int y, int z) {
@@ -476,124 +503,445 @@ __device__ inline bool in_mask(const BpGrid& g, int x, int y, int z) {
 __device__ inline double voxel_x(const BpGrid& g, int x) { return xadd(g.gx0, xmul((double)x, g.gsx)); }
 __device__ inline double voxel_y(const BpGrid& g, int y) { return xadd(g.gy0, xmul((double)y, g.gsy)); }
 
-template <int ZC>
-__global__ __launch_bounds__(256) void backproject_kernel(const float4* __restrict__ quads,
-                                                          const BpView* __restrict__ views, int view0, int nviews,
-                                                          BpGrid g, float* __restrict__ vol, int accumulate,
-                                                          int tile_x, int tiles_x, int tiles_y) {
+// The backprojector reads its bilinear taps from LDS.  A block owns a tile of
+// 256 voxel columns over ZC voxels of z; in one view that tile projects to a
+// small patch of the detector (25 x 22 cells at 325^3 / 512^2), which the block
+// copies into LDS with coalesced loads while it works on the view before.
+// What bounds it: taps gathered from global memory cost 16.4 clocks per wave and
+// load whatever lies in cache (8- and 16-byte gathers alike, 5.4 for 4 bytes),
+// against 3.3 for a pair of words from LDS, so the gathers were the floor of the
+// kernel this one replaced (6.83 ms at 325^3 / 512^2 / 360 views, 21.7 clocks
+// per wave update, and 0.36 ms to write the four taps of every cell side by side,
+// 1.5 GB; 3.8 ms now: the VALU issues 89% of the time and LDS reads take 83%).
+//
+// NQ > 1: a scan of a full turn in V views, of a volume that 1/NQ of a turn maps
+// onto itself, sees voxel column c in view k exactly as it sees c turned by q/NQ
+// in view k + q V / NQ: NQ = 4 for square volumes and V a multiple of 4, NQ = 2
+// for any volume about the axis and V even.  A thread then owns the NQ columns of
+// one orbit: it forms the sample coordinates and weights of its first column once
+// per view and applies them to the patches of NQ views, one per column.  VALU
+// instructions per update: 10 / NQ of geometry and 5 of taps (NQ = 1: 13 in all,
+// by interpolating u, v in turn), and about 70 per column and view.
+//
+// ZEROS: the guard cells around the views are zeros (standard preset), so a
+// sample clamped to the window's edge reads zeros and needs no mask.
+//
+// LDS cell (r, q, c) of a patch is at r kRS + q kCols + c: a wave's copy
+// instruction fills 64 words in a row (straight from memory to LDS), one row of
+// one view (of two views for NQ = 4); the row pitch kRS spreads neighbouring rows
+// over different banks (16 mod 64), and keeps every tap of the four patches
+// within one instruction's offsets of a single address (144 + 3 * 32 + 1 < 256).
+template <int NQ>
+struct PatchLayout {
+  static constexpr int kCols = NQ == 4 ? 32 : 64;
+  static constexpr int kRS = NQ == 1 ? 80 : 144;
+  static constexpr int kMaxRows = NQ == 4 ? 34 : (NQ == 2 ? 45 : 62);  // two patches in 39 to 52 KB of LDS
+};
+
+// One dword per lane from `row` + off (bytes) to 64 consecutive words of LDS, all
+// three wave-uniform but off.  Written as an instruction because the compiler
+// cannot tell the two patches apart and would wait for the copies of one
+// before it reads the other; there is no result register, and the caller waits
+// (vmcnt) and meets the other waves before anything reads the words.
+__device__ inline void copy_to_lds(const char* row, uint32_t off, float* dst) {
+  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)dst;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane((int)at)), "v"(off), "s"(row)
+               : "memory");
+}
+
+// min(max(x, lo), hi) in one instruction
+__device__ inline int clamp_i(int x, int lo, int hi) {
+  int r;
+  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
+  return r;
+}
+
+constexpr float kFracUnit = 2.3283064365386963e-10f;  // 2^-32
+// A voxel's bilinear taps in the patches of its orbit.
+template <int NQ>
+struct Taps {
+  float p[NQ][4];
+  float fv;   // row fraction
+  bool live;  // inside the v window and the mask
+};
+
+constexpr int kRegionViews = 32;  // views whose patch origins are found at a time
+
+template <int ZC, int NQ, bool ZEROS>
+__global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __restrict__ pad,
+                                                             const BpView* __restrict__ views, int view0,
+                                                             int nviews, BpGrid g, float* __restrict__ vol,
+                                                             int accumulate, int tile_x, int tiles_x, int tiles_y,
+                                                             int patch_rows, int turn) {
+  using L = PatchLayout<NQ>;
+  extern __shared__ float patch[];  // two patches of patch_rows rows, one read while the other is filled
+  __shared__ int2 region[2][kRegionViews];
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int per_z = tiles_x * tiles_y;
   const int zc = t / per_z;
   const int rem = t - zc * per_z;
   const int ty_t = rem / tiles_x, tx_t = rem - ty_t * tiles_x;
   const int tile_y = 256 / tile_x;
-  const int x = g.x0 + tx_t * tile_x + (int)(threadIdx.x % tile_x);
-  const int y = ty_t * tile_y + (int)(threadIdx.x / tile_x);
+  const int tid = threadIdx.x;
+  // columns up to (xb, yb) are owned: all of them, or the first quadrant or half of the orbits
+  const int xb = NQ == 4 ? (g.nx + 1) / 2 : g.x1, yb = NQ > 1 ? (g.ny + 1) / 2 : g.ny;
+  const int tx0 = (NQ > 1 ? 0 : g.x0) + tx_t * tile_x, ty0 = ty_t * tile_y;
+  // a wave takes 8 x 8 columns of the tile: the smallest patch, so its taps share
+  // words and fewer rows of them meet in one bank
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wx = tile_x / 8;
+  const int xw = tx0 + wave % wx * 8, yw = ty0 + wave / wx * 8;
+  const bool idle = xw >= xb || yw >= yb;  // (a wave past the edge only copies)
+  const int x = min(xw + lane % 8, xb - 1), y = min(yw + lane / 8, yb - 1);  // (past the end: repeats a column, never stored)
   const int z0 = zc * ZC;
-  if (x >= g.x1 || y >= g.ny) return;
-  const int zb = (z0 / kZBase) * kZBase, joff = z0 - zb;
-  const double X = voxel_x(g, x), Y = voxel_y(g, y), Zb = base_z(g, zb);
-  const float Xf = (float)X, Yf = (float)Y;
-  bool live[ZC];
+  const int zb = (z0 / kZBase) * kZBase, joff = z0 - zb - kZMid;
+  const int patch_words = patch_rows * L::kRS;
+  const int part = g.n_views / NQ;  // views of 1/NQ of a turn
+
+  // Patch origin (row, column of the padded view) of views [first, first + 32):
+  // the sample coordinates are monotonic along any line of the tile, so their
+  // minima lie at its corners.  8 lanes per view evaluate the 8 corners.
+  auto find_regions = [&](int first) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // (opaque: the corners are formed here, not kept in registers over the views)
+    const int k = min(first + (tid >> 3), view0 + nviews - 1);
+    const BpView& c = views[k];
+    const double Xc = voxel_x(g, (tid & 1) ? min(tx0 + tile_x, xb) - 1 : tx0);
+    const double Yc = voxel_y(g, (tid & 2) ? min(ty0 + tile_y, yb) - 1 : ty0);
+    const double Zc = base_z(g, (tid & 4) ? z0 + ZC - 1 : z0);
+    const double inv = recip64(fma(c.cx, Xc, fma(c.cy, Yc, c.c0)));
+    const double su = fma(c.suk * fma(c.ax, Xc, c.ay * Yc), inv, c.su0), sv = fma(c.svk * inv, Zc, c.sv0);
+    float u = (float)fmin(fmax(su, g.lo_u), g.hi_u), v = (float)fmin(fmax(sv, g.lo_v), g.hi_v);
 #pragma unroll
-  for (int j = 0; j < ZC; ++j) live[j] = (z0 + j) < g.nz && in_mask(g, x, y, z0 + j);
+    for (int o = 1; o < 8; o <<= 1) {
+      u = fminf(u, __shfl_xor(u, o, 64));
+      v = fminf(v, __shfl_xor(v, o, 64));
+    }
+    // (0.01: the voxels' own coordinates round differently)
+    if ((tid & 7) == 0)
+      region[((first - view0) / kRegionViews) & 1][tid >> 3] =
+          make_int2(max(floor_i(v - 0.01f) + kPadLo, 0), max(floor_i(u - 0.01f) + kPadLo, 0));
+  };
+
+  // Copies view k's patch, or the patches of views k + q V / NQ mod V: wave w
+  // takes rows w, w + 4, ...; lane l column l % kCols.  Rows and columns past the
+  // padded view repeat its last ones; no tap reads them.
+  const uint32_t view_bytes = (uint32_t)g.rows * (uint32_t)g.pitch * 4u;
+  auto copy = [&](int k, float* buf) {
+    const int2 o = region[((k - view0) / kRegionViews) & 1][(k - view0) % kRegionViews];
+    const int r0 = __builtin_amdgcn_readfirstlane(o.x), c0 = __builtin_amdgcn_readfirstlane(o.y);
+    const uint32_t col = (uint32_t)min(c0 + lane % L::kCols, g.pitch - 1) * 4u;
+    const int kq = NQ > 1 ? k % part : k, turned = NQ > 1 ? k / part : 0;
+    const char* src = (const char*)pad + (size_t)kq * view_bytes;
+#pragma unroll
+    for (int h = 0; h < (NQ > 1 ? 2 : 1); ++h) {
+      // patch q holds view (k + q part) mod V = k mod part + ((q + turned) mod NQ) part
+      const uint32_t q = (uint32_t)(h * (64 / L::kCols) + lane / L::kCols);
+      const uint32_t off = col + (NQ > 1 ? ((q + turned) & (NQ - 1u)) * (uint32_t)part * view_bytes : 0u);
+      for (int r = wave; r < patch_rows; r += 4) {
+        const char* row = src + (uint32_t)min(r0 + r, g.rows - 1) * (uint32_t)g.pitch * 4u;
+        copy_to_lds(row, off, buf + r * L::kRS + h * 64);
+      }
+    }
+  };
+
+  float acc[NQ][ZC];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int j = 0; j < ZC; ++j) acc[q][j] = 0.f;
+
+  find_regions(view0);
+  __syncthreads();
+  copy(view0, patch);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the copies are in LDS
+  __syncthreads();
+  for (int i = 0; i < nviews; ++i) {
+    const int k = view0 + i;
+    const bool more = i + 1 < nviews;
+    if (more) copy(k + 1, patch + ((i + 1) & 1) * patch_words);
+    // the next batch of origins, half a batch ahead of its first use
+    if (i % kRegionViews == kRegionViews / 2 && i + kRegionViews / 2 < nviews)
+      find_regions(k + kRegionViews / 2);
+    if (!idle) {
+      const BpView& c = views[k];
+      int xc = x, yc = y;
+      asm volatile("" : "+v"(xc), "+v"(yc));  // (two registers kept over the views instead of four)
+      const double X = voxel_x(g, xc), Y = voxel_y(g, yc);
+      const ColumnCore cc = column_core<ZEROS>(c, X, Y, (float)X, (float)Y, g);
+      const int2 o = region[(i / kRegionViews) & 1][i % kRegionViews];
+      const float wu = ZEROS || cc.ok ? cc.w : 0.f;
+      const float w1 = wu * cc.fu, w0 = wu - w1;
+      // The reads of one voxel are issued before the sums of the voxel before it
+      // (left to itself the compiler saves registers and waits for each pair of
+      // words: 6.6 against 4.8 ms for the FDK at 325^3 / 512^2 / 360 views).
+      GroupV cb;
+      int base = 0;
+      auto taps_of = [&](int j) {
+        if (j % kZBase == 0) {
+          cb = group_v(cc, c, base_z(g, zb + j + kZMid), g);
+          base = (i & 1) * patch_words + (cb.ivb + kPadLo - o.x) * L::kRS + (cc.iu + kPadLo - o.y);
+          asm volatile("" : "+v"(base));  // (keeps the constants out of the reads' offsets, which the taps need)
+        }
+        const int f = cb.f + (joff + j % kZBase) * cb.d;
+        const int fc = clamp_i(f, cb.flo, cb.fhi);
+        const float* s = patch + (base + __mul24(fc >> kVBits, L::kRS));
+        Taps<NQ> t;
+        t.fv = kFracUnit * (float)((uint32_t)fc << (32 - kVBits));
+        t.live = ZEROS || (in_window(cc, c, g, z0 + j) && in_mask(g, x, y, z0 + j));
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const float* sq = s + q * L::kCols;
+          t.p[q][0] = sq[0];
+          t.p[q][1] = sq[1];
+          t.p[q][2] = sq[L::kRS];
+          t.p[q][3] = sq[L::kRS + 1];
+        }
+        return t;
+      };
+      Taps<NQ> cur = taps_of(0);
+#pragma unroll
+      for (int j = 0; j < ZC; ++j) {
+        const Taps<NQ> t = cur;
+        if (j + 1 < ZC) cur = taps_of(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (NQ == 1) {
+          const float a = fmaf(cc.fu, t.p[0][1] - t.p[0][0], t.p[0][0]);
+          const float b = fmaf(cc.fu, t.p[0][3] - t.p[0][2], t.p[0][2]);
+          acc[0][j] = fmaf(t.live ? wu : 0.f, fmaf(t.fv, b - a, a), acc[0][j]);
+        } else {
+          const float b0 = w0 * t.fv, b1 = w1 * t.fv, a0 = w0 - b0, a1 = w1 - b1;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) {
+            float val = a0 * t.p[q][0];
+            val = fmaf(a1, t.p[q][1], val);
+            val = fmaf(b0, t.p[q][2], val);
+            val = fmaf(b1, t.p[q][3], val);
+            acc[q][j] += val;
+          }
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    __syncthreads();
+  }
+  // (the lane's column again: kept over the views it would cost registers)
+  int tl = threadIdx.x;
+  asm volatile("" : "+v"(tl));
+  const int xs = xw + tl % 8, ys = yw + (tl & 63) / 8;
+  if (xs >= xb || ys >= yb) return;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    int xq = xs, yq = ys;
+    // an odd volume's middle row holds whole orbits (half turns), or turned middle
+    // columns and the centre (quarter turns): each voxel is stored once
+    if (NQ > 1 && 2 * ys + 1 == g.ny && (q > 0 || (NQ == 4 && 2 * xs + 1 != g.nx))) continue;
+    if (NQ > 1) {
+      const int m = NQ == 2 ? 2 * q : (turn > 0 ? q : (4 - q) & 3);  // quarter turns (x, y) -> (n - 1 - y, x)
+      xq = m == 0 ? xs : (m == 1 ? g.nx - 1 - ys : (m == 2 ? g.nx - 1 - xs : ys));
+      yq = m == 0 ? ys : (m == 1 ? xs : (m == 2 ? g.ny - 1 - ys : g.nx - 1 - xs));
+    }
+#pragma unroll
+    for (int j = 0; j < ZC; ++j) {
+      if (z0 + j >= g.nz) break;
+      float* o = vol + ((size_t)(z0 + j) * g.ny + yq) * g.nx + xq;
+      *o = accumulate ? *o + acc[q][j] : acc[q][j];
+    }
+  }
+}
+
+// Volumes too small to fill the chip with tiles, and voxels so coarse on the
+// detector that a tile's patch does not fit in LDS: taps straight from the
+// padded views (four 4-byte gathers, 21.7 clocks a wave, where two 8-byte ones
+// cost 32.7).  A wave takes 64 columns in a row (x fastest) over ZC voxels, and
+// the block's waves share the views out, so a small volume's chain of views is
+// short (one voxel takes the latency of a view's set-up and gathers after
+// another); their sums are added in wave order, so the volume does not depend
+// on scheduling.
+template <int ZC, bool ZEROS>
+__global__ __launch_bounds__(1024) void backproject_direct_kernel(const float* __restrict__ pad,
+                                                                  const BpView* __restrict__ views, int view0,
+                                                                  int nviews, BpGrid g, float* __restrict__ vol,
+                                                                  int accumulate, int col_blocks) {
+  extern __shared__ float part[];  // [waves][ZC][64]
+  const int cb_i = blockIdx.x % col_blocks, zc = blockIdx.x / col_blocks;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int ncx = g.x1 - g.x0, ncol = ncx * g.ny;
+  const int col = min(cb_i * 64 + lane, ncol - 1);
+  const int y = col / ncx, x = g.x0 + col - y * ncx;
+  const int z0 = zc * ZC;
+  const int zb = (z0 / kZBase) * kZBase, joff = z0 - zb - kZMid;
+  const double X = voxel_x(g, x), Y = voxel_y(g, y), Zb = base_z(g, zb + kZMid);
+  const float Xf = (float)X, Yf = (float)Y;
+  const size_t view_stride = (size_t)g.rows * g.pitch;
   float acc[ZC];
 #pragma unroll
   for (int j = 0; j < ZC; ++j) acc[j] = 0.f;
-
-  // One 16-byte load per voxel: the vector memory pipeline costs about the
-  // same per instruction whatever its width, so the four bilinear taps come
-  // from one tap quad rather than two 8-byte row pairs.
-  const size_t view_stride = (size_t)g.rows * g.pitch;
-  const uint32_t prow = (uint32_t)g.pitch * 16u;
-  for (int k = view0; k < view0 + nviews; ++k) {
+  const int ka = view0 + (int)((long)wave * nviews / waves), kb = view0 + (int)((long)(wave + 1) * nviews / waves);
+  for (int k = ka; k < kb; ++k) {
     const BpView& c = views[k];
-    const ColumnCore cc = column_core(c, X, Y, Xf, Yf, g);
-    const ChunkBase cb = chunk_base(cc, c, Zb, g);
-    const char* vb = (const char*)(quads + (size_t)k * view_stride);
-    const uint32_t off0 = (uint32_t)(cb.ivb + kPadLo) * prow + (uint32_t)(cc.iu + kPadLo) * 16u;
-    const float wu = cc.ok ? cc.w : 0.f;
+    const ColumnCore cc = column_core<ZEROS>(c, X, Y, Xf, Yf, g);
+    // v in 32.32 fixed point: any step per voxel
+    long long sv = __double2ll_rn(fmin(fmax(fma(cc.kv, Zb, c.sv0), -1.0e6), 1.0e6) * 4294967296.0);
+    const long long dv = __double2ll_rn(cc.kv * g.gsz * 4294967296.0);
+    const long long lo = (long long)g.lo_v << 32, hi = (long long)g.hi_v << 32;
+    const float* src = pad + (size_t)k * view_stride;
+    const uint32_t off0 = (uint32_t)(kPadLo * g.pitch + cc.iu + kPadLo);
+    sv += joff * dv;
+    const float wu = ZEROS || cc.ok ? cc.w : 0.f;
+    const float w1 = wu * cc.fu, w0 = wu - w1;
 #pragma unroll
     for (int j = 0; j < ZC; ++j) {
-      uint32_t off;
-      float fv;
-      const bool okv = chunk_tap(cc, cb, joff + j, off0, prow, off, fv);
-      const float4 t = *(const float4*)(vb + off);
-      const float a = fmaf(cc.fu, t.y, t.x);
-      const float b = fmaf(cc.fu, t.w, t.z);
-      const float val = fmaf(fv, b - a, a);
-      acc[j] = fmaf((okv && live[j]) ? wu : 0.f, val, acc[j]);
+      const bool live = ZEROS || (in_window(cc, c, g, z0 + j) && in_mask(g, x, y, z0 + j));
+      const long long sc = sv < lo ? lo : (sv > hi ? hi : sv);
+      const float fv = (float)(uint32_t)sc * 2.3283064365386963e-10f;  // 2^-32
+      const float m0 = live ? w0 : 0.f, m1 = live ? w1 : 0.f;
+      const float b0 = m0 * fv, b1 = m1 * fv;
+      const uint32_t at = off0 + (uint32_t)__mul24((int)(sc >> 32), g.pitch);
+      sv += dv;
+      float val = (m0 - b0) * src[at];
+      val = fmaf(m1 - b1, src[at + 1], val);
+      val = fmaf(b0, src[at + (uint32_t)g.pitch], val);
+      val = fmaf(b1, src[at + (uint32_t)g.pitch + 1], val);
+      acc[j] += val;
     }
   }
 #pragma unroll
-  for (int j = 0; j < ZC; ++j) {
+  for (int j = 0; j < ZC; ++j) part[(wave * ZC + j) * 64 + lane] = acc[j];
+  __syncthreads();
+  const int own = cb_i * 64 + lane;
+  const int oy = own / ncx, ox = g.x0 + own - oy * ncx;
+  if (own >= ncol) return;
+  for (int j = wave; j < ZC; j += waves) {
     if (z0 + j >= g.nz) break;
-    float* o = vol + ((size_t)(z0 + j) * g.ny + y) * g.nx + x;
-    *o = accumulate ? *o + acc[j] : acc[j];
+    float sum = 0.f;
+    for (int w = 0; w < waves; ++w) sum += part[(w * ZC + j) * 64 + lane];
+    float* o = vol + ((size_t)(z0 + j) * g.ny + oy) * g.nx + ox;
+    *o = accumulate ? *o + sum : sum;
   }
 }
 
-static void bp_tiling(const BpGrid& grid, const monte_tuning& t, int zc, int& tile_x, int& tiles_x, int& tiles_y,
-                      long& nblocks) {
-  tile_x = t.bp_tile_x > 0 ? t.bp_tile_x : 16;
-  const int tile_y = 256 / tile_x;
-  const int ncols = grid.x1 - grid.x0;
-  tiles_x = (ncols + tile_x - 1) / tile_x;
-  tiles_y = (grid.ny + tile_y - 1) / tile_y;
-  const int zchunks = (grid.nz + zc - 1) / zc;
-  nblocks = (long)tiles_x * tiles_y * zchunks;
+// Bounds on the patch of a tile of tile_x x tile_y columns and zc voxels: rows
+// and columns of the detector it can touch in any view, taps included.  su and
+// sv move by at most |suk| s and |svk| s per unit of length across the tile,
+// s = sqrt(U^2 + y'^2) / U^2 for su (largest on the circle through the volume's
+// farthest corner), 1 / U along z and |Z| / U^2 across for sv.
+static void patch_bounds(const BpGrid& g, const BpReach& r, int tile_x, int tile_y, int zc, int& rows, int& cols) {
+  const double dx = (tile_x - 1) * std::fabs(g.gsx), dy = (tile_y - 1) * std::fabs(g.gsy);
+  const double diag = std::sqrt(dx * dx + dy * dy);
+  double c = -(r.sod * r.sod + 2.0 * r.rad * r.rad) / (3.0 * r.sod * std::max(r.rad, 1e-30));
+  c = std::min(1.0, std::max(-1.0, c));
+  const double U = r.sod + r.rad * c, s = std::sqrt(r.sod * r.sod + 2.0 * r.sod * r.rad * c + r.rad * r.rad) / (U * U);
+  const double um = r.sod - r.rad;
+  const double zs = std::fabs(g.gsz);
+  const double zmax = std::max(std::fabs(g.gz0), std::fabs(g.gz0 + (g.nz + zc) * g.gsz));
+  const double wu = r.suk * s * diag, wv = r.svk * ((zc - 1) * zs / um + zmax * diag / (um * um));
+  // floor of the two ends' difference, the 0.01 margin of the origin, and the tap above
+  cols = wu < 1e6 ? (int)std::floor(wu + 0.03) + 3 : 1 << 20;
+  rows = wv < 1e6 ? (int)std::floor(wv + 0.03) + 3 : 1 << 20;
 }
 
-// quads [view][rows][pitch]: quad (r, c) = (p[r][c], p[r][c + 1] - p[r][c], p[r + 1][c],
-// p[r + 1][c + 1] - p[r + 1][c]) of the padded filtered view p (zero past the last
-// row or column): the two rows of a voxel's bilinear taps with their u
-// differences, which the backprojector would otherwise form per voxel.
-// One thread per padded cell: blocks of 64 columns x 4 rows, one grid layer
-// per view, so the cell's view, row and column need no division.
-constexpr int kQuadCols = 64, kQuadRows = 4;
-__global__ __launch_bounds__(kQuadCols * kQuadRows) void tap_quads_kernel(const float* __restrict__ pad,
-                                                                          float4* __restrict__ quads, int rows,
-                                                                          int pitch) {
-  const int cl = blockIdx.x * kQuadCols + (int)(threadIdx.x % kQuadCols);
-  const int r = blockIdx.y * kQuadRows + (int)(threadIdx.x / kQuadCols);
-  if (cl >= pitch || r >= rows) return;
-  const size_t i = ((size_t)blockIdx.z * rows + r) * pitch + cl;
-  const float* p = pad + i;
-  const bool rr = r + 1 < rows, cr = cl + 1 < pitch;
-  const float p00 = p[0], p01 = cr ? p[1] : 0.f;
-  const float p10 = rr ? p[pitch] : 0.f, p11 = (rr && cr) ? p[pitch + 1] : 0.f;
-  quads[i] = make_float4(p00, p01 - p00, p10, p11 - p10);
+// Which kernel takes a backprojection: a property of the scan alone (sizes of
+// the default tiling), so the volume does not depend on the tuned tile shape.
+//   4, 2 columns an orbit   1/4 or 1/2 of a turn maps the scan onto itself, the
+//                           patches fit, and at least 2 tiles per CU
+//   1 column                patches fit, and at least 2 tiles per CU
+//   0                       straight from memory
+// Fewer tiles leave the chip idle: 65^3 from 36 views (125 tiles) took 46 us as
+// tiles of the kernel before this one.
+template <int NQ>
+static bool patch_fits(int rows, int cols) { return cols <= PatchLayout<NQ>::kCols && rows <= PatchLayout<NQ>::kMaxRows; }
+
+static int bp_orbits(const BpGrid& g, const BpReach& r) {
+  int rows, cols;
+  patch_bounds(g, r, 16, 16, 16, rows, cols);
+  auto tiles = [&](int nx, int ny) { return (long)((nx + 15) / 16) * ((ny + 15) / 16) * ((g.nz + 15) / 16); };
+  // (the views' offsets from the first are 32-bit)
+  const bool near = (double)g.n_views * g.rows * g.pitch * 4.0 < 4294967296.0;
+  const int hx = (g.nx + 1) / 2, hy = (g.ny + 1) / 2;
+  if (near && r.turn != 0 && patch_fits<4>(rows, cols) && tiles(hx, hy) >= 512) return 4;
+  if (near && r.half && patch_fits<2>(rows, cols) && tiles(g.nx, hy) >= 512) return 2;
+  if (patch_fits<1>(rows, cols) && tiles(g.x1 - g.x0, g.ny) >= 512) return 1;
+  return 0;
 }
 
-hipError_t launch_tap_quads(const float* filt_pad, float4* quads, int n_views, int rows, int pitch, hipStream_t s) {
-  if (n_views <= 0 || rows <= 0 || pitch <= 0) return hipSuccess;
-  if (n_views > 65535) return hipErrorInvalidValue;  // grid z limit
-  const dim3 grid((unsigned)((pitch + kQuadCols - 1) / kQuadCols), (unsigned)((rows + kQuadRows - 1) / kQuadRows),
-                  (unsigned)n_views);
-  hipLaunchKernelGGL(tap_quads_kernel, grid, dim3(kQuadCols * kQuadRows), 0, s, filt_pad, quads, rows, pitch);
-  return hipGetLastError();
-}
-
-hipError_t launch_backproject(const float4* quads, const BpView* views, int view0, int nviews_chunk,
-                              const BpGrid& grid, float* vol, int accumulate, const monte_tuning& t,
-                              hipStream_t s) {
-  const int zc = t.bp_zchunk > 0 ? t.bp_zchunk : 8;
-  int tile_x, tiles_x, tiles_y;
-  long nblocks;
+hipError_t launch_backproject(const float* filt_pad, const BpView* views, int view0, int nviews_chunk,
+                              const BpGrid& grid, const BpReach& reach, float* vol, int accumulate,
+                              const monte_tuning& t, hipStream_t s) {
+  // taps are addressed by 32-bit offsets with a 24-bit row multiply
+  if (grid.pitch >= (1 << 23) || (long long)grid.rows * grid.pitch * 4 >= (1LL << 32)) return hipErrorInvalidValue;
   if (t.bp_tile_x > 0 && 256 % t.bp_tile_x) return hipErrorInvalidValue;
-  // quads are addressed by 32-bit byte offsets with a 24-bit row multiply
-  if ((long long)grid.pitch * 16 >= (1LL << 23) || (long long)grid.rows * grid.pitch * 16 >= (1LL << 32))
-    return hipErrorInvalidValue;
-  bp_tiling(grid, t, zc, tile_x, tiles_x, tiles_y, nblocks);
-  if (nblocks <= 0) return hipSuccess;
-  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
-  dim3 gd((unsigned)nblocks), bd(256);
-  switch (zc) {
-    case 4: hipLaunchKernelGGL((backproject_kernel<4>), gd, bd, 0, s, quads, views, view0, nviews_chunk, grid, vol, accumulate, tile_x, tiles_x, tiles_y); break;
-    case 8: hipLaunchKernelGGL((backproject_kernel<8>), gd, bd, 0, s, quads, views, view0, nviews_chunk, grid, vol, accumulate, tile_x, tiles_x, tiles_y); break;
-    case 16: hipLaunchKernelGGL((backproject_kernel<16>), gd, bd, 0, s, quads, views, view0, nviews_chunk, grid, vol, accumulate, tile_x, tiles_x, tiles_y); break;
-    default: return hipErrorInvalidValue;
+  int zc = t.bp_zchunk > 0 ? t.bp_zchunk : 16;
+  if (zc != 4 && zc != 8 && zc != 16) return hipErrorInvalidValue;
+  const int ncx = grid.x1 - grid.x0;
+  if (ncx <= 0 || grid.ny <= 0 || grid.nz <= 0 || nviews_chunk <= 0) return hipSuccess;
+  int nq = bp_orbits(grid, reach);
+  if (nq > 1 && nviews_chunk != grid.n_views) {  // orbits need the whole turn
+    int rows, cols;
+    patch_bounds(grid, reach, 16, 16, 16, rows, cols);
+    nq = patch_fits<1>(rows, cols) ? 1 : 0;
   }
+  if (nq == 0) {
+    // 8 voxels a lane, and waves per block until about 4 per SIMD are in flight
+    const long ncol = (long)ncx * grid.ny;
+    const int zd = 8;
+    const long cb = (ncol + 63) / 64, blocks = cb * ((grid.nz + zd - 1) / zd);
+    int waves = 1;
+    while (waves < 16 && blocks * waves < 4096 && 2 * waves < nviews_chunk) waves *= 2;
+    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+#define MONTE_BP(ZEROS)                                                                                       \
+  hipLaunchKernelGGL((backproject_direct_kernel<8, ZEROS>), dim3((unsigned)blocks), dim3(64 * waves),          \
+                     sizeof(float) * waves * zd * 64, s, filt_pad, views, view0, nviews_chunk, grid, vol,      \
+                     accumulate, (int)cb)
+    if (reach.zeros) MONTE_BP(true); else MONTE_BP(false);
+#undef MONTE_BP
+    return hipGetLastError();
+  }
+  int tile_x = std::min(32, std::max(8, (int)t.bp_tile_x));  // whole 8 x 8 sub-tiles, one per wave
+  auto fits = [&](int rows, int cols) {
+    return nq == 4 ? patch_fits<4>(rows, cols) : (nq == 2 ? patch_fits<2>(rows, cols) : patch_fits<1>(rows, cols));
+  };
+  const int nx = nq == 4 ? (grid.nx + 1) / 2 : ncx, ny = nq > 1 ? (grid.ny + 1) / 2 : grid.ny;
+  auto blocks_of = [&](int tx, int z) {
+    return (long)((nx + tx - 1) / tx) * ((ny + 256 / tx - 1) / (256 / tx)) * ((grid.nz + z - 1) / z);
+  };
+  int rows, cols;
+  patch_bounds(grid, reach, tile_x, 256 / tile_x, zc, rows, cols);
+  if (!fits(rows, cols)) {  // the tuned shape does not fit: the default does
+    tile_x = 16;
+    zc = 16;
+    patch_bounds(grid, reach, 16, 16, 16, rows, cols);
+  }
+  if (nq == 1 && zc == 16 && reach.zeros) {
+    // two groups of 16 share a column's set-up, where their patch fits and they fill the chip
+    int r2, c2;
+    patch_bounds(grid, reach, tile_x, 256 / tile_x, 32, r2, c2);
+    if (fits(r2, c2) && blocks_of(tile_x, 32) >= 768) {
+      zc = 32;
+      rows = r2;
+    }
+  }
+  const int tiles_x = (nx + tile_x - 1) / tile_x, tiles_y = (ny + 256 / tile_x - 1) / (256 / tile_x);
+  const long nblocks = blocks_of(tile_x, zc);
+  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+#define MONTE_BP(ZC, NQ, ZEROS)                                                                                \
+  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256),                         \
+                     2 * sizeof(float) * rows * PatchLayout<NQ>::kRS, s, filt_pad, views, view0, nviews_chunk,  \
+                     grid, vol, accumulate, tile_x, tiles_x, tiles_y, rows, reach.turn)
+#define MONTE_BP_Z(NQ, ZEROS)                                                                                    \
+  switch (zc) {                                                                                                \
+    case 4: MONTE_BP(4, NQ, ZEROS); break;                                                                            \
+    case 8: MONTE_BP(8, NQ, ZEROS); break;                                                                            \
+    default: MONTE_BP(16, NQ, ZEROS); break;                                                                   \
+  }
+  if (nq == 4) { MONTE_BP_Z(4, true) }
+  else if (nq == 2) { MONTE_BP_Z(2, true) }
+  else if (zc == 32) MONTE_BP(32, 1, true);
+  else if (reach.zeros) { MONTE_BP_Z(1, true) }
+  else { MONTE_BP_Z(1, false) }
+#undef MONTE_BP_Z
+#undef MONTE_BP
   return hipGetLastError();
 }
 

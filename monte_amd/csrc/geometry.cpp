@@ -78,6 +78,7 @@ void compute_bp_views(const monte_geom& g, std::vector<BpView>& out) {
 BpGrid compute_bp_grid(const monte_geom& g) {
   BpGrid q{};
   q.nx = g.nx; q.ny = g.ny; q.nz = g.nz; q.nu = g.nu; q.nv = g.nv;
+  q.n_views = g.n_views;
   q.pitch = g.nu + kPadLo + kPadHi;
   q.rows = g.nv + kPadLo + kPadHi;
   if (g.preset == MONTE_PRESET_BP3D20) {
@@ -103,6 +104,25 @@ BpGrid compute_bp_grid(const monte_geom& g) {
     q.mask = 0;
   }
   return q;
+}
+
+BpReach compute_bp_reach(const monte_geom& g, const BpGrid& grid) {
+  BpReach r{};
+  r.sod = g.sod;
+  for (int x : {grid.x0, grid.x1 - 1})
+    for (int y : {0, grid.ny - 1})
+      r.rad = std::max(r.rad, std::hypot(grid.gx0 + x * grid.gsx, grid.gy0 + y * grid.gsy));
+  r.suk = g.sdd / g.du;
+  r.svk = g.sdd / g.dv;
+  r.zeros = g.preset == MONTE_PRESET_STANDARD;
+  // a full turn (a part of it off by 1e-12 moves a sample by less than 1e-8
+  // pixels) about the centre of the volume
+  const double turns = g.n_views * g.dangle / (2.0 * kPi);
+  const bool full = g.preset == MONTE_PRESET_STANDARD && std::fabs(std::fabs(turns) - 1.0) < 1e-12 && g.ox == 0.0 &&
+                    g.oy == 0.0;
+  r.half = full && g.n_views % 2 == 0;
+  if (full && g.n_views % 4 == 0 && g.nx == g.ny && g.vx == g.vy) r.turn = turns > 0 ? 1 : -1;
+  return r;
 }
 
 FilterParams compute_filter_params(const monte_geom& g) {

@@ -66,7 +66,7 @@ static_assert(sizeof(BpView) == 120, "BpView layout");
 
 // Geometry-wide constants of the backprojector.
 struct BpGrid {
-  int nx, ny, nz, nu, nv;
+  int nx, ny, nz, nu, nv, n_views;
   int pitch;          // padded row pitch of filtered projections (nu + kPadLo + kPadHi)
   int rows;           // padded rows (nv + kPadLo + kPadHi)
   double gx0, gsx;    // X = gx0 + x * gsx (unfused, as recon/bp3d20_325.cpp:107)
@@ -80,6 +80,17 @@ struct BpGrid {
   int mcx, mcy, mcz;  // mask centre (voxel index)
 };
 
+// What the backprojector's tiling has to know of a scan: how far the volume
+// reaches from the axis, the scale of the sample coordinates, and whether a
+// quarter turn maps the scan onto itself.
+struct BpReach {
+  double sod, rad;  // source distance; largest in-plane distance of a voxel centre from the axis
+  double suk, svk;  // |d(su)| per unit of y'/U, |d(sv)| per unit of Z/U
+  bool zeros;       // the guard cells of the padded views hold zeros, and there is no mask
+  bool half;        // view k + V/2 is view k turned by 180 degrees and so is the volume
+  int turn;         // +-1: view k + V/4 is view k turned by +-90 degrees and so is the volume; 0: neither
+};
+
 // Filter constants: weight(r,c) = D / sqrt(D^2 + (a_u + b_u r)^2 + (a_v + b_v c)^2),
 // out = cs * sum_r weight * p * h[r - b].
 struct FilterParams {
@@ -91,6 +102,7 @@ struct FilterParams {
 
 void compute_bp_views(const monte_geom& g, std::vector<BpView>& out);
 BpGrid compute_bp_grid(const monte_geom& g);
+BpReach compute_bp_reach(const monte_geom& g, const BpGrid& grid);
 FilterParams compute_filter_params(const monte_geom& g);
 void compute_filter_taps(const monte_geom& g, std::vector<float>& h);  // h[0..2nu-2], centre nu-1
 
@@ -209,7 +221,7 @@ struct monte_ctx {
   //   2 MC descriptors                    3 FDK constants (taps + per-view coefficients)
   //   4..7 staging for host-pointer mode and tuning scratch
   //   8 z-fastest copy of the volume for the matched projector
-  //   9 tap quads of the forward filtered stack (backprojection input)
+  //   9 unused
   //  10 column lists of the matched projector (per geometry)
   //  11 end-to-end step: MC descriptors and loss partial sums
   //  12 first-flight label sets of MC launches   13 those of the end-to-end step
@@ -273,12 +285,10 @@ hipError_t launch_unpad_copy(const float* filt_pad, float* filt, int n_views, in
                              hipStream_t s);
 hipError_t launch_fill_pads(float* buf, int n_views, int nu, int nv, int pitch, int rows, int wrap, hipStream_t s);
 hipError_t launch_fold_pads(float* buf, int n_views, int nu, int nv, int pitch, int rows, hipStream_t s);
-// Tap quads of the padded filtered views: quads[i] holds the 2 x 2 bilinear
-// neighbourhood whose top-left cell is padded cell i (n_views * rows * pitch),
-// as (p00, p01 - p00, p10, p11 - p10).
-hipError_t launch_tap_quads(const float* filt_pad, float4* quads, int n_views, int rows, int pitch, hipStream_t s);
-hipError_t launch_backproject(const float4* quads, const BpView* views, int view0, int nviews_chunk,
-                              const BpGrid& grid, float* vol, int accumulate, const monte_tuning& t, hipStream_t s);
+// filt_pad [n_views][rows][pitch] -> vol, views [view0, view0 + nviews_chunk)
+hipError_t launch_backproject(const float* filt_pad, const BpView* views, int view0, int nviews_chunk,
+                              const BpGrid& grid, const BpReach& reach, float* vol, int accumulate,
+                              const monte_tuning& t, hipStream_t s);
 // volT: the volume with z fastest ([y][x][z], see launch_transpose_zx); every
 // cell of the padded views [view0, view0 + nviews_chunk) is written.  Padded
 // rows [lds_r0, lds_r0 + lds_rows) must hold every row the views' voxels can
