@@ -46,6 +46,8 @@ constexpr int kSlotFwd = 0, kSlotAdj = 1, kSlotMc = 2, kSlotConst = 3, kSlotStag
               kSlotTuneA = 6, kSlotTuneB = 7, kSlotVolT = 8,
               kSlotPlan = 10, kSlotE2E = 11, kSlotRay = 12, kSlotE2ERay = 13;
 
+constexpr size_t kHostCounters = 2048;  // sets of counters copied to pinned host memory (160 KB)
+
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 int check_geom(monte_ctx* c, const monte_geom* g, bool need_volume) {
@@ -254,12 +256,12 @@ int run_filter_T_padded(monte_ctx* c, const monte_geom& g, const float* pad, flo
 // ------------------------------------------------------------------ MC
 struct HostJob {
   McJob d{};
-  double org[3] = {0, 0, 0}, vox[3] = {1, 1, 1};  // phantom grid origin (corner) and voxel size
+  double vox[3] = {1, 1, 1};    // phantom voxel size
   McTables tables{};
   std::vector<float> cdf;       // empty = mono
   std::vector<float2> view_cs;  // all views of the geometry
   std::vector<double> cs64;     // FP64 (cos, sin) of all views, for the first-flight label sets
-  RayGrid ray{};                // first-flight label-set geometry (box and bricks filled in by prepare_mc)
+  RayGrid ray{};                // first-flight label-set geometry (bricks filled in by prepare_mc)
 };
 
 // Work units: groups of detector tiles over blocks of photon cycles, about
@@ -378,8 +380,8 @@ int build_job(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, const 
   J.view_begin = vb;
   J.n_views_sim = ve - vb;
   J.vx = (float)ph->vx; J.vy = (float)ph->vy; J.vz = (float)ph->vz;
-  hj.org[0] = ph->ox - 0.5 * ph->nx * ph->vx; hj.org[1] = ph->oy - 0.5 * ph->ny * ph->vy;
-  hj.org[2] = ph->oz - 0.5 * ph->nz * ph->vz;
+  R.org[0] = ph->ox - 0.5 * ph->nx * ph->vx; R.org[1] = ph->oy - 0.5 * ph->ny * ph->vy;
+  R.org[2] = ph->oz - 0.5 * ph->nz * ph->vz;
   hj.vox[0] = ph->vx; hj.vox[1] = ph->vy; hj.vox[2] = ph->vz;
   J.bx0 = (float)(ph->ox - 0.5 * ph->nx * ph->vx); J.bx1 = (float)(ph->ox + 0.5 * ph->nx * ph->vx);
   J.by0 = (float)(ph->oy - 0.5 * ph->ny * ph->vy); J.by1 = (float)(ph->oy + 0.5 * ph->ny * ph->vy);
@@ -407,7 +409,9 @@ int build_job(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, const 
   return MONTE_OK;
 }
 
-McLayout mc_layout(const std::vector<HostJob>& hj) {
+// `sets`: with room for the FP64 view tables of the first-flight label sets;
+// `slots`: sets of counters per job.
+McLayout mc_layout(const std::vector<HostJob>& hj, bool sets, int slots) {
   const int n = (int)hj.size();
   McLayout L;
   size_t off = 0;
@@ -415,149 +419,137 @@ McLayout mc_layout(const std::vector<HostJob>& hj) {
   L.tab_off = off; off = align_up(off + sizeof(McTables) * n, 256);
   L.cdf_off.resize(n);
   L.cs_off.resize(n);
+  L.cs64_off.resize(n);
   for (int i = 0; i < n; ++i) {
     L.cdf_off[i] = off; off = align_up(off + sizeof(float) * hj[i].cdf.size(), 256);
     L.cs_off[i] = off; off = align_up(off + sizeof(float2) * hj[i].view_cs.size(), 256);
+    L.cs64_off[i] = off; if (sets) off = align_up(off + sizeof(double) * hj[i].cs64.size(), 256);
   }
   L.q_off = off; off = align_up(off + kMcQueueBytes, 256);
-  L.cnt_off = off; off = align_up(off + sizeof(McCounters) * n, 256);
-  L.box_off = off; off = align_up(off + sizeof(int) * 8 * n, 256);
+  L.cnt_off = off; off = align_up(off + sizeof(McCounters) * n * slots, 256);
+  L.prep_off = off; off = align_up(off + sizeof(McPrep) * n, 256);
   L.total = off;
   return L;
 }
 
-// First-flight label sets of every job (tuning mc_ray_brick > 0) in workspace
-// slot `slot`: the FP64 view tables, the brick sets and the per-view,
-// per-pixel sets; each job's descriptor then points at its sets.  The flight
-// boxes must be final.
-int prepare_ray_sets(monte_ctx* c, std::vector<HostJob>& hj, int slot) {
-  const int b = c->tuning.mc_ray_brick;
-  const int n = (int)hj.size();
-  std::vector<size_t> cs_off(n), br_off(n), set_off(n);
-  size_t off = 0;
-  for (int i = 0; i < n; ++i) {
-    HostJob& h = hj[i];
-    const McJob& J = h.d;
-    RayGrid& R = h.ray;
-    const int dims[3] = {J.nx, J.ny, J.nz};
-    for (int a = 0; a < 3; ++a) {
-      R.org[a] = h.org[a];
-      R.bw[a] = b * h.vox[a];
-      R.nb[a] = (dims[a] + b - 1) / b;
-    }
-    cs_off[i] = off; off = align_up(off + sizeof(double) * h.cs64.size(), 256);
-    br_off[i] = off; off = align_up(off + (size_t)R.nb[0] * R.nb[1] * R.nb[2], 256);
-    set_off[i] = off; off = align_up(off + (size_t)J.n_views_sim * J.nu * J.nv, 256);
-  }
-  char* base = (char*)workspace(c, slot, off);
-  if (!base) return fail(c, MONTE_ERR_NOMEM, "first-flight label set allocation failed");
-  for (int i = 0; i < n; ++i) {
-    HostJob& h = hj[i];
-    McJob& J = h.d;
-    MONTE_HIP(c, hipMemcpyAsync(base + cs_off[i], h.cs64.data(), sizeof(double) * h.cs64.size(),
-                                hipMemcpyHostToDevice, c->stream));
-    uint8_t* bricks = (uint8_t*)(base + br_off[i]);
-    uint8_t* sets = (uint8_t*)(base + set_off[i]);
-    MONTE_HIP(c, launch_brick_sets(J.labels, J.nx, J.ny, J.nz, b, h.ray.nb, bricks, c->stream));
-    MONTE_HIP(c, launch_ray_sets(h.ray, (const double*)(base + cs_off[i]), J.view_begin, J.n_views_sim, bricks, sets,
-                                 c->stream));
-    J.ray_set = sets;
-  }
-  return MONTE_OK;
-}
+// Sets of counters per job: the static scratch of the allocation-free projection
+// (ray slot -1) has room for 3.
+int mc_slots(int ray_slot) { return ray_slot >= 0 ? kMcSlots : kMcSlotsNoAlloc; }
 
-// Lays out the jobs in `base` (at least mc_layout(hj).total bytes; the
-// context's MC workspace when null), computes each job's flight box and, with
-// tuning mc_ray_brick > 0 and ray_slot >= 0, its first-flight label sets in
-// workspace slot ray_slot, and uploads everything; returns once the uploads
-// are complete.
+// Whether a launch with this ray slot forms first-flight label sets.
+bool wants_sets(const monte_ctx* c, int ray_slot) { return ray_slot >= 0 && c->tuning.mc_ray_brick > 0; }
+
+// Lays out the jobs in `base` (at least mc_layout(hj, wants_sets(...)).total
+// bytes; the context's MC workspace when null), queue and counters set,
+// uploads everything in one copy, and launches what forms each job's flight box
+// and, with tuning mc_ray_brick > 0 and ray_slot >= 0, its first-flight label
+// sets in workspace slot ray_slot.  Nothing waits: P.host must outlive the upload.
 int prepare_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per_cu, char* base, McPrepared& P,
                int ray_slot) {
   const int n = (int)hj.size();
-  const McLayout Lo = mc_layout(hj);
+  const int brick = wants_sets(c, ray_slot) ? c->tuning.mc_ray_brick : 0;
+  const int slots = mc_slots(ray_slot);
+  const McLayout Lo = mc_layout(hj, brick > 0, slots);
   if (!base) base = (char*)workspace(c, kSlotMc, Lo.total);
   if (!base) return fail(c, MONTE_ERR_NOMEM, "MC descriptor allocation failed");
+  P.host.assign(Lo.total, 0);
+  char* const host = P.host.data();
+  McPrep* const preps = (McPrep*)(host + Lo.prep_off);
 
-  // Flights are clipped to the bounding box of the voxels that attenuate at
-  // some energy: outside it mu is 0, so no history changes, and no Woodcock
-  // steps are spent crossing the empty margin of the phantom grid.
-  {
-    std::vector<int> box(8 * (size_t)n);
-    for (int i = 0; i < n; ++i) {
-      int* b = box.data() + 8 * i;
-      b[0] = b[1] = b[2] = INT_MAX;
-      b[3] = b[4] = b[5] = -1;
+  std::vector<size_t> br_off(n), set_off(n);
+  size_t ray_bytes = 0;
+  uint64_t prep_blocks = 0, ray_blocks = 0, max_planes = 0;
+  for (int i = 0; i < n; ++i) {
+    HostJob& h = hj[i];
+    const McJob& J = h.d;
+    McPrep& Q = preps[i];
+    Q.labels = J.labels;
+    Q.nx = J.nx; Q.ny = J.ny; Q.nz = J.nz;
+    for (int l = 0; l < kMaxLabels; ++l)
+      for (int e = 0; e < kRows; ++e)
+        if (h.tables.m[l][e].x > 0.f) { Q.solid |= 1u << l; break; }
+    for (int a = 0; a < 3; ++a) {
+      Q.box[a] = INT_MAX;
+      Q.box[3 + a] = -1;
+      Q.vox[a] = h.vox[a];
     }
-    int* dbox = (int*)(base + Lo.box_off);
-    MONTE_HIP(c, hipMemcpyAsync(dbox, box.data(), sizeof(int) * box.size(), hipMemcpyHostToDevice, c->stream));
-    for (int i = 0; i < n; ++i) {
-      uint32_t solid = 0;
-      for (int l = 0; l < kMaxLabels; ++l)
-        for (int e = 0; e < kRows; ++e)
-          if (hj[i].tables.m[l][e].x > 0.f) { solid |= 1u << l; break; }
-      const McJob& J = hj[i].d;
-      MONTE_HIP(c, launch_support_box(J.labels, J.nx, J.ny, J.nz, solid, dbox + 8 * i, c->stream));
-    }
-    MONTE_HIP(c, hipMemcpyAsync(box.data(), dbox, sizeof(int) * box.size(), hipMemcpyDeviceToHost, c->stream));
-    MONTE_HIP(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < n; ++i) {
-      const int* b = box.data() + 8 * i;
-      McJob& J = hj[i].d;
-      const double* o = hj[i].org;
-      const double* v = hj[i].vox;
-      RayGrid& R = hj[i].ray;
+    // a block of the box takes 4 chunks of 16 bytes a thread, up to 2048 blocks
+    const uint64_t voxels = (uint64_t)J.nx * J.ny * J.nz;
+    Q.box_blocks = (uint32_t)std::min<uint64_t>(2048, voxels / (16 * 256 * 4) + 1);
+    Q.prep_begin = (uint32_t)prep_blocks;
+    prep_blocks += Q.box_blocks;
+    Q.brick = brick;
+    Q.ray_begin = (uint32_t)ray_blocks;
+    if (brick > 0) {
+      RayGrid& R = h.ray;
       const int dims[3] = {J.nx, J.ny, J.nz};
-      if (b[3] < 0) {  // nothing attenuates: keep the grid box
-        for (int a = 0; a < 3; ++a) {
-          R.c0[a] = o[a];
-          R.c1[a] = o[a] + dims[a] * v[a];
-        }
-        continue;
-      }
+      uint64_t planes = 3;
       for (int a = 0; a < 3; ++a) {
-        R.c0[a] = o[a] + b[a] * v[a];
-        R.c1[a] = o[a] + (b[3 + a] + 1) * v[a];
+        R.bw[a] = brick * h.vox[a];
+        R.nb[a] = (dims[a] + brick - 1) / brick;
+        planes += (uint64_t)R.nb[a];
       }
-      J.bx0 = (float)R.c0[0]; J.bx1 = (float)R.c1[0];
-      J.by0 = (float)R.c0[1]; J.by1 = (float)R.c1[1];
-      J.bz0 = (float)R.c0[2]; J.bz1 = (float)R.c1[2];
+      max_planes = std::max(max_planes, planes);
+      const uint64_t nbricks = (uint64_t)R.nb[0] * R.nb[1] * R.nb[2];
+      br_off[i] = ray_bytes; ray_bytes = align_up(ray_bytes + nbricks, 256);
+      set_off[i] = ray_bytes; ray_bytes = align_up(ray_bytes + (size_t)J.n_views_sim * J.nu * J.nv, 256);
+      prep_blocks += (nbricks + 255) / 256;
+      ray_blocks += (uint64_t)J.n_views_sim * (((uint64_t)J.nu * J.nv + kRayBlock - 1) / kRayBlock);
     }
+    Q.ray = h.ray;
   }
-  for (int i = 0; i < n; ++i) hj[i].d.ray_set = nullptr;
-  if (ray_slot >= 0 && c->tuning.mc_ray_brick > 0) {
-    const int rc = prepare_ray_sets(c, hj, ray_slot);
-    if (rc) return rc;
+  if (prep_blocks > 0x7fffffffull || ray_blocks > 0x7fffffffull)
+    return fail(c, MONTE_ERR_INVALID, "too many first-flight label sets in one launch");
+  if (brick > 0) {
+    char* rays = (char*)workspace(c, ray_slot, ray_bytes);
+    if (!rays) return fail(c, MONTE_ERR_NOMEM, "first-flight label set allocation failed");
+    for (int i = 0; i < n; ++i) {
+      preps[i].cs64 = (const double*)(base + Lo.cs64_off[i]);
+      preps[i].bricks = (uint8_t*)(rays + br_off[i]);
+      preps[i].sets = (uint8_t*)(rays + set_off[i]);
+      std::memcpy(host + Lo.cs64_off[i], hj[i].cs64.data(), sizeof(double) * hj[i].cs64.size());
+    }
   }
 
   uint64_t units = 0;
-  std::vector<McJob> jobs(n);
+  McJob* const jobs = (McJob*)(host + Lo.jobs_off);
   for (int i = 0; i < n; ++i) {
-    McJob J = hj[i].d;
+    McJob& J = hj[i].d;
+    J.ray_set = preps[i].sets;
     J.tables = (const McTables*)(base + Lo.tab_off) + i;
     J.spectrum_cdf = hj[i].cdf.empty() ? nullptr : (const float*)(base + Lo.cdf_off[i]);
     J.view_cs = (const float2*)(base + Lo.cs_off[i]);
     J.unit_begin = units;
     units += J.unit_count;
     jobs[i] = J;
+    std::memcpy(host + Lo.tab_off + sizeof(McTables) * i, &hj[i].tables, sizeof(McTables));
+    if (!hj[i].cdf.empty())
+      std::memcpy(host + Lo.cdf_off[i], hj[i].cdf.data(), sizeof(float) * hj[i].cdf.size());
+    std::memcpy(host + Lo.cs_off[i], hj[i].view_cs.data(), sizeof(float2) * hj[i].view_cs.size());
   }
+
   // the 32-bit queue counter passes the last unit by one fetch per wave
   const int grid_waves = std::max(1, c->n_cu * blocks_per_cu) * (block / 64);
   if (units > 0xFFFFFFFFull - (uint64_t)grid_waves)
     return fail(c, MONTE_ERR_INVALID, "too many work units in one launch (raise the batch)");
-  MONTE_HIP(c, hipMemcpyAsync(base + Lo.jobs_off, jobs.data(), sizeof(McJob) * n, hipMemcpyHostToDevice, c->stream));
-  for (int i = 0; i < n; ++i) {
-    MONTE_HIP(c, hipMemcpyAsync(base + Lo.tab_off + sizeof(McTables) * i, &hj[i].tables, sizeof(McTables),
-                                hipMemcpyHostToDevice, c->stream));
-    if (!hj[i].cdf.empty())
-      MONTE_HIP(c, hipMemcpyAsync(base + Lo.cdf_off[i], hj[i].cdf.data(), sizeof(float) * hj[i].cdf.size(),
-                                  hipMemcpyHostToDevice, c->stream));
-    MONTE_HIP(c, hipMemcpyAsync(base + Lo.cs_off[i], hj[i].view_cs.data(), sizeof(float2) * hj[i].view_cs.size(),
-                                hipMemcpyHostToDevice, c->stream));
+  unsigned int* const queue = (unsigned int*)(host + Lo.q_off);
+  for (int q = 0; q < kMcQueues; ++q)
+    queue[q * kMcQueueStride] = mc_queue_start(q, block / 64, std::max(1, c->n_cu * blocks_per_cu));
+  MONTE_HIP(c, hipMemcpyAsync(base, host, Lo.total, hipMemcpyHostToDevice, c->stream));
+  McPrep* const dpreps = (McPrep*)(base + Lo.prep_off);
+  McJob* const djobs = (McJob*)(base + Lo.jobs_off);
+  hipError_t le = launch_mc_prep(dpreps, n, (uint32_t)prep_blocks, c->stream);
+  if (le == hipSuccess)
+    le = brick > 0 ? launch_ray_sets(dpreps, djobs, n, (uint32_t)ray_blocks, max_planes, c->stream)
+                   : launch_mc_boxes(dpreps, djobs, n, c->stream);
+  if (le != hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);  // the upload is done with its host copy
+    return fail(c, MONTE_ERR_HIP, std::string("MC set-up launch: ") + hipGetErrorString(le));
   }
-  MONTE_HIP(c, hipStreamSynchronize(c->stream));  // the host copies above must outlive the uploads
   P.base = base;
   P.L = Lo;
   P.n = n;
+  P.slots = slots;
   P.units = units;
   // A chunk is one tile group over all of the first job's views.  A wave changes
   // job only once its photons of the old job have all ended, so in a launch of
@@ -571,36 +563,55 @@ int prepare_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per
   return MONTE_OK;
 }
 
-// Resets the work queue and counters, then launches the transport (with
-// `start` recorded between the two when given, so it times the transport alone).
-hipError_t launch_prepared(monte_ctx* c, const McPrepared& P, int block, int blocks_per_cu,
+// Launches the transport, after clearing the work queue and counters when it is
+// not the first launch since prepare_mc (with `start` recorded just before it
+// when given, so it times the transport alone).
+hipError_t launch_prepared(monte_ctx* c, const McPrepared& P, int block, int blocks_per_cu, bool again,
                            hipEvent_t start = nullptr) {
-  hipError_t e = launch_mc_reset(P.queue(), P.counters(), P.n, c->stream);
+  const int grid = std::max(1, c->n_cu * blocks_per_cu);
+  hipError_t e = again ? launch_mc_reset(P.queue(), P.counters(), P.n * P.slots, block, grid, c->stream) : hipSuccess;
   if (e != hipSuccess) return e;
   if (start && (e = hipEventRecord(start, c->stream)) != hipSuccess) return e;
-  const int grid = std::max(1, c->n_cu * blocks_per_cu);
   return launch_mc_transport((const McJob*)(P.base + P.L.jobs_off), P.n, P.units, P.chunk, P.queue(), P.counters(),
-                             block, grid, c->stream);
+                             P.slots, block, grid, c->stream);
 }
 
 int read_counters(monte_ctx* c, const McPrepared& P, std::vector<McCounters>& cnt) {
-  cnt.resize(P.n);
-  MONTE_HIP(c, hipMemcpyAsync(cnt.data(), P.counters(), sizeof(McCounters) * P.n, hipMemcpyDeviceToHost, c->stream));
+  const size_t all = (size_t)P.n * P.slots;
+  std::vector<McCounters> own(all <= kHostCounters ? 0 : all);
+  McCounters* const from = own.empty() ? c->host_counters : own.data();
+  MONTE_HIP(c, hipMemcpyAsync(from, P.counters(), sizeof(McCounters) * all, hipMemcpyDeviceToHost, c->stream));
   MONTE_HIP(c, hipStreamSynchronize(c->stream));
+  cnt.assign(P.n, McCounters{});
+  for (size_t i = 0; i < all; ++i) {
+    McCounters& k = cnt[i / P.slots];
+    const McCounters& f = from[i];
+    k.histories += f.histories; k.steps += f.steps; k.interactions += f.interactions;
+    k.photo += f.photo; k.coherent += f.coherent; k.compton += f.compton;
+    k.tallied_primary += f.tallied_primary; k.tallied_scatter += f.tallied_scatter;
+    k.missed += f.missed; k.capped += f.capped;
+  }
   return MONTE_OK;
 }
 
 // Prepares and runs one launch in a device buffer: the context's MC workspace,
-// or `base` (at least mc_layout(hj).total bytes) when the caller provides one.
+// or `base` (at least mc_layout's total bytes) when the caller provides one.
 int run_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per_cu, float* ms_out,
            std::vector<McCounters>* counters_out, char* base = nullptr, int ray_slot = kSlotRay) {
   McPrepared P;
   int rc = prepare_mc(c, hj, block, blocks_per_cu, base, P, ray_slot);
-  if (rc) return rc;
-  const hipError_t le = launch_prepared(c, P, block, blocks_per_cu, c->ev0);
-  MONTE_HIP(c, hipEventRecord(c->ev1, c->stream));
+  hipError_t le = hipSuccess;
   std::vector<McCounters> cnt;
-  if ((rc = read_counters(c, P, cnt))) return rc;
+  if (!rc) {
+    le = launch_prepared(c, P, block, blocks_per_cu, false, c->ev0);
+    const hipError_t e = hipEventRecord(c->ev1, c->stream);
+    if (e != hipSuccess) rc = fail(c, MONTE_ERR_HIP, std::string("event record: ") + hipGetErrorString(e));
+    if (!rc) rc = read_counters(c, P, cnt);
+  }
+  if (rc) {
+    (void)hipStreamSynchronize(c->stream);  // P.host outlives its upload
+    return rc;
+  }
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
   if (le != hipSuccess) return fail(c, MONTE_ERR_HIP, std::string("transport launch: ") + hipGetErrorString(le));
@@ -647,7 +658,7 @@ int e2e_launches(monte_ctx* c, const monte_geom& g, const monte_e2e_buffers& b, 
   MONTE_HIP(c, launch_fill((float*)b.primary, 0.f, 2 * np, c->stream));
   MONTE_HIP(c, launch_fill((float*)b.scatter, 0.f, 2 * np, c->stream));
   const monte_tuning& t = c->tuning;
-  MONTE_HIP(c, launch_prepared(c, c->e2e_mc, t.mc_block, t.mc_blocks_per_cu));
+  MONTE_HIP(c, launch_prepared(c, c->e2e_mc, t.mc_block, t.mc_blocks_per_cu, true));
   MONTE_HIP(c, launch_counts_to_lineint(b.primary, b.scatter, b.lineint, g.n_views, g.nu, g.nv, ppv, c->stream));
   float* pad = (float*)c->ws[kSlotFwd];
   int rc = run_filter_padded(c, g, b.lineint, pad);
@@ -720,7 +731,8 @@ int monte_create(monte_ctx** out, int device) {
     return MONTE_ERR_HIP;
   }
   // the allocation-free entry points' scratch: located once per device
-  if (noalloc_setup(device) != 0) {
+  if (noalloc_setup(device) != 0 ||
+      hipHostMalloc((void**)&c->host_counters, sizeof(McCounters) * kHostCounters) != hipSuccess) {
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->own_stream);
@@ -744,6 +756,7 @@ void monte_destroy(monte_ctx* c) {
   if (c->e2e_graph) (void)hipGraphDestroy(c->e2e_graph);
   for (int i = 0; i < monte_ctx::kSlots; ++i)
     if (c->ws[i]) (void)hipFree(c->ws[i]);
+  if (c->host_counters) (void)hipHostFree(c->host_counters);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -980,7 +993,10 @@ int monte_mc_batch(monte_ctx* c, const monte_mc_job* jobs, int n_jobs, monte_mc_
   // launch holding fewer than 32 units of `batch` photons per wave of the grid
   // halves its units, down to 16 cycles of a tile.  The tallies do not depend on
   // the unit size.  64 uneven jobs (4.6e8 histories): 12.7 ms with units of 64
-  // cycles, 12.2-12.4 with 32, 12.4-12.5 with 16 and 13.5 with 8.
+  // cycles, 12.2-12.4 with 32, 12.4-12.5 with 16 and 13.5 with 8.  Launches of
+  // fewer than 4 of those units per wave halve them further, down to one cycle:
+  // 7.2e5 histories (36 views of 128^2) in 720 units left seven waves of eight
+  // without any and took 324 us.
   {
     uint64_t hist = 0;
     for (const HostJob& h : hj) hist += (uint64_t)h.d.photons_per_view * (uint64_t)h.d.n_views_sim;
@@ -988,6 +1004,7 @@ int monte_mc_batch(monte_ctx* c, const monte_mc_job* jobs, int n_jobs, monte_mc_
         (uint64_t)std::max(1, c->n_cu * c->tuning.mc_blocks_per_cu) * (uint64_t)(c->tuning.mc_block / 64);
     int b = batch;
     while (b > 64 * 16 && hist < (uint64_t)b * 32 * waves) b /= 2;
+    while (b > 64 && hist < (uint64_t)b * 4 * waves) b /= 2;
     if (b != batch)
       for (HostJob& h : hj) set_units(h.d, b);
   }
@@ -1034,7 +1051,7 @@ int monte_mc_project_noalloc(monte_ctx* c, const monte_geom* g, const monte_phan
   std::vector<HostJob> hj(1);
   int rc = build_job(c, g, ph, cfg, hj[0], batch);
   if (rc) return rc;
-  const size_t need = mc_layout(hj).total;
+  const size_t need = mc_layout(hj, false, mc_slots(-1)).total;
   if (need > kNoAllocScratchBytes)
     return fail(c, MONTE_ERR_INVALID, "the job needs " + std::to_string(need) + " bytes of scratch, more than the " +
                                           std::to_string(kNoAllocScratchBytes) + " available (fewer views)");
@@ -1436,11 +1453,13 @@ int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, c
     if ((rc = build_job(c, g, ph, cfg, hj[0], batch))) return rc;
     hj[0].d.primary = b.primary;
     hj[0].d.scatter = b.scatter;
-    const size_t need = mc_layout(hj).total + kLossBlocks * sizeof(double);
+    const size_t need = mc_layout(hj, wants_sets(c, kSlotE2ERay), mc_slots(kSlotE2ERay)).total + kLossBlocks * sizeof(double);
     char* base = (char*)workspace(c, kSlotE2E, need);
     if (!base) return fail(c, MONTE_ERR_NOMEM, "end-to-end descriptor allocation failed");
     if ((rc = prepare_mc(c, hj, c->tuning.mc_block, c->tuning.mc_blocks_per_cu, base, c->e2e_mc, kSlotE2ERay)))
       return rc;
+    MONTE_HIP(c, hipStreamSynchronize(c->stream));  // the upload is done with its host copy
+    c->e2e_mc.host = std::vector<char>();
     c->e2e_mc_key = mkey;
   }
   double* partial = (double*)(c->e2e_mc.base + c->e2e_mc.L.total);

@@ -160,11 +160,30 @@ struct McJob {
 struct RayGrid {
   double un0, u_step, vn0, v_step;  // pixel centre: y' = (iu + 1/2 - un0) u_step, z' likewise
   double sod, xd;                   // source distance, detector plane x' = xd
-  double c0[3], c1[3];              // flight box (bounding box of the attenuating voxels)
-  double org[3], bw[3];             // brick grid corner and brick size
+  double org[3], bw[3];             // brick grid corner (the phantom's) and brick size
   int nb[3];                        // bricks per axis
   int nu, nv;
 };
+
+// What the launches before a transport need of one job: its flight box (the
+// bounding box of its attenuating voxels, formed in `box`) and its first-flight
+// label sets.  The jobs of a launch share the grids of these kernels; a job's
+// blocks start at prep_begin and ray_begin.
+struct McPrep {
+  const uint8_t* labels;
+  const double* cs64;            // FP64 (cos, sin) of every view, or null without sets
+  uint8_t* bricks;               // brick sets [nb2][nb1][nb0]
+  uint8_t* sets;                 // label sets [n_views][nu nv]
+  RayGrid ray;
+  double vox[3];                 // voxel size
+  uint32_t solid;                // bit l: label l attenuates at some energy
+  int nx, ny, nz;
+  int box[6];                    // minima, maxima (voxels); {INT_MAX x 3, -1 x 3} before the launch
+  int brick;                     // voxels a side, 0: no sets
+  uint32_t box_blocks;           // the first of the job's prep blocks, for the box; the rest for bricks
+  uint32_t prep_begin, ray_begin;
+};
+static_assert(sizeof(McPrep) <= 256, "the static scratch of the allocation-free projection counts 256 bytes for it");
 
 // FP64 ray geometry of the exact primary estimator.
 struct PrimaryGeom {
@@ -174,7 +193,7 @@ struct PrimaryGeom {
   int nu, nv, n_views;
 };
 
-struct McCounters {  // device-side statistics, one per job
+struct McCounters {  // device-side statistics
   unsigned long long histories, steps, interactions, photo, coherent, compton;
   unsigned long long tallied_primary, tallied_scatter, missed, capped;
 };
@@ -182,8 +201,8 @@ struct McCounters {  // device-side statistics, one per job
 // Where a launch's job descriptors, tables, CDFs, view tables, queue, counters
 // and flight boxes sit in its device buffer.
 struct McLayout {
-  size_t jobs_off = 0, tab_off = 0, q_off = 0, cnt_off = 0, box_off = 0, total = 0;
-  std::vector<size_t> cdf_off, cs_off;
+  size_t jobs_off = 0, tab_off = 0, q_off = 0, cnt_off = 0, prep_off = 0, total = 0;
+  std::vector<size_t> cdf_off, cs_off, cs64_off;
 };
 
 // A transport launch whose descriptors are in place in device memory;
@@ -191,9 +210,10 @@ struct McLayout {
 struct McPrepared {
   char* base = nullptr;
   McLayout L;
-  int n = 0;
+  int n = 0, slots = 1;
   uint64_t units = 0;
   uint32_t chunk = 1;  // units per queue chunk (the first job's simulated views; more with several jobs)
+  std::vector<char> host;  // the uploaded descriptors, kept until the stream has passed the upload
   unsigned int* queue() const { return (unsigned int*)(base + L.q_off); }
   McCounters* counters() const { return (McCounters*)(base + L.cnt_off); }
 };
@@ -209,6 +229,9 @@ struct monte_ctx {
   bool host_ptrs = false;
   std::string err;
   int n_cu = 256;
+
+  // pinned host memory the transport's counters are copied to (as many jobs as fit)
+  monte::McCounters* host_counters = nullptr;
 
   // attenuation tables (host copy, FP64): [n_tables][4][201]
   std::vector<double> tables;
@@ -324,20 +347,33 @@ hipError_t launch_fdk_filter_T(const float* filt_pad, float* proj, const float* 
 constexpr int kMcQueues = 24;
 constexpr int kMcQueueStride = 16;
 constexpr size_t kMcQueueBytes = sizeof(unsigned int) * kMcQueues * kMcQueueStride;
+// Counter q starts past the units that the queue's waves take by rank, and a bit
+// per spent queue sits in a word of the last counter's line.
+constexpr int kMcSpentWord = (kMcQueues - 1) * kMcQueueStride + kMcQueueStride / 2;
+static_assert(kMcQueues < 32, "one bit per queue");
+__host__ __device__ inline unsigned int mc_queue_start(int q, int waves_per_block, int grid) {
+  return (unsigned int)(waves_per_block * ((grid - q + kMcQueues - 1) / kMcQueues));
+}
+// Statistics: `slots` sets of counters per job, a block adding to set b mod slots
+// (in one set, the adds of the 6144 waves of a short launch took 400 us); the
+// host adds them up.
+constexpr int kMcSlots = 32, kMcSlotsNoAlloc = 3;
 hipError_t launch_mc_transport(const McJob* jobs_dev, int n_jobs, uint64_t total_units, uint32_t chunk,
-                               unsigned int* queue, McCounters* counters, int block, int grid, hipStream_t s);
-hipError_t launch_mc_reset(unsigned int* queue, McCounters* counters, int n_jobs, hipStream_t s);
-// First-flight label sets: per brick of b^3 voxels widened by one voxel
-// (bricks [nb2][nb1][nb0]), then per view of [view_begin, view_begin +
-// n_views) and pixel in aim order (sets [n_views][nu nv]); cs64 holds FP64
-// (cos, sin) of every view of the scan.
-hipError_t launch_brick_sets(const uint8_t* labels, int nx, int ny, int nz, int b, const int nb[3], uint8_t* bricks,
-                             hipStream_t s);
-hipError_t launch_ray_sets(const RayGrid& R, const double* cs64, int view_begin, int n_views, const uint8_t* bricks,
-                           uint8_t* sets, hipStream_t s);
-// Bounding box (voxel indices, inclusive) of voxels whose clamped label has bit set in `solid`:
-// box[0..2] = minima, box[3..5] = maxima; the caller initialises it to {INT_MAX x 3, -1 x 3}.
-hipError_t launch_support_box(const uint8_t* labels, int nx, int ny, int nz, uint32_t solid, int* box, hipStream_t s);
+                               unsigned int* queue, McCounters* counters, int slots, int block, int grid,
+                               hipStream_t s);
+hipError_t launch_mc_reset(unsigned int* queue, McCounters* counters, int n_counters, int block, int grid,
+                           hipStream_t s);
+// The flight boxes and brick sets of all jobs (prep_blocks in all), then their
+// label sets (ray_blocks) and the boxes written into their descriptors.
+// Brick sets: per brick of b^3 voxels widened by one voxel; label sets: per
+// simulated view and pixel in aim order.  max_planes: the largest job's brick
+// planes (nb0 + nb1 + nb2 + 3).  Without sets, launch_mc_boxes does the latter
+// alone.
+hipError_t launch_mc_prep(McPrep* preps, int n_jobs, uint32_t prep_blocks, hipStream_t s);
+hipError_t launch_ray_sets(const McPrep* preps, McJob* jobs, int n_jobs, uint32_t ray_blocks, uint64_t max_planes,
+                           hipStream_t s);
+hipError_t launch_mc_boxes(const McPrep* preps, McJob* jobs, int n_jobs, hipStream_t s);
+constexpr int kRayBlock = 256;  // pixels per block of the label sets
 hipError_t launch_primary_exact(const PrimaryGeom& P, const double* cs64, const uint8_t* labels,
                                 const McTables* tables, float e_kev, const float* spec_w, int use_spec, float* out,
                                 hipStream_t s);

@@ -460,10 +460,11 @@ constexpr unsigned kRefillBatch = 16;
 __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restrict__ jobs, int n_jobs,
                                                            uint64_t total_units, uint32_t chunk,
                                                            unsigned int* __restrict__ queue,
-                                                           McCounters* __restrict__ counters) {
+                                                           McCounters* __restrict__ counters, int slots) {
   int job = -1;
   const int q_first = (int)(blockIdx.x % kMcQueues);
-  int q_tried = 0;  // queues found spent (the wave then draws from the next)
+  int q_own = q_first;   // the queue the wave draws from
+  bool q_begun = false;  // the wave has had its first unit
   // the current unit (wave-uniform): tiles [unit_t0, unit_t0 + unit_nt) over photon
   // cycles [unit_cyc, unit_cyc_end); the next birth takes tile unit_t0 + unit_g of
   // cycle unit_cyc
@@ -526,18 +527,33 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
         // one per round, so no queue keeps the same detector rows when kMcQueues chunks
         // span a whole number of detector sweeps.  Units increase with k, so a queue is
         // spent once it hands out a unit past the end.
-        while (q_tried < kMcQueues) {
-          const int q = (q_first + q_tried) % kMcQueues;
+        // A wave's first unit is the one of its rank among the queue's waves (the
+        // counters start past those), so a launch of few units per wave hardly
+        // touches the counters.  A wave that finds its queue spent marks it, and
+        // moves to the next one not marked: without the marks every wave of a
+        // launch ended by drawing once from each of the 24.
+        for (;;) {
           unsigned int k = 0;
-          if (lane == 0) k = atomicAdd(queue + q * kMcQueueStride, 1u);
+          if (!q_begun) {
+            q_begun = true;
+            k = (blockIdx.x / kMcQueues) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+          } else if (lane == 0) {
+            k = atomicAdd(queue + q_own * kMcQueueStride, 1u);
+          }
           k = (unsigned int)__builtin_amdgcn_readfirstlane((int)k);
           const uint32_t r = k / chunk;
-          const uint64_t u = ((uint64_t)r * kMcQueues + (uint64_t)((q + r) % kMcQueues)) * chunk + (k - r * chunk);
+          const uint64_t u = ((uint64_t)r * kMcQueues + (uint64_t)((q_own + r) % kMcQueues)) * chunk + (k - r * chunk);
           if (u < total_units) {
             pending = (long long)u;
             break;
           }
-          ++q_tried;
+          unsigned int spent = 0;
+          if (lane == 0) spent = atomicOr(queue + kMcSpentWord, 1u << q_own) | (1u << q_own);
+          spent = (unsigned int)__builtin_amdgcn_readfirstlane((int)spent);
+          if (spent == (1u << kMcQueues) - 1u) break;
+          do {
+            q_own = q_own + 1 == kMcQueues ? 0 : q_own + 1;
+          } while ((spent >> q_own) & 1u);
         }
         if (pending < 0) exhausted = true;
       }
@@ -546,7 +562,7 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
         if (pj == job || (all_dead && buf_n == 0 && pend == 0)) {  // buffered and ended photons are of the current job
           const bool switched = pj != job;
           if (switched) {
-            if (job >= 0) flush(counters + job);
+            if (job >= 0) flush(counters + job * slots + blockIdx.x % slots);
             job = pj;
             ray_tile = ~0u;  // another job's geometry
           }
@@ -828,7 +844,7 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
     }
     count_lanes(wt, kStatSteps, two);
   }
-  if (job >= 0) flush(counters + job);
+  if (job >= 0) flush(counters + job * slots + blockIdx.x % slots);
 }
 
 // --------------------------------------------- first-flight label sets
@@ -837,65 +853,242 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
 
 __device__ inline uint32_t label_bit(int lab) { return lab < 4 ? 1u << lab : kAnyLabel; }
 
+// The label sets of the bytes of w.
+__device__ inline uint32_t label_bits(uint32_t w) {
+  return label_bit((int)(w & 255u)) | label_bit((int)((w >> 8) & 255u)) | label_bit((int)((w >> 16) & 255u)) |
+         label_bit((int)(w >> 24));
+}
+
+__device__ inline uint32_t load_u32(const uint8_t* p) {  // (any alignment)
+  uint32_t w;
+  __builtin_memcpy(&w, p, 4);
+  return w;
+}
+
 // One thread per brick: the labels of the brick's voxels and of their
 // neighbours one voxel outside it, so a sample point rounded across a brick
-// face into a voxel of the next brick is still covered.
-__global__ __launch_bounds__(256) void brick_sets_kernel(const uint8_t* __restrict__ labels, int nx, int ny, int nz,
-                                                         int b, int nb0, int nb1, int nb2,
-                                                         uint8_t* __restrict__ bricks) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long)nb0 * nb1 * nb2) return;
+// face into a voxel of the next brick is still covered.  Bricks of 4^3 read
+// their rows of up to 8 bytes as two words, the second overlapping the first,
+// and look at the labels only once the words have differed (a phantom is mostly
+// uniform): byte by byte, 216 loads a brick took 95 us at 325^3.
+__device__ inline void brick_set(const McPrep& P, long i) {
+  const int nx = P.nx, ny = P.ny, nz = P.nz, b = P.brick, nb0 = P.ray.nb[0], nb1 = P.ray.nb[1];
   const int bx = (int)(i % nb0), by = (int)((i / nb0) % nb1), bz = (int)(i / ((long)nb0 * nb1));
   const int x0 = max(bx * b - 1, 0), x1 = min(bx * b + b, nx - 1);
   const int y0 = max(by * b - 1, 0), y1 = min(by * b + b, ny - 1);
   const int z0 = max(bz * b - 1, 0), z1 = min(bz * b + b, nz - 1);
   uint32_t m = 0;
-  for (int z = z0; z <= z1; ++z)
-    for (int y = y0; y <= y1; ++y) {
-      const uint8_t* row = labels + ((size_t)z * ny + y) * nx;
-      for (int x = x0; x <= x1; ++x) m |= label_bit(row[x]);
+  if (x1 - x0 < 3 || x1 - x0 > 7) {
+    for (int z = z0; z <= z1; ++z)
+      for (int y = y0; y <= y1; ++y) {
+        const uint8_t* row = P.labels + ((size_t)z * ny + y) * nx;
+        int x = x0;
+        for (; x + 3 <= x1; x += 4) m |= label_bits(load_u32(row + x));
+        for (; x <= x1; ++x) m |= label_bit(row[x]);
+      }
+  } else {  // rows of two words, six rows (the last repeated past y1) in flight
+    uint32_t any = 0, all = ~0u;
+    for (int z = z0; z <= z1; ++z)
+      for (int y = y0; y <= y1; y += 6) {
+        uint32_t w[12];
+#pragma unroll
+        for (int r = 0; r < 6; ++r) {
+          const uint8_t* row = P.labels + ((size_t)z * ny + min(y + r, y1)) * nx;
+          w[2 * r] = load_u32(row + x0);
+          w[2 * r + 1] = load_u32(row + x1 - 3);
+        }
+#pragma unroll
+        for (int r = 0; r < 12; ++r) {
+          any |= w[r];
+          all &= w[r];
+        }
+        if (any != all) {  // not uniform so far: these words' own labels
+#pragma unroll
+          for (int r = 0; r < 12; ++r) m |= label_bits(w[r]);
+        }
+      }
+    // the words before the first difference equal the first word
+    m |= label_bits(load_u32(P.labels + ((size_t)z0 * ny + y0) * nx + x0));
+  }
+  P.bricks[i] = (uint8_t)m;
+}
+
+// Bounding box of the voxels whose label attenuates at some energy (labels are
+// clamped as in transport), over 16-byte chunks of the label map taken as one
+// array.  A chunk within a row costs two divisions; the box takes six atomics
+// per block.  One block per slice reading bytes row after row took 232 us at
+// 325^3.
+__device__ inline void support_box(McPrep& P, uint32_t block) {
+  __shared__ int red[4][6];
+  const uint32_t n = (uint32_t)P.nx * (uint32_t)P.ny * (uint32_t)P.nz;  // (below 2^32)
+  const uint32_t nx = (uint32_t)P.nx, ny = (uint32_t)P.ny, solid = P.solid;
+  const uint32_t lead = (uint32_t)((uintptr_t)P.labels & 15u);  // bytes of the first chunk before the map
+  const uint64_t chunks = ((uint64_t)lead + n + 15u) / 16u;
+  int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {-1, -1, -1};
+  auto add = [&](uint32_t first, uint32_t last) {  // voxels first .. last of one row
+    const uint32_t r = first / nx, z = r / ny, y = r - z * ny;
+    lo[0] = min(lo[0], (int)(first - r * nx)); hi[0] = max(hi[0], (int)(last - r * nx));
+    lo[1] = min(lo[1], (int)y); hi[1] = max(hi[1], (int)y);
+    lo[2] = min(lo[2], (int)z); hi[2] = max(hi[2], (int)z);
+  };
+  for (uint64_t c = (uint64_t)block * 256 + threadIdx.x; c < chunks; c += (uint64_t)P.box_blocks * 256) {
+    const int64_t at = (int64_t)c * 16 - lead;  // voxel of the chunk's first byte
+    uint32_t mask = 0;  // bit i: byte i attenuates
+    if (at >= 0 && at + 16 <= (int64_t)n) {
+      const uint4 w = *(const uint4*)(P.labels + at);
+      if ((w.x | w.y | w.z | w.w) == 0u && !(solid & 1u)) continue;
+      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        mask |= ((solid >> min((ws[i / 4] >> (8 * (i % 4))) & 255u, (uint32_t)kMaxLabels - 1u)) & 1u) << i;
+    } else {
+      for (int i = 0; i < 16; ++i)
+        if (at + i >= 0 && at + i < (int64_t)n)
+          mask |= ((solid >> min((uint32_t)P.labels[at + i], (uint32_t)kMaxLabels - 1u)) & 1u) << i;
     }
-  bricks[i] = (uint8_t)m;
+    if (mask == 0) continue;
+    const uint32_t first = (uint32_t)(at + __ffs((int)mask) - 1), last = (uint32_t)(at + 31 - __clz((int)mask));
+    if (first / nx == last / nx) {
+      add(first, last);
+    } else {
+      for (int i = 0; i < 16; ++i)
+        if ((mask >> i) & 1u) add((uint32_t)(at + i), (uint32_t)(at + i));
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    for (int a = 0; a < 3; ++a) {
+      lo[a] = min(lo[a], __shfl_xor(lo[a], o, 64));
+      hi[a] = max(hi[a], __shfl_xor(hi[a], o, 64));
+    }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0)
+    for (int a = 0; a < 3; ++a) {
+      red[w][a] = lo[a];
+      red[w][3 + a] = hi[a];
+    }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int a = threadIdx.x;
+    int v = red[0][a];
+    for (int i = 1; i < 4; ++i) v = a < 3 ? min(v, red[i][a]) : max(v, red[i][a]);
+    if (a < 3 && v != INT_MAX) atomicMin(&P.box[a], v);
+    if (a >= 3 && v >= 0) atomicMax(&P.box[a], v);
+  }
+}
+
+// The job whose blocks of a shared grid include block b (begin: its first).
+template <class F>
+__device__ inline int job_of_block(int n_jobs, uint32_t b, F begin) {
+  int lo = 0, hi = n_jobs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (begin(mid) <= b) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+// Flight boxes and brick sets of all jobs in one launch: they read the same
+// labels and do not depend on each other.  (A launch each per job, with the box
+// read back by the host in between, took 4.3 of 10 ms of 24 uneven jobs.)
+__global__ __launch_bounds__(256) void mc_prep_kernel(McPrep* __restrict__ preps, int n_jobs) {
+  const int j = job_of_block(n_jobs, blockIdx.x, [&](int i) { return preps[i].prep_begin; });
+  McPrep& P = preps[j];
+  const uint32_t b = blockIdx.x - P.prep_begin;
+  if (b < P.box_blocks) {
+    support_box(P, b);
+    return;
+  }
+  const long i = (long)(b - P.box_blocks) * 256 + threadIdx.x;
+  if (i < (long)P.ray.nb[0] * P.ray.nb[1] * P.ray.nb[2]) brick_set(P, i);
+}
+
+// The flight box along axis a: [lo, hi) of the attenuating voxels, or of the
+// phantom when nothing attenuates.
+__device__ inline void flight_box(const McPrep& P, int a, double& lo, double& hi) {
+  const double v = P.vox[a];
+  const int dims[3] = {P.nx, P.ny, P.nz};
+  const bool any = P.box[3] >= 0;
+  lo = any ? xadd(P.ray.org[a], xmul((double)P.box[a], v)) : P.ray.org[a];
+  hi = xadd(P.ray.org[a], xmul((double)(any ? P.box[3 + a] + 1 : dims[a]), v));
+}
+
+// Flights are clipped to that box: outside it mu is 0, so no history changes,
+// and no Woodcock steps are spent crossing the empty margin of the phantom.
+__device__ inline void set_job_box(const McPrep& P, McJob& J) {
+  if (P.box[3] < 0) return;
+  double lo[3], hi[3];
+  for (int a = 0; a < 3; ++a) flight_box(P, a, lo[a], hi[a]);
+  J.bx0 = (float)lo[0]; J.bx1 = (float)hi[0];
+  J.by0 = (float)lo[1]; J.by1 = (float)hi[1];
+  J.bz0 = (float)lo[2]; J.bz1 = (float)hi[2];
+}
+
+__global__ void mc_boxes_kernel(const McPrep* __restrict__ preps, McJob* __restrict__ jobs, int n_jobs) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_jobs) set_job_box(preps[i], jobs[i]);
 }
 
 // One thread per (view, pixel): the union of the brick sets along the segment
 // source -> pixel centre inside the flight box, by index-stepping traversal of
 // the brick grid (every crossing recomputed from its plane index), or
-// kAnyLabel if the segment misses the box.
-__global__ __launch_bounds__(256) void ray_sets_kernel(RayGrid R, const double* __restrict__ cs64, int view_begin,
-                                                       int n_views, const uint8_t* __restrict__ bricks,
-                                                       uint8_t* __restrict__ sets) {
-  const long npix = (long)R.nu * R.nv;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= npix * n_views) return;
-  const int kk = (int)(i / npix);
-  const int pix = (int)(i - (long)kk * npix);
+// kAnyLabel if the segment misses the box.  A block's rays share a view, hence
+// the source: with PLANES the distances of all brick planes from it are formed
+// once per block in LDS, which leaves one FP64 multiply per axis and step (the
+// walk of ~60 bricks a ray issues FP64 and integer VALU all the time: 5.2 ms at
+// 325^3 / 512^2 / 360 views with the planes formed at every step, 3.2 ms so).
+template <bool PLANES>
+__global__ __launch_bounds__(kRayBlock) void ray_sets_kernel(const McPrep* __restrict__ preps, McJob* __restrict__ jobs,
+                                                             int n_jobs) {
+  extern __shared__ double planes[];
+  const int j = job_of_block(n_jobs, blockIdx.x, [&](int i) { return preps[i].ray_begin; });
+  const McPrep& P = preps[j];
+  const RayGrid& R = P.ray;
+  const int view_begin = jobs[j].view_begin;
+  const int npix = R.nu * R.nv, per_view = (npix + kRayBlock - 1) / kRayBlock;
+  const uint32_t b = blockIdx.x - P.ray_begin;
+  const int kk = (int)(b / (uint32_t)per_view), pix = (int)(b - (uint32_t)kk * (uint32_t)per_view) * kRayBlock + (int)threadIdx.x;
+  if (b == 0 && threadIdx.x == 0) set_job_box(P, jobs[j]);
+  const double cb = P.cs64[2 * (view_begin + kk)], sb = P.cs64[2 * (view_begin + kk) + 1];
+  const double S[3] = {xmul(-R.sod, cb), xmul(-R.sod, sb), 0.0};
+  const int nb0 = R.nb[0], nb1 = R.nb[1], nb2 = R.nb[2];
+  if (PLANES) {
+    for (int i = threadIdx.x; i < nb0 + nb1 + nb2 + 3; i += kRayBlock) {
+      const int a = i <= nb0 ? 0 : (i <= nb0 + 1 + nb1 ? 1 : 2);
+      const int p = a == 0 ? i : (a == 1 ? i - nb0 - 1 : i - nb0 - nb1 - 2);
+      const double org = a == 0 ? R.org[0] : (a == 1 ? R.org[1] : R.org[2]);
+      const double bw = a == 0 ? R.bw[0] : (a == 1 ? R.bw[1] : R.bw[2]);
+      planes[i] = xsub(xadd(org, xmul((double)p, bw)), a == 0 ? S[0] : (a == 1 ? S[1] : S[2]));
+    }
+    __syncthreads();
+  }
+  if (pix >= npix) return;
+  uint8_t* out = P.sets + (size_t)kk * npix + pix;
   const int iv = pix / R.nu, iu = pix - iv * R.nu;
-  const double cb = cs64[2 * (view_begin + kk)], sb = cs64[2 * (view_begin + kk) + 1];
   const double yp = xmul(xsub(xadd((double)iu, 0.5), R.un0), R.u_step);
   const double zp = xmul(xsub(xadd((double)iv, 0.5), R.vn0), R.v_step);
-  const double S[3] = {xmul(-R.sod, cb), xmul(-R.sod, sb), 0.0};
-  const double P[3] = {xsub(xmul(R.xd, cb), xmul(yp, sb)), xadd(xmul(R.xd, sb), xmul(yp, cb)), zp};
+  const double T[3] = {xsub(xmul(R.xd, cb), xmul(yp, sb)), xadd(xmul(R.xd, sb), xmul(yp, cb)), zp};
   double d[3], inv[3];
   double lo = 0.0, hi = 1.0;
-  uint32_t m = 0;
   bool miss = false;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    d[a] = xsub(P[a], S[a]);
+    double c0, c1;
+    flight_box(P, a, c0, c1);
+    d[a] = xsub(T[a], S[a]);
     if (d[a] != 0.0) {
       inv[a] = 1.0 / d[a];
-      const double ta = xmul(xsub(R.c0[a], S[a]), inv[a]), tb = xmul(xsub(R.c1[a], S[a]), inv[a]);
+      const double ta = xmul(xsub(c0, S[a]), inv[a]), tb = xmul(xsub(c1, S[a]), inv[a]);
       const double tl = ta < tb ? ta : tb, th = ta < tb ? tb : ta;
       if (tl > lo) lo = tl;
       if (th < hi) hi = th;
     } else {
       inv[a] = 0.0;
-      if (S[a] < R.c0[a] || S[a] >= R.c1[a]) miss = true;
+      if (S[a] < c0 || S[a] >= c1) miss = true;
     }
   }
   if (miss || !(hi > lo)) {
-    sets[i] = (uint8_t)kAnyLabel;
+    *out = (uint8_t)kAnyLabel;
     return;
   }
   const double span = xsub(hi, lo);
@@ -905,116 +1098,88 @@ __global__ __launch_bounds__(256) void ray_sets_kernel(RayGrid R, const double* 
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const double q = xadd(S[a], xmul(tm, d[a]));
-    const int j = (int)floor(xsub(q, R.org[a]) / R.bw[a]);
-    idx[a] = j < 0 ? 0 : (j > R.nb[a] - 1 ? R.nb[a] - 1 : j);
+    const int i = (int)floor(xsub(q, R.org[a]) / R.bw[a]);
+    idx[a] = i < 0 ? 0 : (i > R.nb[a] - 1 ? R.nb[a] - 1 : i);
   }
-  for (int guard = 0; guard < 4 * (R.nb[0] + R.nb[1] + R.nb[2]) + 8; ++guard) {
-    m |= bricks[((size_t)idx[2] * R.nb[1] + idx[1]) * R.nb[0] + idx[0]];
-    double tn[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      if (d[a] > 0.0) tn[a] = xmul(xsub(xadd(R.org[a], xmul((double)(idx[a] + 1), R.bw[a])), S[a]), inv[a]);
-      else if (d[a] < 0.0) tn[a] = xmul(xsub(xadd(R.org[a], xmul((double)idx[a], R.bw[a])), S[a]), inv[a]);
-      else tn[a] = INFINITY;
-    }
-    int a = 0;
-    if (tn[1] < tn[a]) a = 1;
-    if (tn[2] < tn[a]) a = 2;
-    if (!(tn[a] < hi)) break;
-    idx[a] += d[a] > 0.0 ? 1 : -1;
-    if (idx[a] < 0 || idx[a] >= R.nb[a]) break;
+  // per axis: index of the next plane, and the crossings left before the grid's end
+  const int s0 = d[0] > 0.0 ? 1 : -1, s1 = d[1] > 0.0 ? 1 : -1, s2 = d[2] > 0.0 ? 1 : -1;
+  int p0 = idx[0] + (s0 > 0), p1 = idx[1] + (s1 > 0), p2 = idx[2] + (s2 > 0);
+  int left0 = s0 > 0 ? nb0 - 1 - idx[0] : idx[0], left1 = s1 > 0 ? nb1 - 1 - idx[1] : idx[1],
+      left2 = s2 > 0 ? nb2 - 1 - idx[2] : idx[2];
+  uint32_t at = ((uint32_t)idx[2] * (uint32_t)nb1 + (uint32_t)idx[1]) * (uint32_t)nb0 + (uint32_t)idx[0];
+  auto crossing = [&](int a, int p) {
+    if (d[a] == 0.0) return (double)INFINITY;
+    const int first = a == 0 ? 0 : (a == 1 ? nb0 + 1 : nb0 + nb1 + 2);
+    return xmul(PLANES ? planes[first + p] : xsub(xadd(R.org[a], xmul((double)p, R.bw[a])), S[a]), inv[a]);
+  };
+  uint32_t m = 0, cur = P.bricks[at];  // (a brick's set is waited for a step later)
+  for (;;) {
+    const double t0 = crossing(0, p0), t1 = crossing(1, p1), t2 = crossing(2, p2);
+    const bool c1 = t1 < t0;
+    const double t01 = c1 ? t1 : t0;
+    const bool c2 = t2 < t01;
+    if (!((c2 ? t2 : t01) < hi)) break;
+    const bool y = c1 && !c2, x = !c1 && !c2;
+    if ((c2 ? left2 : (c1 ? left1 : left0)) == 0) break;
+    p0 += x ? s0 : 0;
+    p1 += y ? s1 : 0;
+    p2 += c2 ? s2 : 0;
+    left0 -= x;
+    left1 -= y;
+    left2 -= c2;
+    at += (uint32_t)(c2 ? s2 * nb0 * nb1 : (c1 ? s1 * nb0 : s0));
+    const uint32_t next = P.bricks[at];
+    m |= cur;
+    cur = next;
   }
-  sets[i] = (uint8_t)m;
+  *out = (uint8_t)(m | cur);
 }
 
-hipError_t launch_brick_sets(const uint8_t* labels, int nx, int ny, int nz, int b, const int nb[3], uint8_t* bricks,
-                             hipStream_t s) {
-  const long n = (long)nb[0] * nb[1] * nb[2];
-  if (n <= 0 || b < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(brick_sets_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, labels, nx, ny, nz, b,
-                     nb[0], nb[1], nb[2], bricks);
+hipError_t launch_mc_prep(McPrep* preps, int n_jobs, uint32_t prep_blocks, hipStream_t s) {
+  if (n_jobs < 1 || prep_blocks == 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(mc_prep_kernel, dim3(prep_blocks), dim3(256), 0, s, preps, n_jobs);
   return hipGetLastError();
 }
 
-hipError_t launch_ray_sets(const RayGrid& R, const double* cs64, int view_begin, int n_views, const uint8_t* bricks,
-                           uint8_t* sets, hipStream_t s) {
-  const long n = (long)R.nu * R.nv * n_views;
-  if (n <= 0) return hipSuccess;
-  if ((n + 255) / 256 > 0x7fffffffL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(ray_sets_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, R, cs64, view_begin,
-                     n_views, bricks, sets);
+hipError_t launch_ray_sets(const McPrep* preps, McJob* jobs, int n_jobs, uint32_t ray_blocks, uint64_t max_planes,
+                           hipStream_t s) {
+  if (n_jobs < 1 || ray_blocks == 0) return hipErrorInvalidValue;
+  // the planes of grids up to 4096 bricks along the axes together fit in 32 KB of LDS
+  if (max_planes <= 4096)
+    hipLaunchKernelGGL(ray_sets_kernel<true>, dim3(ray_blocks), dim3(kRayBlock), sizeof(double) * max_planes, s, preps,
+                       jobs, n_jobs);
+  else
+    hipLaunchKernelGGL(ray_sets_kernel<false>, dim3(ray_blocks), dim3(kRayBlock), 0, s, preps, jobs, n_jobs);
   return hipGetLastError();
 }
 
-__global__ void mc_reset_kernel(unsigned int* queue, McCounters* counters, int n_jobs) {
+hipError_t launch_mc_boxes(const McPrep* preps, McJob* jobs, int n_jobs, hipStream_t s) {
+  hipLaunchKernelGGL(mc_boxes_kernel, dim3((n_jobs + 63) / 64), dim3(64), 0, s, preps, jobs, n_jobs);
+  return hipGetLastError();
+}
+
+__global__ void mc_reset_kernel(unsigned int* queue, McCounters* counters, int n_counters, int waves_per_block,
+                                int grid) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kMcQueues) queue[i * kMcQueueStride] = 0u;
-  if (i < n_jobs) counters[i] = McCounters{};
+  if (i < kMcQueues) queue[i * kMcQueueStride] = mc_queue_start(i, waves_per_block, grid);
+  if (i == 0) queue[kMcSpentWord] = 0u;
+  if (i < n_counters) counters[i] = McCounters{};
 }
 
-// Bounding box of the voxels whose label attenuates at some energy
-// (`solid` has bit l set for such labels; labels are clamped as in transport):
-// box = {x_min, y_min, z_min, x_max, y_max, z_max}, initialised by the caller
-// to {INT_MAX x 3, -1 x 3}.  One block per z slice, reduced in the block, so
-// the box takes six atomics per slice.
-__global__ __launch_bounds__(256) void support_box_kernel(const uint8_t* __restrict__ labels, int nx, int ny, int nz,
-                                                          uint32_t solid, int* __restrict__ box) {
-  __shared__ int red[4][4];
-  const int z = blockIdx.x;
-  const uint8_t* slice = labels + (size_t)z * ny * nx;
-  int xmin = INT_MAX, xmax = -1, ymin = INT_MAX, ymax = -1;
-  for (int y = 0; y < ny; ++y) {
-    for (int x = threadIdx.x; x < nx; x += 256) {
-      const int lab = min((int)slice[(size_t)y * nx + x], kMaxLabels - 1);
-      if ((solid >> lab) & 1u) {
-        xmin = min(xmin, x);
-        xmax = max(xmax, x);
-        ymin = min(ymin, y);
-        ymax = y;
-      }
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    xmin = min(xmin, __shfl_xor(xmin, o, 64));
-    xmax = max(xmax, __shfl_xor(xmax, o, 64));
-    ymin = min(ymin, __shfl_xor(ymin, o, 64));
-    ymax = max(ymax, __shfl_xor(ymax, o, 64));
-  }
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    red[w][0] = xmin; red[w][1] = xmax; red[w][2] = ymin; red[w][3] = ymax;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < 4; ++i) {
-      xmin = min(xmin, red[i][0]); xmax = max(xmax, red[i][1]);
-      ymin = min(ymin, red[i][2]); ymax = max(ymax, red[i][3]);
-    }
-    if (xmax >= 0) {
-      atomicMin(box + 0, xmin); atomicMin(box + 1, ymin); atomicMin(box + 2, z);
-      atomicMax(box + 3, xmax); atomicMax(box + 4, ymax); atomicMax(box + 5, z);
-    }
-  }
-}
-
-hipError_t launch_support_box(const uint8_t* labels, int nx, int ny, int nz, uint32_t solid, int* box, hipStream_t s) {
-  if (nx < 1 || ny < 1 || nz < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(support_box_kernel, dim3(nz), dim3(256), 0, s, labels, nx, ny, nz, solid, box);
-  return hipGetLastError();
-}
-
-hipError_t launch_mc_reset(unsigned int* queue, McCounters* counters, int n_jobs, hipStream_t s) {
-  const int n = n_jobs > 1 ? n_jobs : 1;
-  hipLaunchKernelGGL(mc_reset_kernel, dim3((n + 255) / 256), dim3(256), 0, s, queue, counters, n_jobs);
+hipError_t launch_mc_reset(unsigned int* queue, McCounters* counters, int n_counters, int block, int grid,
+                           hipStream_t s) {
+  const int n = std::max(n_counters, (int)kMcQueues);
+  hipLaunchKernelGGL(mc_reset_kernel, dim3((n + 255) / 256), dim3(256), 0, s, queue, counters, n_counters, block / 64,
+                     grid);
   return hipGetLastError();
 }
 
 hipError_t launch_mc_transport(const McJob* jobs_dev, int n_jobs, uint64_t total_units, uint32_t chunk,
-                               unsigned int* queue, McCounters* counters, int block, int grid, hipStream_t s) {
-  if (block % 64 || block > 256 || block <= 0 || grid <= 0 || chunk == 0) return hipErrorInvalidValue;
+                               unsigned int* queue, McCounters* counters, int slots, int block, int grid,
+                               hipStream_t s) {
+  if (block % 64 || block > 256 || block <= 0 || grid <= 0 || chunk == 0 || slots < 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(mc_transport_kernel, dim3(grid), dim3(block), sizeof(WaveTables) * (block / 64), s, jobs_dev,
-                     n_jobs, total_units, chunk, queue, counters);
+                     n_jobs, total_units, chunk, queue, counters, slots);
   return hipGetLastError();
 }
 

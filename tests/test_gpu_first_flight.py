@@ -115,3 +115,30 @@ def test_full_workload_steps_halved(ctx):
     assert stb["steps"] < 0.5 * sta["steps"]
     for k in ("tallied_primary", "photo", "compton"):
         assert abs(sta[k] - stb[k]) < 0.01 * sta[k], k
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (9, 2, 33), (6, 31, 17), (21, 18, 64), (2, 3, 300)])
+@pytest.mark.parametrize("brick", [1, 3, 4, 7])
+@pytest.mark.parametrize("offset", [0, 1, 6])
+def test_sets_of_odd_phantoms_match_oracle(ctx, oracle, ref_tables, shape, brick, offset):
+    """Label maps of rows shorter and longer than the words and 16-byte chunks the set-up kernels
+    read, starting at any byte, with bricks of every remainder: the flight box and the label sets
+    formed from them equal the oracle's."""
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd.mc import first_flight_sets
+    from monte_amd.phantoms import MATERIALS, LabelPhantom
+
+    rng = np.random.default_rng(sum(shape) + brick)
+    lab = np.where(rng.random(shape) < 0.3, rng.choice([1, 2, 7], size=shape), 0).astype(np.uint8)
+    lab.reshape(-1)[lab.size // 2] = 1  # something attenuates
+    v = 6.0 / max(shape)
+    ph = LabelPhantom(lab, (v, v, v), list(MATERIALS) + [(0, 0.7)] * 5)
+    geom = G.small(n_views=3).replace(nu=29, nv=23, du=0.6, dv=0.6, angle0=0.3)
+    buf = torch.zeros(lab.size + 16, dtype=torch.uint8, device="cuda")
+    dev = buf[offset:offset + lab.size]
+    dev.copy_(torch.from_numpy(lab.reshape(-1)).cuda())
+    got = first_flight_sets(ph, geom, brick, labels_dev=dev.view(shape), ctx=ctx).cpu().numpy()
+    ref = oracle.ray_masks(oracle_geom(oracle, geom), oracle_phantom(oracle, ph), oracle.tables(ref_tables), brick)
+    assert np.array_equal(got, ref)
