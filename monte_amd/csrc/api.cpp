@@ -516,6 +516,7 @@ int prepare_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per
   for (int i = 0; i < n; ++i) {
     McJob& J = hj[i].d;
     J.ray_set = preps[i].sets;
+    J.solid_set = (preps[i].solid & 15u) | (preps[i].solid ? 16u : 0u);
     J.tables = (const McTables*)(base + Lo.tab_off) + i;
     J.spectrum_cdf = hj[i].cdf.empty() ? nullptr : (const float*)(base + Lo.cdf_off[i]);
     J.view_cs = (const float2*)(base + Lo.cs_off[i]);

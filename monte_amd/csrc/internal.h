@@ -136,6 +136,7 @@ struct McJob {
   float e_kev;
   int max_int, coherent;
   uint32_t key0, key1, job_id;
+  uint32_t solid_set;            // label-set bits that attenuate at some energy (bit 4: any label does)
   uint32_t photons_per_view;
   // Photon n of a view aims at pixel j = n mod (nu nv) in aim order (iv nu + iu),
   // in cycle c = n / (nu nv).  A work unit is a group of `tile_group` detector

@@ -308,7 +308,7 @@ __device__ inline void count_tallies(WaveTables& wt, int code) {
 }
 
 template <class JT>
-__device__ inline int tally(const Photon& p, const JT& J) {
+__device__ inline int tally_cell(const Photon& p, const JT& J, size_t& idx) {
   const float cx = p.cv, cy = p.sv;
   const float xq = p.px * cx + p.py * cy, yq = -p.px * cy + p.py * cx;
   const float ddx = p.dx * cx + p.dy * cy, ddy = -p.dx * cy + p.dy * cx;
@@ -324,13 +324,18 @@ __device__ inline int tally(const Photon& p, const JT& J) {
   int iu = (int)floorf(ui), iv = (int)floorf(vi);
   iu = iu > J.nu - 1 ? J.nu - 1 : iu;
   iv = iv > J.nv - 1 ? J.nv - 1 : iv;
-  const size_t idx = ((size_t)p.view * J.nu + iu) * J.nv + iv;
-  if (p.nint == 0) {
-    unsafeAtomicAdd(J.primary + idx, 1.0);
-    return kTallyPrimary;
-  }
-  unsafeAtomicAdd(J.scatter + idx, 1.0);
-  return kTallyScatter;
+  idx = ((size_t)p.view * J.nu + iu) * J.nv + iv;
+  return p.nint == 0 ? kTallyPrimary : kTallyScatter;
+}
+
+// Adds a photon that ends its flight here to its image; its tally code.
+template <class JT>
+__device__ inline int tally(const Photon& p, const JT& J) {
+  size_t idx = 0;
+  const int code = tally_cell(p, J, idx);
+  if (code == kTallyPrimary) unsafeAtomicAdd(J.primary + idx, 1.0);
+  if (code == kTallyScatter) unsafeAtomicAdd(J.scatter + idx, 1.0);
+  return code;
 }
 
 // Label set meaning "any label": the flight takes the global majorant.
@@ -465,10 +470,11 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
   const int q_first = (int)(blockIdx.x % kMcQueues);
   int q_own = q_first;   // the queue the wave draws from
   bool q_begun = false;  // the wave has had its first unit
-  // the current unit (wave-uniform): tiles [unit_t0, unit_t0 + unit_nt) over photon
-  // cycles [unit_cyc, unit_cyc_end); the next birth takes tile unit_t0 + unit_g of
-  // cycle unit_cyc
-  uint32_t unit_t0 = 0, unit_nt = 0, unit_g = 0, unit_cyc = 0, unit_cyc_end = 0;
+  // the current unit (wave-uniform): tiles [unit_t0, unit_t0 + unit_nt), each over
+  // photon cycles [unit_cyc0, unit_cyc_end); the next birth takes tile unit_t0 +
+  // unit_g of cycle unit_cyc
+  uint32_t unit_t0 = 0, unit_nt = 0, unit_g = 0, unit_cyc0 = 0, unit_cyc = 0, unit_cyc_end = 0;
+  uint64_t unit_act = 0;  // the tile's lanes (pixels) whose photons may collide
   int unit_view = 0;
   long long pending = -1;
   bool exhausted = false;
@@ -476,8 +482,6 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
   int buf_view = 0;                  // the view of the buffered photons, and its cos and sin
   float buf_cv = 0.f, buf_sv = 0.f;
   uint32_t buf_id0 = 0;              // photon index of the buffer's slot 0 (the tile's corner pixel)
-  uint32_t ray_tile = ~0u;           // the tile and view whose rays the buffer holds (~0u: none)
-  int ray_view = -1;
 
   int state = kDead;
   Photon p{};
@@ -520,7 +524,7 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
     const bool all_dead = (fly | coll) == 0;
 
     // 1) secure a work unit when lanes are idle and the current one is spent
-    if (dead != 0 && unit_cyc >= unit_cyc_end) {
+    if (dead != 0 && unit_g >= unit_nt) {
       if (pending < 0 && !exhausted) {
         // in round r = k / chunk, queue q hands out chunk r kMcQueues + (q + r) mod kMcQueues,
         // unit k mod chunk of it: the chunks of a round are dealt to the queues rotated by
@@ -564,7 +568,6 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
           if (switched) {
             if (job >= 0) flush(counters + job * slots + blockIdx.x % slots);
             job = pj;
-            ray_tile = ~0u;  // another job's geometry
           }
           // units run views fastest, then cycle blocks, then tile groups: the units in
           // flight share a few detector tiles, hence a thin z-slab of the phantom that
@@ -580,9 +583,10 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
             unit_t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tg * grp));
             unit_nt = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(grp, cjobs[pj].tiles - tg * grp));
             unit_g = 0;
-            unit_cyc = (uint32_t)__builtin_amdgcn_readfirstlane((int)(cb * cjobs[pj].cycle_block));
+            unit_cyc0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(cb * cjobs[pj].cycle_block));
+            unit_cyc = unit_cyc0;
             unit_cyc_end = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)min(unit_cyc + cjobs[pj].cycle_block, cjobs[pj].cycles));
+                (int)min(unit_cyc0 + cjobs[pj].cycle_block, cjobs[pj].cycles));
           }
           pending = -1;
           if (switched) {  // J is re-read for the new job at the top of the loop
@@ -603,10 +607,10 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
       }
       count_tallies(wt, code);
     }
-    if (all_dead && unit_cyc >= unit_cyc_end && pending < 0 && exhausted && buf_n == 0) break;
+    if (all_dead && unit_g >= unit_nt && pending < 0 && exhausted && buf_n == 0) break;
 
     // 2) refill dead lanes from the birth buffer, after filling it when it is empty
-    if (dead != 0 && (buf_n != 0 || unit_cyc < unit_cyc_end) && (popc(dead) >= kRefillBatch || fly == 0)) {
+    if (dead != 0 && (buf_n != 0 || unit_g < unit_nt) && (popc(dead) >= kRefillBatch || fly == 0)) {
       if (buf_n == 0) {
         // one tile of the unit in one cycle, one photon per lane with every lane
         // active: lane l aims at the centre of pixel (u_, v_) of the tile
@@ -622,7 +626,7 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
         CU32* vcs = (CU32*)Jp->view_cs + 2 * unit_view;  // read-only during the launch: scalar loads
         const float cv = __uint_as_float(vcs[0]), sv = __uint_as_float(vcs[1]);
         const bool on_det = u_ < (uint32_t)Jp->nu && v_ < (uint32_t)Jp->nv;
-        if (t != ray_tile || unit_view != ray_view) {
+        if (unit_cyc == unit_cyc0) {
           // the tile's rays in this view, one per lane: the first flight runs from the
           // source towards the pixel centre, its majorant comes from the labels the
           // line crosses, and it starts at the flight box (start_flight's clip)
@@ -647,12 +651,41 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
           wt.bb.d0[lane] = make_float4(dx, dy, dz, tin);
           wt.bb.t1[lane] = hit ? t1 : -1.f;
           wt.bb.set[lane] = (uint8_t)set;
-          ray_tile = t;
-          ray_view = unit_view;
+          // A ray that misses the flight box, or crosses only labels that never
+          // attenuate, sends every photon straight to the detector, whatever its
+          // energy: all of the unit's photons on it are tallied here with one add
+          // (sums of ones are exact).  On the full workload (a 15 cm phantom before a
+          // 61 cm detector) these are three photons in four.
+          const bool may = on_det && hit && (set & Jp->solid_set) != 0;
+          unit_act = __ballot(may);
+          const bool inert = on_det && !may;
+          if (unit_act != __ballot(on_det)) {
+            const bool short_ = unit_cyc_end == Jp->cycles &&
+                                (uint64_t)(Jp->cycles - 1) * npix + pix >= Jp->photons_per_view;
+            const uint32_t full = unit_cyc_end - unit_cyc0;
+            int code = -1;
+            if (inert) {
+              Photon q;
+              q.view = unit_view;
+              q.cv = cv; q.sv = sv;
+              q.dx = dx; q.dy = dy; q.dz = dz;
+              q.px = -Jp->sod * cv; q.py = -Jp->sod * sv; q.pz = 0.f;
+              q.nint = 0;
+              size_t idx = 0;
+              code = tally_cell(q, *Jp, idx);
+              const uint32_t n = full - (short_ ? 1u : 0u);
+              if (code == kTallyPrimary && n != 0) unsafeAtomicAdd(Jp->primary + idx, (double)n);
+            }
+            const uint64_t mi = __ballot(inert), mp = __ballot(code == kTallyPrimary), ms = __ballot(short_);
+            if (lane == 0) {
+              atomicAdd(&wt.stats[kStatHistories], (unsigned long long)full * popc(mi) - popc(mi & ms));
+              atomicAdd(&wt.stats[kStatTp], (unsigned long long)full * popc(mp) - popc(mp & ms));
+            }
+          }
         }
         bool born = false;
         int bcode = -1;  // tally code of a photon that misses the flight box
-        const bool valid = on_det && n64 < Jp->photons_per_view;
+        const bool valid = ((unit_act >> lane) & 1u) != 0 && n64 < Jp->photons_per_view;
         if (valid) {
           Photon q;
           q.view = unit_view;
@@ -700,9 +733,9 @@ __global__ __launch_bounds__(256) void mc_transport_kernel(const McJob* __restri
         buf_cv = cv;
         buf_sv = sv;
         buf_id0 = (uint32_t)((uint64_t)unit_cyc * npix + tv * kTileV * (uint32_t)Jp->nu + tu * kTileU);
-        if (++unit_g == unit_nt) {  // the unit's tiles are done for this cycle
-          unit_g = 0;
-          ++unit_cyc;
+        if (unit_act == 0 || ++unit_cyc == unit_cyc_end) {  // the tile is done
+          ++unit_g;
+          unit_cyc = unit_cyc0;
         }
       }
       const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(dead >> 32),

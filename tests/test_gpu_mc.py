@@ -110,6 +110,37 @@ def test_mc_partial_tiles_and_cycles(ctx, oracle, nu, nv, photons, coherent):
     assert abs(prim.sum() - p_ref.sum()) <= max(3, 1e-3 * p_ref.sum())
 
 
+@pytest.mark.parametrize("nu,nv,photons", [(33, 19, 200), (33, 19, 627), (33, 19, 60_000), (24, 24, 100_001)])
+@pytest.mark.parametrize("brick", [0, 4])
+def test_mc_rays_that_cannot_collide(ctx, oracle, nu, nv, photons, brick):
+    """Photons on rays that miss the flight box, or cross only labels that do not attenuate, are
+    tallied a unit at a time: a phantom that covers a few pixels (label 3 is air inside its box),
+    views that end within a cycle or before the last pixel, and no rays left to simulate in most
+    tiles.  Every primary pixel and statistic equals the oracle's."""
+    from monte_amd import geometry as G
+    from monte_amd.phantoms import MATERIALS, LabelPhantom
+
+    lab = np.full((9, 9, 9), 3, np.uint8)
+    lab[0, 0, 0] = lab[8, 8, 8] = lab[3:6, 3:6, 3:6] = 1
+    ph = LabelPhantom(lab, (0.3, 0.3, 0.3), list(MATERIALS) + [(0, 0.0)])
+    geom = G.small(n_views=4).replace(nu=nu, nv=nv, du=0.5, dv=0.5)
+    saved = ctx.tuning
+    ctx.set_tuning(mc_ray_brick=brick)
+    try:
+        prim, scat, st, p_ref, s_ref, st_ref = _mc_pair(ctx, oracle, geom, ph, photons, e_kev=60.0, coherent=0)
+    finally:
+        ctx.set_tuning(**saved)
+    print(nu, nv, photons, brick, "gpu", st, "cpu", st_ref)
+    assert st["histories"] == st_ref["histories"] == photons * geom.n_views
+    assert st["tallied_primary"] + st["tallied_scatter"] + st["missed"] + st["photo"] + st["capped"] == \
+        st["histories"]
+    assert prim.sum() == st["tallied_primary"] and scat.sum() == st["tallied_scatter"]
+    empty = p_ref == p_ref.max()  # rays that lose nothing
+    assert empty.mean() > 0.4 or photons < nu * nv
+    assert np.array_equal(prim[empty], p_ref[empty])
+    assert np.mean(prim == p_ref) > 0.99 and abs(prim.sum() - p_ref.sum()) <= max(3, 1e-4 * p_ref.sum())
+
+
 @pytest.mark.parametrize("label", [1, 2])
 @pytest.mark.parametrize("coherent", [0, 1])
 def test_mc_one_voxel_phantom(ctx, oracle, label, coherent):
