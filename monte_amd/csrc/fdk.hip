@@ -461,8 +461,8 @@ __device__ inline double base_z(const BpGrid& g, int zb) {
 // the base voxel's coordinate, the step per voxel and the window.  Integers add
 // without rounding, so a coordinate is within 2^-(kVBits + 1) rows x 9 of the
 // FP64 line; as FP32 multiply-adds of the step they were 2^-21 off (|f| up to 16).
-// Voxels of a tile that fits in LDS (at most 62 rows, 16 voxels) step by less
-// than 4.1 rows, so a group stays within +-33 rows of its base.
+// The tiled kernel takes steps of up to 4.5 rows per voxel, so a group stays
+// within +-37 rows of its base.
 constexpr int kVBits = 25;
 struct GroupV {
   int ivb;
@@ -570,46 +570,56 @@ struct Taps {
 constexpr int kRegionViews = 32;  // views whose patch origins are found at a time
 
 template <int ZC, int NQ, bool ZEROS>
-__global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __restrict__ pad,
+__global__ __launch_bounds__(1024) void backproject_kernel(const float* __restrict__ pad,
                                                              const BpView* __restrict__ views, int view0,
                                                              int nviews, BpGrid g, float* __restrict__ vol,
                                                              int accumulate, int tile_x, int tiles_x, int tiles_y,
-                                                             int patch_rows, int turn) {
+                                                             int patch_rows, int turn, int stack) {
   using L = PatchLayout<NQ>;
-  extern __shared__ float patch[];  // two patches of patch_rows rows, one read while the other is filled
-  __shared__ int2 region[2][kRegionViews];
+  // per group of 4 waves, two patches of patch_rows rows, one read while the other is filled
+  extern __shared__ float patches[];
+  __shared__ int2 regions[4][2][kRegionViews];
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int per_z = tiles_x * tiles_y;
   const int zc = t / per_z;
   const int rem = t - zc * per_z;
   const int ty_t = rem / tiles_x, tx_t = rem - ty_t * tiles_x;
-  const int tile_y = 256 / tile_x;
-  const int tid = threadIdx.x;
+  const int tile_y = 256 / (tile_x * stack);
+  // The block's groups of 256 threads share its views out (one group when there are
+  // tiles enough); their sums are added in order at the end.
+  const int tid = threadIdx.x & 255, group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), groups = blockDim.x >> 8;
+  const int first_view = view0 + (int)((long)group * nviews / groups);
+  const int my_views = view0 + (int)((long)(group + 1) * nviews / groups) - first_view;
+  const int loop_views = (nviews + groups - 1) / groups;
   // columns up to (xb, yb) are owned: all of them, or the first quadrant or half of the orbits
   const int xb = NQ == 4 ? (g.nx + 1) / 2 : g.x1, yb = NQ > 1 ? (g.ny + 1) / 2 : g.ny;
   const int tx0 = (NQ > 1 ? 0 : g.x0) + tx_t * tile_x, ty0 = ty_t * tile_y;
   // a wave takes 8 x 8 columns of the tile: the smallest patch, so its taps share
   // words and fewer rows of them meet in one bank
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wx = tile_x / 8;
-  const int xw = tx0 + wave % wx * 8, yw = ty0 + wave / wx * 8;
+  const int wz = stack == 1 ? 0 : wave, wt = stack == 1 ? wave : 0;  // (its place along z and in the tile)
+  const int xw = tx0 + wt % wx * 8, yw = ty0 + wt / wx * 8;
   const bool idle = xw >= xb || yw >= yb;  // (a wave past the edge only copies)
   const int x = min(xw + lane % 8, xb - 1), y = min(yw + lane / 8, yb - 1);  // (past the end: repeats a column, never stored)
-  const int z0 = zc * ZC;
-  const int zb = (z0 / kZBase) * kZBase, joff = z0 - zb - kZMid;
+  const int zt = zc * ZC * stack, z0 = zt + wz * ZC;  // the tile's first voxel and the wave's
+  // its groups of 16 start at zb; its first voxel's place from the middle of its group
+  const int zb = ZC % kZBase == 0 ? z0 : (z0 / kZBase) * kZBase, joff = ZC % kZBase == 0 ? -kZMid : z0 - zb - kZMid;
   const int patch_words = patch_rows * L::kRS;
+  float* const patch = patches + group * 2 * patch_words;
+  int2 (*const region)[kRegionViews] = regions[group];
   const int part = g.n_views / NQ;  // views of 1/NQ of a turn
 
   // Patch origin (row, column of the padded view) of views [first, first + 32):
   // the sample coordinates are monotonic along any line of the tile, so their
   // minima lie at its corners.  8 lanes per view evaluate the 8 corners.
   auto find_regions = [&](int first) {
-    int tid = threadIdx.x;
+    int tid = threadIdx.x & 255;
     asm volatile("" : "+v"(tid));  // (opaque: the corners are formed here, not kept in registers over the views)
-    const int k = min(first + (tid >> 3), view0 + nviews - 1);
+    const int k = min(first + (tid >> 3), first_view + my_views - 1);
     const BpView& c = views[k];
     const double Xc = voxel_x(g, (tid & 1) ? min(tx0 + tile_x, xb) - 1 : tx0);
     const double Yc = voxel_y(g, (tid & 2) ? min(ty0 + tile_y, yb) - 1 : ty0);
-    const double Zc = base_z(g, (tid & 4) ? z0 + ZC - 1 : z0);
+    const double Zc = base_z(g, (tid & 4) ? zt + ZC * stack - 1 : zt);
     const double inv = recip64(fma(c.cx, Xc, fma(c.cy, Yc, c.c0)));
     const double su = fma(c.suk * fma(c.ax, Xc, c.ay * Yc), inv, c.su0), sv = fma(c.svk * inv, Zc, c.sv0);
     float u = (float)fmin(fmax(su, g.lo_u), g.hi_u), v = (float)fmin(fmax(sv, g.lo_v), g.hi_v);
@@ -620,7 +630,7 @@ __global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __rest
     }
     // (0.01: the voxels' own coordinates round differently)
     if ((tid & 7) == 0)
-      region[((first - view0) / kRegionViews) & 1][tid >> 3] =
+      region[((first - first_view) / kRegionViews) & 1][tid >> 3] =
           make_int2(max(floor_i(v - 0.01f) + kPadLo, 0), max(floor_i(u - 0.01f) + kPadLo, 0));
   };
 
@@ -629,7 +639,7 @@ __global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __rest
   // padded view repeat its last ones; no tap reads them.
   const uint32_t view_bytes = (uint32_t)g.rows * (uint32_t)g.pitch * 4u;
   auto copy = [&](int k, float* buf) {
-    const int2 o = region[((k - view0) / kRegionViews) & 1][(k - view0) % kRegionViews];
+    const int2 o = region[((k - first_view) / kRegionViews) & 1][(k - first_view) % kRegionViews];
     const int r0 = __builtin_amdgcn_readfirstlane(o.x), c0 = __builtin_amdgcn_readfirstlane(o.y);
     const uint32_t col = (uint32_t)min(c0 + lane % L::kCols, g.pitch - 1) * 4u;
     const int kq = NQ > 1 ? k % part : k, turned = NQ > 1 ? k / part : 0;
@@ -652,19 +662,19 @@ __global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __rest
 #pragma unroll
     for (int j = 0; j < ZC; ++j) acc[q][j] = 0.f;
 
-  find_regions(view0);
+  if (my_views > 0) find_regions(first_view);
   __syncthreads();
-  copy(view0, patch);
+  if (my_views > 0) copy(first_view, patch);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the copies are in LDS
   __syncthreads();
-  for (int i = 0; i < nviews; ++i) {
-    const int k = view0 + i;
-    const bool more = i + 1 < nviews;
+  for (int i = 0; i < loop_views; ++i) {
+    const int k = first_view + i;
+    const bool more = i + 1 < my_views;
     if (more) copy(k + 1, patch + ((i + 1) & 1) * patch_words);
     // the next batch of origins, half a batch ahead of its first use
-    if (i % kRegionViews == kRegionViews / 2 && i + kRegionViews / 2 < nviews)
+    if (i % kRegionViews == kRegionViews / 2 && i + kRegionViews / 2 < my_views)
       find_regions(k + kRegionViews / 2);
-    if (!idle) {
+    if (!idle && i < my_views) {
       const BpView& c = views[k];
       int xc = x, yc = y;
       asm volatile("" : "+v"(xc), "+v"(yc));  // (two registers kept over the views instead of four)
@@ -681,12 +691,12 @@ __global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __rest
       auto taps_of = [&](int j) {
         if (j % kZBase == 0) {
           cb = group_v(cc, c, base_z(g, zb + j + kZMid), g);
-          base = (i & 1) * patch_words + (cb.ivb + kPadLo - o.x) * L::kRS + (cc.iu + kPadLo - o.y);
+          base = (group * 2 + (i & 1)) * patch_words + (cb.ivb + kPadLo - o.x) * L::kRS + (cc.iu + kPadLo - o.y);
           asm volatile("" : "+v"(base));  // (keeps the constants out of the reads' offsets, which the taps need)
         }
         const int f = cb.f + (joff + j % kZBase) * cb.d;
         const int fc = clamp_i(f, cb.flo, cb.fhi);
-        const float* s = patch + (base + __mul24(fc >> kVBits, L::kRS));
+        const float* s = patches + (base + __mul24(fc >> kVBits, L::kRS));
         Taps<NQ> t;
         t.fv = kFracUnit * (float)((uint32_t)fc << (32 - kVBits));
         t.live = ZEROS || (in_window(cc, c, g, z0 + j) && in_mask(g, x, y, z0 + j));
@@ -726,8 +736,25 @@ __global__ __launch_bounds__(256, 4) void backproject_kernel(const float* __rest
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
   }
+  if (groups > 1) {  // group g hands its sums to group 0 through LDS, in order
+    for (int g1 = 1; g1 < groups; ++g1) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int j = 0; j < ZC; ++j)
+          if (group == g1) patches[(q * ZC + j) * 256 + tid] = acc[q][j];
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int j = 0; j < ZC; ++j)
+          if (group == 0) acc[q][j] += patches[(q * ZC + j) * 256 + tid];
+      __syncthreads();
+    }
+    if (group != 0) return;
+  }
   // (the lane's column again: kept over the views it would cost registers)
-  int tl = threadIdx.x;
+  int tl = threadIdx.x;  // (below 256: group 0)
   asm volatile("" : "+v"(tl));
   const int xs = xw + tl % 8, ys = yw + (tl & 63) / 8;
   if (xs >= xb || ys >= yb) return;
@@ -789,12 +816,21 @@ __global__ __launch_bounds__(1024) void backproject_direct_kernel(const float* _
     const float* src = pad + (size_t)k * view_stride;
     const uint32_t off0 = (uint32_t)(kPadLo * g.pitch + cc.iu + kPadLo);
     sv += joff * dv;
+    int zo = z0, xm = x;  // (opaque: voxel coordinates and mask squares are formed where they are used)
+    asm volatile("" : "+s"(zo), "+v"(xm));
+    // whether a lane's voxels come within a row of the window's edge
+    const long long sl = sv + (ZC - 1) * dv, one = 1LL << 32;
+    const bool edge = __any(min(sv, sl) < lo + one || max(sv, sl) > hi - one);
     const float wu = ZEROS || cc.ok ? cc.w : 0.f;
     const float w1 = wu * cc.fu, w0 = wu - w1;
 #pragma unroll
     for (int j = 0; j < ZC; ++j) {
-      const bool live = ZEROS || (in_window(cc, c, g, z0 + j) && in_mask(g, x, y, z0 + j));
-      const long long sc = sv < lo ? lo : (sv > hi ? hi : sv);
+      bool live = ZEROS || in_mask(g, xm, y, zo + j);
+      long long sc = sv;
+      if (edge) {
+        if (!ZEROS) live = live && in_window(cc, c, g, zo + j);
+        sc = sv < lo ? lo : (sv > hi ? hi : sv);
+      }
       const float fv = (float)(uint32_t)sc * 2.3283064365386963e-10f;  // 2^-32
       const float m0 = live ? w0 : 0.f, m1 = live ? w1 : 0.f;
       const float b0 = m0 * fv, b1 = m1 * fv;
@@ -842,28 +878,59 @@ static void patch_bounds(const BpGrid& g, const BpReach& r, int tile_x, int tile
   rows = wv < 1e6 ? (int)std::floor(wv + 0.03) + 3 : 1 << 20;
 }
 
+// Whether the patches of an orbit fit, two for each of `groups` in a CU's 160 KB of LDS.
+template <int NQ>
+static bool patch_fits(int rows, int cols, int groups) {
+  using L = PatchLayout<NQ>;
+  return cols <= L::kCols && rows <= L::kMaxRows && 2 * sizeof(float) * rows * L::kRS * groups <= 156 * 1024;
+}
+static bool patch_fits(int orbit, int rows, int cols, int groups) {
+  return orbit == 4 ? patch_fits<4>(rows, cols, groups)
+                    : (orbit == 2 ? patch_fits<2>(rows, cols, groups) : patch_fits<1>(rows, cols, groups));
+}
+
 // Which kernel takes a backprojection: a property of the scan alone (sizes of
 // the default tiling), so the volume does not depend on the tuned tile shape.
-//   4, 2 columns an orbit   1/4 or 1/2 of a turn maps the scan onto itself, the
-//                           patches fit, and at least 2 tiles per CU
-//   1 column                patches fit, and at least 2 tiles per CU
-//   0                       straight from memory
-// Fewer tiles leave the chip idle: 65^3 from 36 views (125 tiles) took 46 us as
-// tiles of the kernel before this one.
-template <int NQ>
-static bool patch_fits(int rows, int cols) { return cols <= PatchLayout<NQ>::kCols && rows <= PatchLayout<NQ>::kMaxRows; }
+struct BpPlan {
+  int orbit;   // columns a thread owns: 4 or 2 where 1/4 or 1/2 of a turn maps the scan onto itself, 1, or 0: straight from memory
+  int groups;  // groups of 4 waves that share a tile's views out
+  int zc;      // voxels per thread at most
+  int stack;   // 1: a block's 4 waves lie side by side over its columns; 4: one above the other
+};
 
-static int bp_orbits(const BpGrid& g, const BpReach& r) {
-  int rows, cols;
-  patch_bounds(g, r, 16, 16, 16, rows, cols);
-  auto tiles = [&](int nx, int ny) { return (long)((nx + 15) / 16) * ((ny + 15) / 16) * ((g.nz + 15) / 16); };
+// The tiled kernel runs where the patches fit and there are 512 groups of 4 waves
+// (2 per CU) at least: tiles of 16 voxels of z (32 for single columns, which
+// halves what the set-up costs a voxel), else of 8 or 4, whose views up to 4 groups
+// share; where 16 x 16 columns are too wide a patch, 8 x 8 of 4 times the
+// depth (99x72x92 on 373x75, 3 pixels a voxel: 0.92 ms with its adjoint straight
+// from memory).  117x83x109 from 61 views of 175x94 (252 tiles) took 143 us
+// straight from memory and 114 us by the kernel before these.
+//
+// A region of fewer than 8 columns along x (the reference's 5 of 256) goes straight
+// from memory, whose waves take columns in a row: tiles of 8 x 8 would idle 24 lanes
+// of 64 (0.83 against 0.76 ms for the reference geometry's FDK).
+static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
+  // a group of 16 voxels has to stay within the 40 rows of group_v's clamp
+  if (g.x1 - g.x0 < 8 || !(r.svk * std::fabs(g.gsz) / (r.sod - r.rad) <= 4.5)) return {0, 1, 8, 1};
   // (the views' offsets from the first are 32-bit)
   const bool near = (double)g.n_views * g.rows * g.pitch * 4.0 < 4294967296.0;
   const int hx = (g.nx + 1) / 2, hy = (g.ny + 1) / 2;
-  if (near && r.turn != 0 && patch_fits<4>(rows, cols) && tiles(hx, hy) >= 512) return 4;
-  if (near && r.half && patch_fits<2>(rows, cols) && tiles(g.nx, hy) >= 512) return 2;
-  if (patch_fits<1>(rows, cols) && tiles(g.x1 - g.x0, g.ny) >= 512) return 1;
-  return 0;
+  for (int orbit : {4, 2, 1}) {
+    if (orbit > 1 && !(near && (orbit == 4 ? r.turn != 0 : r.half))) continue;
+    for (int stack : {1, 4})
+      for (int zc : {32, 16, 8, 4}) {
+        if (zc == 32 && (orbit > 1 || stack > 1 || !r.zeros)) continue;
+        const int nx = orbit == 4 ? hx : g.x1 - g.x0, ny = orbit > 1 ? hy : g.ny;
+        const int tx = stack == 1 ? 16 : 8, ty = 256 / (tx * stack);
+        int rows, cols;
+        patch_bounds(g, r, tx, ty, zc * stack, rows, cols);
+        const long tiles = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((g.nz + zc * stack - 1) / (zc * stack));
+        for (int groups : {1, 2, 4})
+          if (tiles * groups >= 512 && g.n_views >= 4 * groups && patch_fits(orbit, rows, cols, groups))
+            return {orbit, groups, zc, stack};
+      }
+  }
+  return {0, 1, 8, 1};
 }
 
 hipError_t launch_backproject(const float* filt_pad, const BpView* views, int view0, int nviews_chunk,
@@ -876,59 +943,59 @@ hipError_t launch_backproject(const float* filt_pad, const BpView* views, int vi
   if (zc != 4 && zc != 8 && zc != 16) return hipErrorInvalidValue;
   const int ncx = grid.x1 - grid.x0;
   if (ncx <= 0 || grid.ny <= 0 || grid.nz <= 0 || nviews_chunk <= 0) return hipSuccess;
-  int nq = bp_orbits(grid, reach);
-  if (nq > 1 && nviews_chunk != grid.n_views) {  // orbits need the whole turn
+  BpPlan plan = bp_plan(grid, reach);
+  if (plan.orbit > 1 && nviews_chunk != grid.n_views) {  // orbits need the whole turn
     int rows, cols;
-    patch_bounds(grid, reach, 16, 16, 16, rows, cols);
-    nq = patch_fits<1>(rows, cols) ? 1 : 0;
+    const int tx = plan.stack == 1 ? 16 : 8;
+    patch_bounds(grid, reach, tx, 256 / (tx * plan.stack), plan.zc * plan.stack, rows, cols);
+    plan = {patch_fits<1>(rows, cols, 1) ? 1 : 0, 1, plan.zc, plan.stack};
   }
+  const int nq = plan.orbit, groups = plan.groups, stack = plan.stack;
+  zc = zc == 16 ? std::min(32, plan.zc) : std::min(zc, plan.zc);  // (the largest tuned chunk stands for 32 too)
   if (nq == 0) {
-    // 8 voxels a lane, and waves per block until about 4 per SIMD are in flight
-    const long ncol = (long)ncx * grid.ny;
-    const int zd = 8;
-    const long cb = (ncol + 63) / 64, blocks = cb * ((grid.nz + zd - 1) / zd);
+    // 8 voxels a lane (16 spill registers in the bp3d20 preset), and waves per block
+    // until about 4 per SIMD are in flight
+    constexpr int zd = 8;
+    const long ncol = (long)ncx * grid.ny, cb = (ncol + 63) / 64;
+    const int most = std::min(16, std::max(1, nviews_chunk / 2));
+    const long blocks = cb * ((grid.nz + zd - 1) / zd);
     int waves = 1;
-    while (waves < 16 && blocks * waves < 4096 && 2 * waves < nviews_chunk) waves *= 2;
+    while (2 * waves <= most && blocks * waves < 4096) waves *= 2;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-#define MONTE_BP(ZEROS)                                                                                       \
-  hipLaunchKernelGGL((backproject_direct_kernel<8, ZEROS>), dim3((unsigned)blocks), dim3(64 * waves),          \
+#define MONTE_BP(ZEROS)                                                                                        \
+  hipLaunchKernelGGL((backproject_direct_kernel<zd, ZEROS>), dim3((unsigned)blocks), dim3(64 * waves),         \
                      sizeof(float) * waves * zd * 64, s, filt_pad, views, view0, nviews_chunk, grid, vol,      \
                      accumulate, (int)cb)
     if (reach.zeros) MONTE_BP(true); else MONTE_BP(false);
 #undef MONTE_BP
     return hipGetLastError();
   }
-  int tile_x = std::min(32, std::max(8, (int)t.bp_tile_x));  // whole 8 x 8 sub-tiles, one per wave
-  auto fits = [&](int rows, int cols) {
-    return nq == 4 ? patch_fits<4>(rows, cols) : (nq == 2 ? patch_fits<2>(rows, cols) : patch_fits<1>(rows, cols));
-  };
   const int nx = nq == 4 ? (grid.nx + 1) / 2 : ncx, ny = nq > 1 ? (grid.ny + 1) / 2 : grid.ny;
+  // whole 8 x 8 sub-tiles, one per wave
+  int tile_x = stack == 1 ? std::min(32, std::max(8, (int)t.bp_tile_x)) : 8;
   auto blocks_of = [&](int tx, int z) {
-    return (long)((nx + tx - 1) / tx) * ((ny + 256 / tx - 1) / (256 / tx)) * ((grid.nz + z - 1) / z);
+    const int ty = 256 / (tx * stack);
+    return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((grid.nz + z * stack - 1) / (z * stack));
   };
   int rows, cols;
-  patch_bounds(grid, reach, tile_x, 256 / tile_x, zc, rows, cols);
-  if (!fits(rows, cols)) {  // the tuned shape does not fit: the default does
-    tile_x = 16;
-    zc = 16;
-    patch_bounds(grid, reach, 16, 16, 16, rows, cols);
+  patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
+  if (!patch_fits(nq, rows, cols, groups)) {  // the tuned shape does not fit: the default does
+    tile_x = stack == 1 ? 16 : 8;
+    zc = plan.zc;
+    patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
   }
-  if (nq == 1 && zc == 16 && reach.zeros) {
-    // two groups of 16 share a column's set-up, where their patch fits and they fill the chip
-    int r2, c2;
-    patch_bounds(grid, reach, tile_x, 256 / tile_x, 32, r2, c2);
-    if (fits(r2, c2) && blocks_of(tile_x, 32) >= 768) {
-      zc = 32;
-      rows = r2;
-    }
-  }
-  const int tiles_x = (nx + tile_x - 1) / tile_x, tiles_y = (ny + 256 / tile_x - 1) / (256 / tile_x);
+  const int tiles_x = (nx + tile_x - 1) / tile_x, tile_y = 256 / (tile_x * stack), tiles_y = (ny + tile_y - 1) / tile_y;
   const long nblocks = blocks_of(tile_x, zc);
   if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+  // the groups' patches, which the sums of a group go through at the end
+  auto lds_of = [&](int row_words, int sums) {
+    const size_t patch = (size_t)2 * rows * row_words * groups;
+    return sizeof(float) * (groups > 1 ? std::max(patch, (size_t)sums * 256) : patch);
+  };
 #define MONTE_BP(ZC, NQ, ZEROS)                                                                                \
-  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256),                         \
-                     2 * sizeof(float) * rows * PatchLayout<NQ>::kRS, s, filt_pad, views, view0, nviews_chunk,  \
-                     grid, vol, accumulate, tile_x, tiles_x, tiles_y, rows, reach.turn)
+  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256 * groups),                       \
+                     lds_of(PatchLayout<NQ>::kRS, NQ * ZC), s, filt_pad, views, view0, nviews_chunk,          \
+                     grid, vol, accumulate, tile_x, tiles_x, tiles_y, rows, reach.turn, stack)
 #define MONTE_BP_Z(NQ, ZEROS)                                                                                    \
   switch (zc) {                                                                                                \
     case 4: MONTE_BP(4, NQ, ZEROS); break;                                                                            \

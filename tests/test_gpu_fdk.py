@@ -174,8 +174,8 @@ def test_quarter_turn_equivariance(ctx):
 
 # Which kernel backprojects depends on the scan: orbits of four or two columns
 # (a quarter or half turn maps scan and volume onto themselves), one column per
-# thread over 16 or 32 voxels, or taps straight from memory (few tiles, or voxels
-# too coarse for a patch in LDS).  Tall thin volumes reach the tiled kernels at
+# thread over 8 to 32 voxels, up to four groups of waves sharing a tile's views, or
+# taps straight from memory (few tiles, or voxels too coarse for a patch in LDS).  Tall thin volumes reach the tiled kernels at
 # small sizes; odd sides have a middle row and a centre column that orbits share.
 _BP_KINDS = {
     "quarter_even": dict(nx=66, ny=66, nz=910, n_views=8),
@@ -187,6 +187,15 @@ _BP_KINDS = {
     "one_16": dict(nx=51, ny=66, nz=420, n_views=5),
     "one_32": dict(nx=51, ny=66, nz=1301, n_views=5),
     "one_offset": dict(nx=64, ny=64, nz=560, n_views=8, ox=0.03, oy=-0.02),
+    "quarter_groups": dict(nx=65, ny=65, nz=130, n_views=16),
+    "half_groups": dict(nx=51, ny=67, nz=300, n_views=18),
+    "one_two_groups": dict(nx=100, ny=90, nz=110, n_views=9),
+    "one_four_groups": dict(nx=100, ny=90, nz=64, n_views=71),
+    "one_steep": dict(nx=100, ny=90, nz=64, n_views=21, nv=300, dv=0.021),
+    "half_steep": dict(nx=100, ny=90, nz=64, n_views=22, nv=300, dv=0.022),
+    "one_stacked": dict(nx=100, ny=72, nz=90, n_views=21, nu=400, du=0.02),
+    "half_stacked": dict(nx=100, ny=72, nz=93, n_views=22, nu=400, du=0.02),
+    "quarter_stacked": dict(nx=101, ny=101, nz=131, n_views=24, nu=300, du=0.03),
     "direct_few": dict(nx=33, ny=31, nz=45, n_views=9),
     "direct_coarse": dict(nx=130, ny=131, nz=140, n_views=3, vx=0.045, vy=0.045, vz=0.045, du=0.012, nu=500),
 }
