@@ -439,6 +439,26 @@ int mc_slots(int ray_slot) { return ray_slot >= 0 ? kMcSlots : kMcSlotsNoAlloc; 
 // Whether a launch with this ray slot forms first-flight label sets.
 bool wants_sets(const monte_ctx* c, int ray_slot) { return ray_slot >= 0 && c->tuning.mc_ray_brick > 0; }
 
+// The part of a job's set-up descriptor that forms its flight box; adds the box's
+// blocks to `blocks`.
+void box_prep(const HostJob& h, const uint8_t* labels, uint32_t solid, McPrep& Q, uint32_t& blocks) {
+  const McJob& J = h.d;
+  Q.labels = labels;
+  Q.nx = J.nx; Q.ny = J.ny; Q.nz = J.nz;
+  Q.solid = solid;
+  for (int a = 0; a < 3; ++a) {
+    Q.box[a] = INT_MAX;
+    Q.box[3 + a] = -1;
+    Q.vox[a] = h.vox[a];
+  }
+  Q.ray = h.ray;
+  // a block takes 4 chunks of 16 bytes a thread, up to 2048 blocks
+  const uint64_t voxels = (uint64_t)J.nx * J.ny * J.nz;
+  Q.box_blocks = (uint32_t)std::min<uint64_t>(2048, voxels / (16 * 256 * 4) + 1);
+  Q.prep_begin = blocks;
+  blocks += Q.box_blocks;
+}
+
 // Lays out the jobs in `base` (at least mc_layout(hj, wants_sets(...)).total
 // bytes; the context's MC workspace when null), queue and counters set,
 // uploads everything in one copy, and launches what forms each job's flight box
@@ -463,20 +483,12 @@ int prepare_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per
     HostJob& h = hj[i];
     const McJob& J = h.d;
     McPrep& Q = preps[i];
-    Q.labels = J.labels;
-    Q.nx = J.nx; Q.ny = J.ny; Q.nz = J.nz;
+    uint32_t solid = 0;
     for (int l = 0; l < kMaxLabels; ++l)
       for (int e = 0; e < kRows; ++e)
-        if (h.tables.m[l][e].x > 0.f) { Q.solid |= 1u << l; break; }
-    for (int a = 0; a < 3; ++a) {
-      Q.box[a] = INT_MAX;
-      Q.box[3 + a] = -1;
-      Q.vox[a] = h.vox[a];
-    }
-    // a block of the box takes 4 chunks of 16 bytes a thread, up to 2048 blocks
-    const uint64_t voxels = (uint64_t)J.nx * J.ny * J.nz;
-    Q.box_blocks = (uint32_t)std::min<uint64_t>(2048, voxels / (16 * 256 * 4) + 1);
-    Q.prep_begin = (uint32_t)prep_blocks;
+        if (h.tables.m[l][e].x > 0.f) { solid |= 1u << l; break; }
+    uint32_t first = (uint32_t)prep_blocks;
+    box_prep(h, J.labels, solid, Q, first);
     prep_blocks += Q.box_blocks;
     Q.brick = brick;
     Q.ray_begin = (uint32_t)ray_blocks;
@@ -1110,14 +1122,23 @@ int monte_primary_exact(monte_ctx* c, const monte_geom* g, const monte_phantom* 
   const size_t np = proj_elems(*g);
   float* dout = (float*)st.out(kSlotStageB, lineint, np * sizeof(float), false);
   if (st.code) return st.code;
-  // tables, FP64 view table and spectrum weights in the MC slot
-  size_t off = 0;
-  const size_t tab_off = off; off = align_up(off + sizeof(McTables), 256);
-  const size_t cs_off = off; off = align_up(off + sizeof(double) * 2 * g->n_views, 256);
-  const size_t w_off = off; off = align_up(off + sizeof(float) * kRows, 256);
-  char* base = (char*)workspace(c, kSlotMc, off);
-  if (!base) return fail(c, MONTE_ERR_NOMEM, "primary descriptor allocation failed");
-  std::vector<float> w(kRows, 0.f);
+  // per spectral bin its weight and the attenuation of the labels up to the last
+  // that attenuates (weights and attenuations in FP32, as the transport holds them)
+  uint32_t solid = 0;
+  int n_labels = 0;
+  for (int l = 0; l < kMaxLabels; ++l)
+    for (int e = 0; e < kRows; ++e)
+      if (hj.tables.m[l][e].x > 0.f) {
+        solid |= 1u << l;
+        n_labels = l + 1;
+        break;
+      }
+  std::vector<double> bins;
+  double weight = 0.0;
+  auto add_bin = [&](int row, double w) {
+    bins.push_back(w);
+    for (int l = 0; l < n_labels; ++l) bins.push_back((double)hj.tables.m[l][row].x);
+  };
   if (spectrum) {
     double tot = 0;
     for (int e = 1; e < kRows; ++e) {
@@ -1125,8 +1146,17 @@ int monte_primary_exact(monte_ctx* c, const monte_geom* g, const monte_phantom* 
       tot += spectrum[e];
     }
     if (!(tot > 0)) return fail(c, MONTE_ERR_INVALID, "empty spectrum");
-    for (int e = 1; e < kRows; ++e) w[e] = (float)(spectrum[e] / tot);
+    for (int e = 1; e < kRows; ++e) {
+      const double w = (double)(float)(spectrum[e] / tot);
+      if (w <= 0.0) continue;
+      add_bin(e, w);
+      weight += w;
+    }
+  } else {
+    const int row = (int)((float)cfg.e_kev + 0.5f);
+    add_bin(std::min(std::max(row, 1), kRows - 1), 1.0);
   }
+  const int n_bins = (int)(bins.size() / (size_t)(n_labels + 1));
   std::vector<double> cs(2 * g->n_views);
   for (int k = 0; k < g->n_views; ++k) {
     const double b = g->preset == MONTE_PRESET_BP3D20 ? 3.14159265358979323846 * (k * g->step_deg) / 180.0
@@ -1151,12 +1181,26 @@ int monte_primary_exact(monte_ctx* c, const monte_geom* g, const monte_phantom* 
     P.b1[a] = org[a] + 0.5 * n[a] * vox[a];
   }
   P.nu = g->nu; P.nv = g->nv; P.n_views = g->n_views;
-  MONTE_HIP(c, hipMemcpyAsync(base + tab_off, &hj.tables, sizeof(McTables), hipMemcpyHostToDevice, c->stream));
-  MONTE_HIP(c, hipMemcpyAsync(base + cs_off, cs.data(), sizeof(double) * cs.size(), hipMemcpyHostToDevice, c->stream));
-  MONTE_HIP(c, hipMemcpyAsync(base + w_off, w.data(), sizeof(float) * kRows, hipMemcpyHostToDevice, c->stream));
-  MONTE_HIP(c, launch_primary_exact(P, (const double*)(base + cs_off), dph.labels, (const McTables*)(base + tab_off),
-                                    (float)cfg.e_kev, (const float*)(base + w_off), spectrum ? 1 : 0, dout,
-                                    c->stream));
+  // the descriptor of the phantom's box, the FP64 view table and the bins, in the MC slot by one copy
+  const size_t cs_off = 256, bin_off = align_up(cs_off + sizeof(double) * cs.size(), 256);
+  const size_t bytes = align_up(bin_off + sizeof(double) * bins.size(), 256);
+  char* base = (char*)workspace(c, kSlotMc, bytes);
+  if (!base) return fail(c, MONTE_ERR_NOMEM, "primary descriptor allocation failed");
+  std::vector<char> host(bytes, 0);
+  McPrep& Q = *(McPrep*)host.data();
+  uint32_t blocks = 0;
+  box_prep(hj, dph.labels, solid, Q, blocks);
+  std::memcpy(host.data() + cs_off, cs.data(), sizeof(double) * cs.size());
+  std::memcpy(host.data() + bin_off, bins.data(), sizeof(double) * bins.size());
+  MONTE_HIP(c, hipMemcpyAsync(base, host.data(), bytes, hipMemcpyHostToDevice, c->stream));
+  hipError_t le = launch_mc_prep((McPrep*)base, 1, blocks, c->stream);
+  if (le == hipSuccess)
+    le = launch_primary_exact(P, (const McPrep*)base, (const double*)(base + cs_off), dph.labels,
+                              (const double*)(base + bin_off), n_bins, n_labels, weight, dout, c->stream);
+  if (le != hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);  // the upload is done with its host copy
+    return fail(c, MONTE_ERR_HIP, std::string("primary launch: ") + hipGetErrorString(le));
+  }
   MONTE_HIP(c, hipStreamSynchronize(c->stream));  // host tables above must outlive the copies
   return st.back(lineint, dout, np * sizeof(float));
 }

@@ -375,8 +375,11 @@ hipError_t launch_ray_sets(const McPrep* preps, McJob* jobs, int n_jobs, uint32_
                            hipStream_t s);
 hipError_t launch_mc_boxes(const McPrep* preps, McJob* jobs, int n_jobs, hipStream_t s);
 constexpr int kRayBlock = 256;  // pixels per block of the label sets
-hipError_t launch_primary_exact(const PrimaryGeom& P, const double* cs64, const uint8_t* labels,
-                                const McTables* tables, float e_kev, const float* spec_w, int use_spec, float* out,
+// prep: the phantom's flight box (launch_mc_prep without bricks).  bins:
+// [n_bins][1 + n_labels] weight and attenuation of labels 0 .. n_labels - 1; weight
+// is the sum of the weights, or 0 for one mono-energetic bin.
+hipError_t launch_primary_exact(const PrimaryGeom& P, const McPrep* prep, const double* cs64, const uint8_t* labels,
+                                const double* bins, int n_bins, int n_labels, double weight, float* out,
                                 hipStream_t s);
 // counts2 (nullable) is added to counts before the conversion
 hipError_t launch_counts_to_lineint(const double* counts, const double* counts2, float* out, int n_views, int nu,

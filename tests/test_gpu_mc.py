@@ -346,3 +346,61 @@ def test_woodcock_majorant_invariance(ctx):
         assert abs(tot) < 5.0
     for k in ("tallied_primary", "tallied_scatter", "photo", "compton", "coherent"):
         assert abs(sta[k] - stb[k]) < 6 * np.sqrt(max(sta[k] + stb[k], 1)), k
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 4001), (2, 3, 3892), (1, 1, 1), (17, 5, 40)])
+@pytest.mark.parametrize("spectrum", [False, True])
+def test_primary_exact_grids(ctx, oracle, shape, spectrum):
+    """Grids with more voxel planes than fit in LDS (a long one), just as many, one voxel, and an
+    ordinary odd one; attenuating voxels in a corner, so rays enter their box past the grid's edge;
+    labels above the last that attenuates.  Against the FP64 Siddon oracle at 1e-5."""
+    from monte_amd import geometry as G
+    from monte_amd import tables
+    from monte_amd.mc import primary_exact
+    from monte_amd.phantoms import MATERIALS, LabelPhantom
+
+    nz, ny, nx = shape
+    lab = np.zeros(shape, np.uint8)
+    lab[: (nz + 1) // 2, : (ny + 1) // 2, nx // 3:] = 1
+    lab[nz // 4: nz // 2 + 1, :, nx // 2: nx // 2 + max(1, nx // 5)] = 5
+    lab[-1:, :, : nx // 4] = 3  # vacuum
+    ph = LabelPhantom(lab, (8.0 / nx, 4.0 / ny, 5.0 / nz), list(MATERIALS) + [(-1, 0.0), (0, 0.0), (1, 0.6)])
+    geom = G.small(n_views=2).replace(nu=21, nv=18, du=0.9, dv=0.8, angle0=0.4)
+    w = tables.kramers_spectrum(120.0, 2.5) if spectrum else None
+    got = primary_exact(ph, geom, e_kev=60.0, spectrum=w, ctx=ctx).cpu().numpy()
+    ref = oracle.primary_lineint(oracle_geom(oracle, geom), oracle_phantom(oracle, ph), _tables(oracle), 60.0,
+                                 **({"spectrum": w} if spectrum else {}))
+    assert np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("views,nu,nv", [(1, 1, 1), (13, 5, 7), (12, 6, 5), (25, 31, 3), (37, 16, 24)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("flat_views", [None, 1, "all"])
+def test_lineint_layouts(ctx, views, nu, nv, offset, flat_views):
+    """Odd and even pixel counts, buffers 8 and 16 bytes aligned, and view counts around the group
+    a thread takes, against numpy in FP64; counts of 0 and above the top are clamped, dead pixels 0."""
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd.mc import counts_to_lineint, counts_to_lineint_flat, photons_per_pixel
+
+    geom = G.small(n_views=views).replace(nu=nu, nv=nv)
+    photons = 40 * nu * nv + nu * nv // 2
+    rng = np.random.default_rng(views + nu)
+    n = views * nu * nv
+    buf = torch.zeros(n + 2, dtype=torch.float64, device="cuda")
+    c = rng.poisson(30.0, (views, nu, nv)).astype(np.float64)
+    c.reshape(-1)[:: 7] = 0.0
+    dev = buf[offset:offset + n].view(views, nu, nv)
+    dev.copy_(torch.from_numpy(c))
+    if flat_views is None:
+        top = np.broadcast_to(photons_per_pixel(geom, photons), c.shape)
+        got = counts_to_lineint(dev, geom, photons, ctx)
+    else:
+        top = rng.poisson(35.0, (views if flat_views == "all" else 1, nu, nv)).astype(np.float64)
+        top[rng.random(top.shape) < 0.1] = 0.0
+        got = counts_to_lineint_flat(dev, geom, torch.from_numpy(top).cuda(), ctx)
+        top = np.broadcast_to(top, c.shape)
+    safe = np.maximum(top, 1e-300)
+    ref = np.where(top > 0, np.log(safe) - np.log(np.maximum(np.minimum(c, safe), 1.0)), 0.0)
+    assert np.abs(got.cpu().numpy() - ref).max() <= 1e-6 * max(1.0, np.abs(ref).max())
