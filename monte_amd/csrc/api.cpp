@@ -109,16 +109,17 @@ int ensure_constants(monte_ctx* c, const monte_geom& g, const float** taps, cons
 // Build the projector's column lists once per geometry: a counting pass, the
 // prefix sums on the host, then a writing pass.
 int ensure_projector_plan(monte_ctx* c, const monte_geom& g, const BpView* views, const BpGrid& grid,
-                          const uint32_t** offs, const uint32_t** list) {
+                          int orbit, const uint32_t** offs, const uint32_t** list) {
   std::vector<double> key = geom_key(g);
   key.push_back((double)project_strips(grid));
+  key.push_back((double)orbit);
   const size_t ncell = (size_t)g.n_views * project_strips(grid);
   const size_t obytes = align_up((ncell + 1) * sizeof(uint32_t), 256);
   if (key != c->plan_key || !c->ws[kSlotPlan]) {
     c->plan_key.clear();
     uint32_t* d = (uint32_t*)workspace(c, kSlotPlan, obytes);
     if (!d) return fail(c, MONTE_ERR_NOMEM, "projector plan allocation failed");
-    MONTE_HIP(c, launch_project_plan(views, g.n_views, grid, d, nullptr, false, c->stream));
+    MONTE_HIP(c, launch_project_plan(views, g.n_views, grid, orbit, d, nullptr, false, c->stream));
     std::vector<uint32_t> h(ncell + 1);
     MONTE_HIP(c, hipMemcpyAsync(h.data(), d, ncell * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     MONTE_HIP(c, hipStreamSynchronize(c->stream));
@@ -133,8 +134,8 @@ int ensure_projector_plan(monte_ctx* c, const monte_geom& g, const BpView* views
     char* base = (char*)workspace(c, kSlotPlan, obytes + total * sizeof(uint32_t));
     if (!base) return fail(c, MONTE_ERR_NOMEM, "projector plan allocation failed");
     MONTE_HIP(c, hipMemcpyAsync(base, h.data(), h.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    MONTE_HIP(c, launch_project_plan(views, g.n_views, grid, (uint32_t*)base, (uint32_t*)(base + obytes), true,
-                                     c->stream));
+    MONTE_HIP(c, launch_project_plan(views, g.n_views, grid, orbit, (uint32_t*)base, (uint32_t*)(base + obytes),
+                                     true, c->stream));
     MONTE_HIP(c, hipStreamSynchronize(c->stream));
     c->plan_key = key;
     c->plan_list_off = obytes;
@@ -221,8 +222,10 @@ int run_project_padded(monte_ctx* c, const monte_geom& g, const float* vol, floa
   int rc = ensure_constants(c, g, &taps, &views);
   if (rc) return rc;
   const BpGrid grid = compute_bp_grid(g);
+  const BpReach reach = compute_bp_reach(g, grid);
+  const int by_rows = project_orbit(grid, reach, c->tuning);  // 0: by voxels
   const uint32_t *plan_offs, *plan_list;
-  if ((rc = ensure_projector_plan(c, g, views, grid, &plan_offs, &plan_list))) return rc;
+  if ((rc = ensure_projector_plan(c, g, views, grid, std::max(by_rows, 1), &plan_offs, &plan_list))) return rc;
   float* volT = (float*)workspace(c, kSlotVolT, vol_elems(g) * sizeof(float));
   if (!volT) return fail(c, MONTE_ERR_NOMEM, "transposed volume allocation failed");
   MONTE_HIP(c, launch_transpose_zx(vol, volT, g.nx, g.ny, g.nz, c->stream));
@@ -235,8 +238,12 @@ int run_project_padded(monte_ctx* c, const monte_geom& g, const float* vol, floa
     const int n = std::min(chunk, g.n_views - v0);
     int lds_r0, lds_rows;
     projector_rows(host_views, v0, n, grid, lds_r0, lds_rows);
-    MONTE_HIP(c, launch_project(volT, views, v0, n, grid, pad, lds_r0, lds_rows, plan_offs, plan_list, c->tuning,
-                                c->stream));
+    if (by_rows)
+      MONTE_HIP(c, launch_project_rows(volT, views, v0, n, grid, reach, by_rows, pad, lds_r0, lds_rows, plan_offs,
+                                       plan_list, c->stream));
+    else
+      MONTE_HIP(c, launch_project(volT, views, v0, n, grid, pad, lds_r0, lds_rows, plan_offs, plan_list, c->tuning,
+                                  c->stream));
   }
   if (g.preset == MONTE_PRESET_BP3D20)
     MONTE_HIP(c, launch_fold_pads(pad, g.n_views, g.nu, g.nv, grid.pitch, grid.rows, c->stream));
@@ -1515,7 +1522,8 @@ int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, c
   if ((rc = ensure_constants(c, *g, &taps, &views))) return rc;
   const BpGrid grid = compute_bp_grid(*g);
   const uint32_t *plan_offs, *plan_list;
-  if ((rc = ensure_projector_plan(c, *g, views, grid, &plan_offs, &plan_list))) return rc;
+  const int orbit = std::max(1, project_orbit(grid, compute_bp_reach(*g, grid), c->tuning));
+  if ((rc = ensure_projector_plan(c, *g, views, grid, orbit, &plan_offs, &plan_list))) return rc;
   if (!workspace(c, kSlotFwd, padded_elems(*g) * sizeof(float)) ||
       !workspace(c, kSlotAdj, padded_elems(*g) * sizeof(float)) ||
       !workspace(c, kSlotVolT, vol_elems(*g) * sizeof(float)))

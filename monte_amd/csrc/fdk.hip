@@ -1381,6 +1381,13 @@ __device__ inline float permute_f(int dst, float v) {
   return __int_as_float(__builtin_amdgcn_ds_permute(dst << 2, __float_as_int(v)));
 }
 
+// Whether column (x, y) of the first quadrant or half stands for its orbit: an odd
+// volume's middle row holds whole orbits of half a turn, and turned middle columns.
+__device__ inline bool orbit_first(int orbit, int x, int y, int nx, int ny) {
+  if (orbit == 1 || 2 * y + 1 != ny || 2 * x + 1 == nx) return true;
+  return orbit == 2 && 2 * x + 1 < nx;
+}
+
 // Walks the strip's slabs four at a time, 16 lanes per slab, and appends the
 // kept columns to the batch (each kept lane pushes its column to lane n + its
 // rank; the other lanes push to the lanes past the new end), until the batch
@@ -1391,7 +1398,7 @@ struct Enumerator {
   int rnd = 0;  // 16-column round within the group
 
   __device__ bool fill(ColumnBatch& cb, const BpView& c, const BpGrid& g, bool x_slabs, int n_slabs, int u_lo,
-                       int u_hi, int lane) {
+                       int u_hi, int lane, int orbit, int full_ny) {
     cb.n = 0;
     for (;;) {
       if (s0 >= n_slabs) return cb.n > 0;
@@ -1413,7 +1420,8 @@ struct Enumerator {
       const int x = min(xo, g.x1 - 1), y = min(yo, g.ny - 1);
       const double X = voxel_x(g, x), Y = voxel_y(g, y);
       const ColumnCore mine = column_core(c, X, Y, (float)X, (float)Y, g);
-      const bool keep = sl < n_slabs && off <= b && mine.ok && mine.iu >= u_lo && mine.iu <= u_hi;
+      const bool keep = sl < n_slabs && off <= b && mine.ok && mine.iu >= u_lo && mine.iu <= u_hi &&
+                        orbit_first(orbit, x, y, g.nx, full_ny);
       const uint64_t m = __ballot(keep);
       const int cnt = (int)__popcll(m);
       if (cb.n + cnt > 64) return true;  // full: this round is taken again by the next fill
@@ -1464,7 +1472,8 @@ struct StripSetup {
 // writes the list at list + offs[k * n_strips + st] (offsets by then).
 template <bool WRITE>
 __global__ __launch_bounds__(64) void project_plan_kernel(const BpView* __restrict__ views, int n_strips, BpGrid g,
-                                                          uint32_t* __restrict__ offs, uint32_t* __restrict__ list) {
+                                                          uint32_t* __restrict__ offs, uint32_t* __restrict__ list,
+                                                          int orbit, int full_ny) {
   const int k = blockIdx.x / n_strips;
   const int st = blockIdx.x - k * n_strips;
   const int lane = threadIdx.x;
@@ -1475,7 +1484,7 @@ __global__ __launch_bounds__(64) void project_plan_kernel(const BpView* __restri
   ColumnBatch cb;
   const uint32_t base = WRITE ? offs[blockIdx.x] : 0u;
   uint32_t n = 0;
-  while (en.fill(cb, c, g, ss.x_slabs, ss.n_slabs, ss.u_lo, ss.u_hi, lane)) {
+  while (en.fill(cb, c, g, ss.x_slabs, ss.n_slabs, ss.u_lo, ss.u_hi, lane, orbit, full_ny)) {
     if (WRITE && lane < cb.n) list[base + n + lane] = (uint32_t)cb.x | ((uint32_t)cb.y << 16);
     n += (uint32_t)cb.n;
   }
@@ -1688,17 +1697,272 @@ hipError_t launch_transpose_zx(const float* vol, float* volT, int nx, int ny, in
 
 int project_strips(const BpGrid& grid) { return (grid.pitch + kStripW - 1) / kStripW; }
 
-hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& grid, uint32_t* offs, uint32_t* list,
-                               bool write, hipStream_t s) {
+hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& grid, int orbit, uint32_t* offs,
+                               uint32_t* list, bool write, hipStream_t s) {
   const long nblocks = (long)project_strips(grid) * n_views;
   if (nblocks <= 0) return hipSuccess;
   if (nblocks > 0x7fffffffL || grid.nx > 65536 || grid.ny > 65536) return hipErrorInvalidValue;
+  BpGrid g = grid;  // the first quadrant or half
+  if (orbit == 4) g.x1 = (g.nx + 1) / 2;
+  if (orbit > 1) g.ny = (g.ny + 1) / 2;
   if (write)
     hipLaunchKernelGGL(project_plan_kernel<true>, dim3((unsigned)nblocks), dim3(64), 0, s, views,
-                       project_strips(grid), grid, offs, list);
+                       project_strips(grid), g, offs, list, orbit, grid.ny);
   else
     hipLaunchKernelGGL(project_plan_kernel<false>, dim3((unsigned)nblocks), dim3(64), 0, s, views,
-                       project_strips(grid), grid, offs, list);
+                       project_strips(grid), g, offs, list, orbit, grid.ny);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------ projector by rows
+// The matched projector as a gather over detector rows, without read-add-writes:
+// a wave owns one detector column (strip) of a view, its lanes the rows, and walks
+// the strip's voxel columns.  Row r takes the voxels whose v coordinate lies
+// within a row of it, with the bilinear tent max(0, 1 - |sv - r|): sv(z) = A + z D,
+// so they are the J consecutive voxels from z0 = floor((r - 1 - A) / D) + 1, J =
+// ceil(2 / D), at s0 = sv(z0) - r, s0 + D, ...  The sum is added to the lane's two
+// registers per row, for the column itself and for the one to its right.
+//   (r - 1 - A) / D is formed in 32.32 fixed point from the row's integer offset,
+// so z0 is its high word and s0 comes from the low one to 2^-22 rows.
+// A column's voxels come from memory straight into the wave's LDS, `depth` - 1
+// columns ahead, between zeros that the rows past its ends read.
+//   NQ > 1: as the backprojector, the NQ columns of an orbit share all of a row's
+// geometry; the wave forms the strip in all NQ views that are a part of a turn
+// apart, taking the lists of first columns of each in turn.
+// Per row and column: 12 / NQ VALU instructions of geometry, 2 J - 1 of sums and 2
+// multiply-adds, J reads of LDS.  The kernel this one replaces in these cases (below:
+// lanes own voxels, two read-add-writes of LDS per voxel) took 9.97 ms at 325^3 ->
+// 360 views of 512^2.
+constexpr int kRowPad = 4;  // zeros before and after a column in LDS (>= J)
+
+__device__ inline void wait_copies(int n) {  // until at most n copies to LDS are in flight
+#define MONTE_WAIT(N) asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory")
+  if (n >= 48) MONTE_WAIT(48);
+  else if (n >= 32) MONTE_WAIT(32);
+  else if (n >= 24) MONTE_WAIT(24);
+  else if (n >= 18) MONTE_WAIT(18);
+  else if (n >= 12) MONTE_WAIT(12);
+  else if (n >= 8) MONTE_WAIT(8);
+  else if (n >= 6) MONTE_WAIT(6);
+  else if (n >= 4) MONTE_WAIT(4);
+  else if (n >= 3) MONTE_WAIT(3);
+  else if (n >= 2) MONTE_WAIT(2);
+  else if (n >= 1) MONTE_WAIT(1);
+  else MONTE_WAIT(0);
+#undef MONTE_WAIT
+}
+
+template <int NQ, int J, int NR>
+__global__ __launch_bounds__(64) void project_rows_kernel(const float* __restrict__ volT,
+                                                          const BpView* __restrict__ views, int view0, int n_strips,
+                                                          int nviews, BpGrid g, float* __restrict__ filt, int row0,
+                                                          int row_end, int row_chunks, int depth,
+                                                          const uint32_t* __restrict__ offs,
+                                                          const uint32_t* __restrict__ list, int turn) {
+  extern __shared__ float cols[];  // [depth][NQ][kRowPad + nz + kRowPad]
+  // XCD x takes the views [x V / 8, (x + 1) V / 8) of the launch in groups of
+  // kProjViewGroup, strip by strip within a group (see project_kernel)
+  const int per_view = n_strips * row_chunks;
+  const int xcd = (int)(blockIdx.x % 8u), jx = (int)(blockIdx.x / 8u);
+  const int va = xcd * nviews / 8, vx = (xcd + 1) * nviews / 8 - va;
+  if (jx >= vx * per_view) return;  // (the whole one-wave block)
+  const int grp = jx / (kProjViewGroup * per_view), rem = jx - grp * kProjViewGroup * per_view;
+  const int gsize = min(kProjViewGroup, vx - grp * kProjViewGroup);
+  const int sr = rem / gsize, st = sr / row_chunks;
+  const int k = view0 + va + grp * kProjViewGroup + (rem - sr * gsize);
+  const int u = st * kStripW - kPadLo;  // the strip's detector column
+  if (u >= g.nu) return;
+  const int lane = threadIdx.x;
+  const int rbase = row0 + (sr - st * row_chunks) * 64 * NR;  // detector row of lane 0
+  const int part = g.n_views / NQ;
+  const int slot_words = kRowPad + g.nz + kRowPad;
+  for (int i = lane; i < depth * NQ * slot_words; i += 64) cols[i] = 0.f;
+  __builtin_amdgcn_wave_barrier();
+  const int chunks = (g.nz + 63) / 64, per_column = NQ * chunks;
+
+  float accl[NQ][NR], accr[NQ][NR];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int p = 0; p < NR; ++p) accl[q][p] = accr[q][p] = 0.f;
+
+  for (int a = 0; a < NQ; ++a) {
+    const int ka = k + a * part;
+    const BpView& c = views[ka];
+    const size_t cell = (size_t)ka * n_strips + st;
+    const uint32_t beg = offs[cell], end = offs[cell + 1];
+    for (uint32_t b0 = beg; b0 < end; b0 += 64) {
+      const int ncols = (int)min(64u, end - b0);
+      // lane i prepares the i-th column: its weights and its line in fixed point
+      int cx = 0, cy = 0;
+      float wl = 0.f, wr = 0.f, d = 0.f;
+      long long q0 = 0;
+      uint32_t inv = 0;
+      int first = 0, last = -1;  // rows (from rbase) it reaches
+      if (lane < ncols) {
+        const uint32_t e = list[b0 + lane];
+        cx = (int)(e & 0xffffu);
+        cy = (int)(e >> 16);
+        const double X = voxel_x(g, cx), Y = voxel_y(g, cy);
+        const ColumnCore mine = column_core<true>(c, X, Y, (float)X, (float)Y, g);
+        // the centre of an odd volume is an orbit of one, taken NQ times
+        const float w = NQ > 1 && 2 * cx + 1 == g.nx && 2 * cy + 1 == g.ny ? mine.w / NQ : mine.w;
+        wr = w * mine.fu;
+        wl = w - wr;
+        const double A = fma(mine.kv, g.gz0, c.sv0) - (double)rbase, D = mine.kv * g.gsz, iD = recip64(D);
+        d = (float)D;
+        const double q = fmin(fmax((-1.0 - A) * iD, -1.0e8), 1.0e8);
+        q0 = __double2ll_rn(q * 4294967296.0);
+        inv = (uint32_t)__double2ll_rn(fmin(iD * 2147483648.0, 4294967295.0));
+        first = (int)floor(fmin(fmax(A - 1.0, -1.0e6), 1.0e6));
+        last = (int)ceil(fmin(fmax(fma((double)(g.nz - 1), D, A) + 1.0, -1.0e6), 1.0e6));
+      }
+      auto fetch = [&](int i, int slot) {
+        const int x = bcast_i(cx, i), y = bcast_i(cy, i);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's last reads are done
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const int m = NQ == 2 ? 2 * q : (turn > 0 ? q : (4 - q) & 3);  // quarter turns (x, y) -> (n - 1 - y, x)
+          const int xq = m == 0 ? x : (m == 1 ? g.nx - 1 - y : (m == 2 ? g.nx - 1 - x : y));
+          const int yq = m == 0 ? y : (m == 1 ? x : (m == 2 ? g.ny - 1 - y : g.nx - 1 - x));
+          const char* col = (const char*)(volT + ((size_t)yq * g.nx + xq) * g.nz);
+          float* dst = cols + (slot * NQ + q) * slot_words + kRowPad;
+          for (int ch = 0; ch < chunks; ++ch)
+            if (ch * 64 + lane < g.nz) copy_to_lds(col + ch * 256, (uint32_t)lane * 4u, dst + ch * 64);
+        }
+      };
+      const int ahead = min(depth - 1, ncols);
+      for (int i = 0; i < ahead; ++i) fetch(i, i);
+      int slot = 0, fslot = ahead;
+      for (int i = 0; i < ncols; ++i) {
+        if (i + ahead < ncols) fetch(i + ahead, fslot);
+        if (++fslot == depth) fslot = 0;
+        wait_copies(min(ahead, ncols - 1 - i) * per_column);
+        const float wli = bcast_f(wl, i), wri = bcast_f(wr, i), di = bcast_f(d, i);
+        const long long q0i = bcast_ll(q0, i);
+        const uint32_t invi = (uint32_t)bcast_i((int)inv, i);
+        const int fi = bcast_i(first, i), la = bcast_i(last, i);
+        const float dm = di * -2.3283064365386963e-10f, d1 = di - 1.0f;  // 2^-32
+        const float* col = cols + slot * NQ * slot_words + kRowPad;
+#pragma unroll
+        for (int p = 0; p < NR; ++p) {
+          if (fi > 64 * p + 63 || la < 64 * p) continue;  // (uniform)
+          const uint64_t q = (uint64_t)invi * (uint32_t)(2 * lane + 128 * p) + (uint64_t)q0i;
+          const int z = clamp_i((int)(uint32_t)(q >> 32) + 1, -kRowPad, g.nz);
+          const float s0 = fmaf((float)(uint32_t)q, dm, d1);
+          float t[J];
+#pragma unroll
+          for (int j = 0; j < J; ++j) t[j] = fmaxf(1.0f - fabsf(fmaf((float)j, di, s0)), 0.f);
+#pragma unroll
+          for (int qq = 0; qq < NQ; ++qq) {
+            const float* v = col + qq * slot_words + z;
+            float sum = t[0] * v[0];
+#pragma unroll
+            for (int j = 1; j < J; ++j) sum = fmaf(t[j], v[j], sum);
+            accl[qq][p] = fmaf(wli, sum, accl[qq][p]);
+            accr[qq][p] = fmaf(wri, sum, accr[qq][p]);
+          }
+        }
+        if (++slot == depth) slot = 0;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch's copies
+    }
+    // column q of the next list belongs to the view of this list's column q + 1
+    if (NQ > 1) {
+#pragma unroll
+      for (int p = 0; p < NR; ++p) {
+        const float l0 = accl[0][p], r0 = accr[0][p];
+#pragma unroll
+        for (int q = 0; q + 1 < NQ; ++q) {
+          accl[q][p] = accl[q + 1][p];
+          accr[q][p] = accr[q + 1][p];
+        }
+        accl[NQ - 1][p] = l0;
+        accr[NQ - 1][p] = r0;
+      }
+    }
+  }
+  // Two strips meet in a detector column: two addends onto zero, the same in
+  // either order.  Guard cells are not used (standard preset).
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    float* out = filt + (size_t)(k + q * part) * g.rows * g.pitch;
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      const int r = rbase + 64 * p + lane;
+      if (r < 0 || r >= min(g.nv, row_end)) continue;
+      float* o = out + (size_t)(r + kPadLo) * g.pitch + u + kPadLo;
+      if (u >= 0 && accl[q][p] != 0.f) unsafeAtomicAdd(o, accl[q][p]);
+      if (u + 1 < g.nu && accr[q][p] != 0.f) unsafeAtomicAdd(o + 1, accr[q][p]);
+    }
+  }
+}
+
+// The row kernel's orbit (4, 2 or 1 views that a wave forms together), or 0 for the
+// voxel kernel above.  The rule takes the standard preset's zero guard cells and the
+// automatic tuning, and these sizes (adjoint with its filter, row kernel against
+// voxel kernel, ms):
+//  - between 0.8 and 2 rows a voxel.  Below, a row takes more than three voxels (0.64
+//    to 1.12x: 0.76 : 0.86 at 65^3, 0.89 : 0.96 at 193^3, 0.77 rows a voxel), above most
+//    rows of a column see one voxel (0.37 : 0.46 at 97^3, 1.81 rows a voxel).
+//  - a column within 384 rows: more take a second wave that reads all columns again
+//    (1.69 : 2.57 at 225^3, 448 rows).
+//  - a volume of up to 48 MB.  Larger ones leave no columns for the next view in the
+//    L2s: a launch reads the volume once per view, 5.2 TB/s (137 MB x 360 views at
+//    325^3: 11.5 against the voxel kernel's 9.97, which walks in z and keeps columns).
+// Within them: 0.050 : 0.071 at 49^3 (36 views of 64^2), 0.117 : 0.172 at 65^3 (90 of
+// 96^2), 0.26 : 0.34 at 97^3 (90 of 160^2), 0.77 : 1.00 at 129^3 (180 of 192^2), 1.2 :
+// 1.54 at 161^3 (180 of 256^2), 2.75 : 3.00 at 225^3 (180 of 384^2).
+//   Orbits save geometry and take waves: of 4 from 10000 waves (2.75 : 3.10 with 2 at
+// 17000, 0.72 : 0.68 at 7200), of 2 from 3000 (0.117 : 0.131 with 1 at 4300, 0.054 : 0.050
+// at 1150).
+int project_orbit(const BpGrid& g, const BpReach& r, const monte_tuning& t) {
+  const double lo = r.svk * std::fabs(g.gsz) / (r.sod + r.rad), hi = r.svk * std::fabs(g.gsz) / (r.sod - r.rad);
+  if (t.pj_zchunk != 0 || !r.zeros || g.gsz <= 0 || !(lo > 0.8) || !(hi < 2.0) || !(hi * g.nz <= 384.0)) return 0;
+  if ((double)g.nx * g.ny * g.nz > 12e6) return 0;
+  if (t.bp_view_chunk > 0 && t.bp_view_chunk < g.n_views) return 1;  // orbits need the whole turn
+  const long waves = (long)g.n_views * project_strips(g);
+  return r.turn != 0 && waves >= 40000 ? 4 : (r.half && waves >= 6000 ? 2 : 1);
+}
+
+hipError_t launch_project_rows(const float* volT, const BpView* views, int view0, int nviews_chunk, const BpGrid& grid,
+                               const BpReach& reach, int orbit, float* filt_pad, int lds_r0, int lds_rows,
+                               const uint32_t* plan_offs, const uint32_t* plan_list, hipStream_t s) {
+  if (nviews_chunk <= 0) return hipSuccess;
+  if (orbit != 1 && nviews_chunk != grid.n_views) return hipErrorInvalidValue;
+  // detector rows that the window of padded rows holds
+  const int row0 = std::max(lds_r0 - kPadLo, 0), row_end = std::min(lds_r0 - kPadLo + lds_rows, grid.nv);
+  if (row_end <= row0) return hipSuccess;
+  const int base_views = nviews_chunk / orbit, n_strips = project_strips(grid);
+  // a block fetches and sets up its columns once for all its rows: few chunks
+  const int rows64 = (row_end - row0 + 63) / 64;
+  const int chunks = (rows64 + 5) / 6, nr = (rows64 + chunks - 1) / chunks;
+  const double lo = reach.svk * std::fabs(grid.gsz) / (reach.sod + reach.rad);
+  if (lo < 2.0 / 3.0) return hipErrorInvalidValue;  // (project_orbit)
+  const int J = lo >= 1.0 ? 2 : 3;
+  const size_t slot = sizeof(float) * orbit * (2 * kRowPad + grid.nz);
+  const int depth = (int)std::min<size_t>(6, std::max<size_t>(2, 12 * 1024 / slot));
+  const long nblocks = (long)n_strips * chunks * 8 * ((base_views + 7) / 8);
+  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+#define MONTE_PR(NQ, JJ, RR)                                                                                   \
+  hipLaunchKernelGGL((project_rows_kernel<NQ, JJ, RR>), dim3((unsigned)nblocks), dim3(64), slot * depth, s,    \
+                     volT, views, view0, n_strips, base_views, grid, filt_pad, row0, row_end, chunks, depth,   \
+                     plan_offs, plan_list, reach.turn)
+#define MONTE_PR_R(NQ, JJ)                                                                                     \
+  switch (nr) {                                                                                                \
+    case 1: MONTE_PR(NQ, JJ, 1); break;                                                                        \
+    case 2: MONTE_PR(NQ, JJ, 2); break;                                                                        \
+    case 3: MONTE_PR(NQ, JJ, 3); break;                                                                        \
+    case 4: MONTE_PR(NQ, JJ, 4); break;                                                                        \
+    case 5: MONTE_PR(NQ, JJ, 5); break;                                                                        \
+    default: MONTE_PR(NQ, JJ, 6); break;                                                                       \
+  }
+#define MONTE_PR_J(NQ)                                                                                         \
+  if (J == 2) { MONTE_PR_R(NQ, 2) } else { MONTE_PR_R(NQ, 3) }
+  if (orbit == 4) { MONTE_PR_J(4) } else if (orbit == 2) { MONTE_PR_J(2) } else { MONTE_PR_J(1) }
+#undef MONTE_PR_J
+#undef MONTE_PR_R
+#undef MONTE_PR
   return hipGetLastError();
 }
 

@@ -322,9 +322,15 @@ int project_strips(const BpGrid& grid);
 // Column lists of the projector for views [0, n_views): with write false,
 // offs[k * project_strips + st] receives each list's length; with write true,
 // offs holds the exclusive prefix sums (plus the total at the end) and the
-// lists are written to list.
-hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& grid, uint32_t* offs, uint32_t* list,
-                               bool write, hipStream_t s);
+// lists are written to list.  orbit 2, 4: of the first columns of orbits only.
+hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& grid, int orbit, uint32_t* offs,
+                               uint32_t* list, bool write, hipStream_t s);
+// The projector by rows, where project_orbit is not 0 (its lists made for that
+// orbit); launch_project elsewhere.
+int project_orbit(const BpGrid& grid, const BpReach& reach, const monte_tuning& t);
+hipError_t launch_project_rows(const float* volT, const BpView* views, int view0, int nviews_chunk, const BpGrid& grid,
+                               const BpReach& reach, int orbit, float* filt_pad, int lds_r0, int lds_rows,
+                               const uint32_t* plan_offs, const uint32_t* plan_list, hipStream_t s);
 hipError_t launch_project(const float* volT, const BpView* views, int view0, int nviews_chunk, const BpGrid& grid,
                           float* filt_pad, int lds_r0, int lds_rows, const uint32_t* plan_offs,
                           const uint32_t* plan_list, const monte_tuning& t, hipStream_t s);
