@@ -1900,16 +1900,18 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
 
 // The row kernel's orbit (4, 2 or 1 views that a wave forms together), or 0 for the
 // voxel kernel above.  The rule takes the standard preset's zero guard cells and the
-// automatic tuning, and these sizes (adjoint with its filter, row kernel against
-// voxel kernel, ms):
-//  - between 0.8 and 2 rows a voxel.  Below, a row takes more than three voxels (0.64
-//    to 1.12x: 0.76 : 0.86 at 65^3, 0.89 : 0.96 at 193^3, 0.77 rows a voxel), above most
-//    rows of a column see one voxel (0.37 : 0.46 at 97^3, 1.81 rows a voxel).
+// automatic tuning, and these sizes (adjoint with its filter, ms, by rows : by
+// voxels):
+//  - between 0.8 and 1.9 rows a voxel.  Below, a row takes more than three voxels (0.076
+//    against 0.085 at 65^3, but 0.97 : 0.89 at 193^3, 0.77 rows a voxel), above most rows
+//    of a column see one voxel (0.46 : 0.37 at 97^3, 1.81 rows a voxel).  Launches of up to
+//    5000 waves wait for a wave's chain of read-add-writes by voxels, and gain up to 2.6
+//    rows a voxel (0.042 : 0.051 at 33^3 / 30 views, 0.068 : 0.076 at 49^3 / 36 views, 2 rows).
 //  - a column within 384 rows: more take a second wave that reads all columns again
 //    (1.69 : 2.57 at 225^3, 448 rows).
 //  - a volume of up to 48 MB.  Larger ones leave no columns for the next view in the
-//    L2s: a launch reads the volume once per view, 5.2 TB/s (137 MB x 360 views at
-//    325^3: 11.5 against the voxel kernel's 9.97, which walks in z and keeps columns).
+//    L2s: a launch reads the volume once per view, at 5.2 TB/s (137 MB x 360 views at
+//    325^3: 11.5 : 9.97, since the voxel kernel keeps columns).
 // Within them: 0.050 : 0.071 at 49^3 (36 views of 64^2), 0.117 : 0.172 at 65^3 (90 of
 // 96^2), 0.26 : 0.34 at 97^3 (90 of 160^2), 0.77 : 1.00 at 129^3 (180 of 192^2), 1.2 :
 // 1.54 at 161^3 (180 of 256^2), 2.75 : 3.00 at 225^3 (180 of 384^2).
@@ -1918,10 +1920,11 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
 // at 1150).
 int project_orbit(const BpGrid& g, const BpReach& r, const monte_tuning& t) {
   const double lo = r.svk * std::fabs(g.gsz) / (r.sod + r.rad), hi = r.svk * std::fabs(g.gsz) / (r.sod - r.rad);
-  if (t.pj_zchunk != 0 || !r.zeros || g.gsz <= 0 || !(lo > 0.8) || !(hi < 2.0) || !(hi * g.nz <= 384.0)) return 0;
+  if (t.pj_zchunk != 0 || !r.zeros || g.gsz <= 0 || !(lo > 0.8) || !(hi * g.nz <= 384.0)) return 0;
   if ((double)g.nx * g.ny * g.nz > 12e6) return 0;
-  if (t.bp_view_chunk > 0 && t.bp_view_chunk < g.n_views) return 1;  // orbits need the whole turn
   const long waves = (long)g.n_views * project_strips(g);
+  if (!(hi < (waves <= 5000 ? 2.6 : 1.9))) return 0;
+  if (t.bp_view_chunk > 0 && t.bp_view_chunk < g.n_views) return 1;  // orbits need the whole turn
   return r.turn != 0 && waves >= 40000 ? 4 : (r.half && waves >= 6000 ? 2 : 1);
 }
 

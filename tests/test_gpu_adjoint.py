@@ -152,6 +152,7 @@ _BY_ROWS = {
     "two_steep": dict(nx=21, ny=18, nz=50, n_views=9, step=1.8, nv=120),
     "long": dict(nx=9, ny=9, nz=354, n_views=8, nv=460, step=1.0),
     "longer": dict(nx=8, ny=9, nz=200, n_views=8, nv=500, step=1.75),
+    "two_steeper": dict(nx=14, ny=14, nz=31, n_views=8, step=2.4),
     "outside": dict(nx=30, ny=30, nz=120, n_views=8, nu=16, nv=20),
     "point": dict(nx=1, ny=1, nz=1, n_views=8),
 }
