@@ -90,15 +90,22 @@ int ensure_constants(monte_ctx* c, const monte_geom& g, const float** taps, cons
     compute_filter_taps(g, h);
     std::vector<BpView> v;
     compute_bp_views(g, v);
-    const size_t toff = 0, voff = align_up(h.size() * sizeof(float), 256);
+    std::vector<float> tables;
+    const int points = filter_fft_points(g.nu);
+    compute_filter_spectrum(g, points, filter_fft_lanes(points), tables);
+    const size_t toff = 0, foff = align_up(h.size() * sizeof(float), 256);
+    const size_t voff = align_up(foff + tables.size() * sizeof(float), 256);
     const size_t bytes = voff + v.size() * sizeof(BpView);
     char* base = (char*)workspace(c, kSlotConst, bytes);
     if (!base) return fail(c, MONTE_ERR_NOMEM, "constants allocation failed");
     MONTE_HIP(c, hipMemcpyAsync(base + toff, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
+    MONTE_HIP(c, hipMemcpyAsync(base + foff, tables.data(), tables.size() * sizeof(float), hipMemcpyHostToDevice,
+                                c->stream));
     MONTE_HIP(c, hipMemcpyAsync(base + voff, v.data(), v.size() * sizeof(BpView), hipMemcpyHostToDevice, c->stream));
     MONTE_HIP(c, hipStreamSynchronize(c->stream));
     c->const_key = key;
     c->taps_off = toff;
+    c->fft_off = foff;
     c->views_off = voff;
   }
   *taps = (const float*)((char*)c->ws[kSlotConst] + c->taps_off);
@@ -190,9 +197,8 @@ int run_filter_padded(monte_ctx* c, const monte_geom& g, const float* proj, floa
   int rc = ensure_constants(c, g, &taps, &views);
   if (rc) return rc;
   const FilterParams fp = compute_filter_params(g);
-  MONTE_HIP(c, launch_fdk_filter(proj, pad, taps, fp, c->stream));
-  MONTE_HIP(c, launch_fill_pads(pad, g.n_views, g.nu, g.nv, fp.pitch, fp.rows, g.preset == MONTE_PRESET_BP3D20,
-                                c->stream));
+  const float2* tables = (const float2*)((char*)c->ws[kSlotConst] + c->fft_off);
+  MONTE_HIP(c, launch_fdk_filter(proj, pad, taps, tables, fp, g.preset == MONTE_PRESET_BP3D20, c->stream));
   return MONTE_OK;
 }
 
@@ -256,7 +262,8 @@ int run_filter_T_padded(monte_ctx* c, const monte_geom& g, const float* pad, flo
   int rc = ensure_constants(c, g, &taps, &views);
   if (rc) return rc;
   const FilterParams fp = compute_filter_params(g);
-  MONTE_HIP(c, launch_fdk_filter_T(pad, proj, taps, fp, c->stream));
+  const float2* tables = (const float2*)((char*)c->ws[kSlotConst] + c->fft_off);
+  MONTE_HIP(c, launch_fdk_filter_T(pad, proj, taps, tables, fp, c->stream));
   return MONTE_OK;
 }
 

@@ -37,6 +37,15 @@ hipError_t launch_fill(float* p, float v, size_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Maps a hardware block index to a logical tile so that the blocks the
+// dispatcher sends to XCD x (blocks x, x+8, x+16, ...) cover one contiguous
+// range of logical tiles.  Tiles are numbered z-chunk slowest.
+__device__ inline int xcd_tile(int b, int nblocks) {
+  const int q = nblocks >> 3, r = nblocks & 7;
+  const int xcd = b & 7, j = b >> 3;
+  return xcd * q + (xcd < r ? xcd : r) + j;
+}
+
 // ---------------------------------------------------------------- filter
 __device__ inline float cos_weight(const FilterParams& fp, int r, int c) {
   const float a = fmaf(fp.b_u, (float)r, fp.a_u);
@@ -46,8 +55,8 @@ __device__ inline float cos_weight(const FilterParams& fp, int r, int c) {
 
 // The ramp filter of one view is a product with a Toeplitz matrix:
 //   out[v][b] = cs sum_c A[v][c] H[c][b],  H[c][b] = h[c - b + nu - 1],
-// with A the cosine-weighted projection (forward) or the filtered stack
-// (transpose; h is symmetric, so the same H serves).  Each block computes a
+// with A the cosine-weighted projection.  Long rows are filtered so (launch_fdk_filter has
+// the rule).  Each block computes a
 // 64 (v) x 64 kFnt (b) tile with v_mfma_f32_32x32x2_f32: wave w owns rows
 // 32 (w & 1) and the kFnt 32-column tiles at 32 kFnt (w >> 1).  A is staged in LDS
 // 32 columns of c at a time as As[c][v]; H is read straight from the taps in
@@ -57,7 +66,6 @@ __device__ inline float cos_weight(const FilterParams& fp, int r, int c) {
 // D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32].
 constexpr int kFnt = 4;  // 32-column product tiles per wave
 constexpr int kFbm = 64, kFbn = 64 * kFnt, kFkc = 32;
-static_assert(kFnt % 2 == 0, "the transposed filter stages its result two tiles per wave at a time");
 constexpr int kFas = kFbm + 1;  // LDS row pitch of As
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -150,102 +158,469 @@ __global__ __launch_bounds__(256) void filter_fwd_mfma_kernel(const float* __res
   }
 }
 
-// filt_pad [view][rows][pitch] (interior) -> proj [view][nu][nv], weighted: the
-// transpose of the forward filter.  Thread (tk, tr) stages A[v0 + tr + 8 j][c0 + tk],
-// j < 8, pipelined like the forward kernel; results go through LDS so the
-// [u][v] output is written in runs along v.
-__global__ __launch_bounds__(256) void filter_T_mfma_kernel(const float* __restrict__ in, float* __restrict__ proj,
-                                                            const float* __restrict__ taps, FilterParams fp) {
-  extern __shared__ float sm[];
-  float* const A0 = sm;  // double-buffered [kFkc][kFas]
-  float* const A1 = sm + kFkc * kFas;
-  float* Ht = sm + 2 * kFkc * kFas;
-  const int nu = fp.nu, nv = fp.nv;
-  const int v0 = blockIdx.x * kFbm, b0 = blockIdx.y * kFbn, view = blockIdx.z;
-  stage_taps(Ht, taps, nu);
-  const float* src = in + (size_t)view * fp.rows * fp.pitch;
-  const int tk = threadIdx.x & 31, tr = threadIdx.x >> 5;
-  float pre[kFbm / 8];
-  auto load = [&](int c0) {
-    const int c = c0 + tk, cc = c < nu ? c : nu - 1;
-#pragma unroll
-    for (int j = 0; j < kFbm / 8; ++j) {
-      const int v = v0 + tr + 8 * j;
-      pre[j] = src[(size_t)((v < nv ? v : nv - 1) + kPadLo) * fp.pitch + cc + kPadLo];
+// The ramp filter by FFT.  With N >= 2 nu points a row's circular convolution is the
+// linear one.  Rows v and v + 1 are the real and imaginary
+// parts of one transform (the taps are real).
+//   What is transformed is the row's difference x[n] - x[n - 1], against the taps' running
+// sum: a ramp filter takes most of a smooth row's size away, and rounding errors that a
+// transform of x itself spreads over all frequencies would stay (rel. errors of smooth
+// rows of 512: 7e-6 by x, 2e-6 by the sums of products, 1.3e-7 by differences).  The
+// running sum closes the circle with a tap in the unused lag N / 2 that makes the taps' sum
+// zero; the spectrum, scaled and with the running sum in it, is made in FP64 (spec).
+//   N = R1 M: M lanes hold a pair of rows, lane m the samples m + M n1.  R1 points in
+// registers, a twiddle, an exchange through LDS (a wave's own, real and imaginary parts
+// in turn), M points in registers, the spectrum, and the same way back.
+//   Rows of a pair 16 times apart in size (the rounding errors of one would show in the other)
+// or with a largest sample beyond 1e+-30 are scaled by powers of two; rows that are not
+// finite are summed directly.
+//   Bound by VALU instructions: 1600 of a wave's 2750 (two pairs of 512) are the four
+// transforms, 400 twiddles and spectrum, 450 the weighted tile.  360 views of 512^2 take
+// 0.285 ms and 0.271 transposed, for 0.94 and 0.87 as products with the taps' Toeplitz matrix
+// (103 TFLOP/s of fp32 matrix instructions, of 147 in a large product); 325^2 takes 0.17 ms
+// for 0.50, 1024 x 768 transposed 1.4 for 4.6.  Rows that just miss a power of two gain
+// least: 180 views of 600 x 512 transposed, with the copy in, 0.52 ms for 0.85.
+// y = DFT of x[OFF + STRIDE i], i < LEN, in order.  HALF: of x, only the first half and
+// x[R / 2] are not zero.
+template <int R, int LEN, int STRIDE, int OFF, bool INV, bool HALF>
+__device__ __forceinline__ void fft_regs(const float (&xr)[R], const float (&xi)[R], float (&yr)[LEN],
+                                         float (&yi)[LEN]) {
+  if constexpr (LEN == 2) {
+    const float ar = xr[OFF], ai = xi[OFF];
+    if constexpr (HALF && OFF != 0) {
+      yr[0] = yr[1] = ar;
+      yi[0] = yi[1] = ai;
+    } else {
+      const float br = xr[OFF + STRIDE], bi = xi[OFF + STRIDE];
+      yr[0] = ar + br;
+      yi[0] = ai + bi;
+      yr[1] = ar - br;
+      yi[1] = ai - bi;
     }
-  };
-  auto stage = [&](float* A, int c0) {
-    const bool cin = c0 + tk < nu;
+  } else {
+    constexpr int H = LEN / 2;
+    float er[H], ei[H], dr[H], di[H];
+    fft_regs<R, H, 2 * STRIDE, OFF, INV, HALF>(xr, xi, er, ei);
+    fft_regs<R, H, 2 * STRIDE, OFF + STRIDE, INV, HALF>(xr, xi, dr, di);
 #pragma unroll
-    for (int j = 0; j < kFbm / 8; ++j) {
-      const int vl = tr + 8 * j;
-      A[tk * kFas + vl] = (cin && v0 + vl < nv) ? pre[j] : 0.f;
-    }
-  };
-  load(0);
-  stage(A0, 0);
-  __syncthreads();
-  floatx16 acc[kFnt] = {};
-  int buf = 0;
-  for (int c0 = 0; c0 < nu; c0 += kFkc) {
-    const bool more = c0 + kFkc < nu;
-    if (more) load(c0 + kFkc);
-    mfma_chunk(buf ? A1 : A0, Ht, c0, b0, nu, acc);
-    if (more) stage(buf ? A0 : A1, c0 + kFkc);
-    __syncthreads();
-    buf ^= 1;
-  }
-  // stage D as Ds[b_local][v_local] over the same LDS (the loop ended on a
-  // barrier), two tiles per wave at a time, then write proj[b][v] along v.
-  // In pass h, Ds row bl holds b = b0 + 32 kFnt (bl / 64) + 64 h + bl % 64.
-  float* Ds = sm;  // [128][kFas]
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  float* dst = proj + (size_t)view * nu * nv;
-#pragma unroll
-  for (int h = 0; h < kFnt / 2; ++h) {
-    if (h > 0) __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int bl = (w >> 1) * 64 + 32 * t + (lane & 31);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int vl = (w & 1) * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-        Ds[bl * kFas + vl] = acc[2 * h + t][i];
+    for (int k = 0; k < H; ++k) {
+      if (k == 0) {
+        yr[0] = er[0] + dr[0];
+        yi[0] = ei[0] + di[0];
+        yr[H] = er[0] - dr[0];
+        yi[H] = ei[0] - di[0];
+      } else if (4 * k == LEN) {  // times -i, or i
+        const float tr = INV ? -di[k] : di[k], ti = INV ? dr[k] : -dr[k];
+        yr[k] = er[k] + tr;
+        yi[k] = ei[k] + ti;
+        yr[k + H] = er[k] - tr;
+        yi[k + H] = ei[k] - ti;
+      } else {
+        const float c = cos64(k * (64 / LEN)), sn = INV ? cos64(k * (64 / LEN) - 16) : -cos64(k * (64 / LEN) - 16);
+        yr[k] = fmaf(c, dr[k], fmaf(-sn, di[k], er[k]));
+        yi[k] = fmaf(c, di[k], fmaf(sn, dr[k], ei[k]));
+        yr[k + H] = fmaf(2.0f, er[k], -yr[k]);
+        yi[k + H] = fmaf(2.0f, ei[k], -yi[k]);
       }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 128 * kFbm; i += 256) {
-      const int bl = i / kFbm, vl = i - bl * kFbm;
-      const int b = b0 + (bl >> 6) * (32 * kFnt) + 64 * h + (bl & 63), v = v0 + vl;
-      if (b < nu && v < nv) dst[(size_t)b * nv + v] = fp.cs * Ds[bl * kFas + vl] * cos_weight(fp, b, v);
-    }
   }
 }
 
-// LDS bytes: two As buffers and the taps; the transposed filter also stages its
-// result, 128 x 64 at a time, over the same memory.
-static size_t filter_mfma_lds(int nu, bool transposed) {
-  const size_t stage = 2 * (size_t)kFkc * kFas + 2 * (size_t)nu + kFkc + 2 * kFbn;
-  const size_t out = transposed ? (size_t)128 * kFas : 0;
-  return sizeof(float) * (stage > out ? stage : out);
+__device__ inline void wave_lds_sync() {  // between a wave's own writes and reads of LDS
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-hipError_t launch_fdk_filter(const float* proj, float* filt_pad, const float* taps, const FilterParams& fp,
-                             hipStream_t s) {
-  const size_t lds = filter_mfma_lds(fp.nu, false);
-  if (lds > 64 * 1024) return hipErrorInvalidValue;
-  dim3 grid((fp.nv + kFbm - 1) / kFbm, (fp.nu + kFbn - 1) / kFbn, fp.n_views);
-  hipLaunchKernelGGL(filter_fwd_mfma_kernel, grid, dim3(256), lds, s, proj, filt_pad, taps, fp);
+// LDS words of a pair of rows: R1 rows of M + 1, padded so that the pairs of a wave
+// take different banks in the exchanges and in the staging of tiles.
+constexpr int fft_stride(int r1, int m) {
+  const int base = r1 * (m + 1);
+  return base + (((m % 32 + 2 - base) % 32 + 32) % 32);
+}
+
+// The cosine weight D / sqrt(s) to about an ulp: an estimate and a Newton step (the
+// divisions and roots above are four fifths of a transform's instructions).
+__device__ inline float cos_weight_of(float D, float s) {
+  const float y = __builtin_amdgcn_rsqf(s);
+  const float dy = D * y;
+  return fmaf(0.5f * dy, fmaf(-s * y, y, 1.0f), dy);
+}
+
+// TRANS false: proj [view][nu][nv], weighted, -> out [view][rows][pitch] with its guard
+// cells (wrap: of the bp3d20 preset, see fill_pads_kernel); true: the transpose (guard cells
+// not read).  A block takes 128 / M rows per wave.
+template <int R1, int M, bool TRANS>
+__global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 : 4)) void filter_fft_kernel(
+    const float* __restrict__ in, float* __restrict__ out, const float* __restrict__ taps,
+    const float2* __restrict__ twid, const float2* __restrict__ spec, FilterParams fp, int tiles, int wrap) {
+  constexpr int N = R1 * M, P = 64 / M, S = R1 / M, kHalf = N / 2, kStride = fft_stride(R1, M);
+  // tables in LDS (from L1, a block's twiddles and spectrum took as long as its transforms:
+  // 0.45 ms where it is 0.29), without the spectrum where 8 waves would not fit
+  constexpr bool kSpLds = N <= 1024;
+  // blocks take tiles in turn, loading the next one's samples while they write: 0.40 -> 0.27 ms
+  // for the transpose at 360 x 512^2; forward, 0.29 -> 0.44 (more waits at barriers)
+  constexpr bool kLoop = TRANS || N > 1024, kAhead = TRANS && R1 <= 32;
+  extern __shared__ float sm[];
+  const int waves = blockDim.x >> 6, rows_b = 2 * P * waves, rshift = 31 - __builtin_clz(rows_b);
+  float2* const twl = (float2*)sm;
+  float2* const spl = twl + N;
+  float* const bufs = sm + (kSpLds ? 4 : 2) * N;
+  const float2* const sp = kSpLds ? spl : spec;
+  const int nu = fp.nu, nv = fp.nv;
+  const int lane0 = threadIdx.x & 63, wave0 = threadIdx.x >> 6;
+  auto tables = [&] {
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+      twl[i] = twid[i];
+      if (kSpLds) spl[i] = spec[i];
+    }
+  };
+  if (kLoop) tables();
+  if (TRANS) __syncthreads();
+  // XCD x takes an eighth of the tiles, as xcd_tile deals them: a view's lines meet in one L2
+  const int xcd = blockIdx.x & 7, q8 = (tiles * fp.n_views) >> 3, r8 = (tiles * fp.n_views) & 7;
+  const int tile0 = xcd * q8 + min(xcd, r8), tile_end = tile0 + q8 + (xcd < r8 ? 1 : 0);
+  const int step = (gridDim.x + 7 - xcd) >> 3;
+  int tile = tile0 + (blockIdx.x >> 3);
+  if (tile >= tile_end) return;
+  // a tile's samples: of [nu][nv], thread t has sample t mod rows_b of the lines t / rows_b +
+  // j M / 2; of [v][u], a lane has its two rows
+  float nx[R1];
+  auto load = [&](int tl, int lane, int wave) {
+    const int view = tl / tiles, v0 = (tl - view * tiles) * rows_b;
+    if (TRANS) {
+      const int m = lane & (M - 1), v = v0 + 2 * (wave * P + lane / M);
+      const float* pad = in + (size_t)view * fp.rows * fp.pitch + kPadLo;
+      const float* row = pad + (size_t)(min(v, nv - 1) + kPadLo) * fp.pitch;
+      const float* row2 = pad + (size_t)(min(v + 1, nv - 1) + kPadLo) * fp.pitch;
+#pragma unroll
+      for (int j = 0; j < R1 / 2; ++j) {
+        const int uc = min(m + M * j, nu - 1);
+        nx[2 * j] = row[uc];
+        nx[2 * j + 1] = row2[uc];
+      }
+    } else {
+      const int t = wave * 64 + lane, tu = t >> rshift;
+      const float* src = in + (size_t)view * nu * nv + min(v0 + (t & (rows_b - 1)), nv - 1);
+#pragma unroll
+      for (int j = 0; j < R1; ++j) nx[j] = src[(size_t)min(tu + j * (M / 2), nu - 1) * nv];
+    }
+  };
+  if (kAhead) load(tile, lane0, wave0);
+  for (;;) {
+    int lane = lane0, wave = wave0;
+    if (kLoop) {  // opaque, or the loop's addresses and weights are kept in registers, and spilt
+      asm volatile("" : "+v"(lane));
+      asm volatile("" : "+v"(wave));
+    }
+    const int m = lane & (M - 1), pair = wave * P + lane / M;
+    float* const buf = bufs + pair * kStride;
+    float* const buf2 = buf + kHalf + 1;  // the second row when staging
+    const int view = tile / tiles, v0 = (tile - view * tiles) * rows_b, v = v0 + 2 * pair;
+    const float* proj = in + (size_t)view * nu * nv;                     // !TRANS
+    const float* pad = in + (size_t)view * fp.rows * fp.pitch + kPadLo;  // TRANS
+    const int t = wave * 64 + lane, tr = t & (rows_b - 1), tu = t >> rshift;
+    float* const tbuf = bufs + (tr >> 1) * kStride + (tr & 1) * (kHalf + 1) + tu;
+    const bool tin = v0 + tr < nv;
+    const float bv = fmaf(fp.b_v, (float)(v0 + tr), fp.a_v), bb = fmaf(fp.D, fp.D, bv * bv);
+    if (!kAhead) load(tile, lane, wave);
+    if (!TRANS) {
+#pragma unroll
+      for (int j = 0; j < R1; ++j) {
+        const int u = tu + j * (M / 2);
+        const float au = fmaf(fp.b_u, (float)u, fp.a_u);
+        const float w = cos_weight_of(fp.D, fmaf(au, au, bb));
+        tbuf[j * (M / 2)] = u < nu && tin ? nx[j] * w : 0.f;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < R1 / 2; ++j) {
+        const int u = m + M * j;
+        buf[u] = u < nu && v < nv ? nx[2 * j] : 0.f;
+        buf2[u] = u < nu && v + 1 < nv ? nx[2 * j + 1] : 0.f;
+      }
+      wave_lds_sync();
+    }
+    if (!kLoop) tables();
+    if (!TRANS) __syncthreads();
+
+    float yr[R1], yi[R1];  // at the end, filtered samples m + M n1 in the first half
+    if (v < nv) {
+      float xr[R1], xi[R1];
+      float big1 = 0.f, big2 = 0.f;  // largest samples (a NaN is left out)
+#pragma unroll
+      for (int j = 0; j < R1 / 2; ++j) {
+        const int u = m + M * j;
+        const float a = buf[u], b = buf2[u];
+        float a0 = buf[j == 0 ? max(u - 1, 0) : u - 1], b0 = buf2[j == 0 ? max(u - 1, 0) : u - 1];
+        if (j == 0 && m == 0) a0 = b0 = 0.f;
+        big1 = fmaxf(big1, fabsf(a));
+        big2 = fmaxf(big2, fabsf(b));
+        xr[j] = a - a0;
+        xi[j] = b - b0;
+        xr[R1 / 2 + j] = xi[R1 / 2 + j] = 0.f;
+      }
+      if (m == 0) {
+        xr[R1 / 2] = -buf[kHalf - 1];
+        xi[R1 / 2] = -buf2[kHalf - 1];
+      }
+#pragma unroll
+      for (int d = 1; d < M; d *= 2) {
+        big1 = fmaxf(big1, __shfl_xor(big1, d));
+        big2 = fmaxf(big2, __shfl_xor(big2, d));
+      }
+      const float big = fmaxf(big1, big2), low = big1 > 0.f && big2 > 0.f ? fminf(big1, big2) : big;
+      const bool scaled = big > 1e30f || low < fmaxf(1e-30f, big * (1.0f / 16.0f));
+      const int e1 = __builtin_amdgcn_frexp_expf(big1), e2 = __builtin_amdgcn_frexp_expf(big2);
+      if (scaled)
+#pragma unroll
+        for (int j = 0; j <= R1 / 2; ++j) {
+          xr[j] = ldexpf(xr[j], -e1);
+          xi[j] = ldexpf(xi[j], -e2);
+        }
+      fft_regs<R1, R1, 1, 0, false, true>(xr, xi, yr, yi);
+      // the lane's sums of differences, or NaN or infinity with one of them
+      float odd = fmaf(0.f, yr[0], 0.f * yi[0]);
+#pragma unroll
+      for (int d = 1; d < M; d *= 2) odd += __shfl_xor(odd, d);
+      const bool direct = !(odd == 0.f) || big == INFINITY;
+      if (direct) {
+#pragma unroll
+        for (int j = 0; j < R1; ++j) yr[j] = yi[j] = 0.f;
+#pragma unroll 1
+        for (int c = 0; c < nu; ++c) {
+          float a, b;
+          if (TRANS) {
+            a = pad[(size_t)(v + kPadLo) * fp.pitch + c];
+            b = v + 1 < nv ? pad[(size_t)(v + 1 + kPadLo) * fp.pitch + c] : 0.f;
+          } else {
+            a = proj[(size_t)c * nv + v] * cos_weight(fp, c, v);
+            b = v + 1 < nv ? proj[(size_t)c * nv + v + 1] * cos_weight(fp, c, v + 1) : 0.f;
+          }
+#pragma unroll
+          for (int j = 0; j < R1 / 2; ++j) {
+            const int u = m + M * j;
+            const float h = taps[u < nu ? c - u + nu - 1 : 0];
+            yr[j] = fmaf(a, h, yr[j]);
+            yi[j] = fmaf(b, h, yi[j]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < R1 / 2; ++j) {
+          yr[j] *= fp.cs;
+          yi[j] *= fp.cs;
+        }
+      } else {
+#pragma unroll
+        for (int k = 1; k < R1; ++k) {
+          const float2 t = twl[k * M + m];
+          const float a = yr[k];
+          yr[k] = fmaf(a, t.x, -yi[k] * t.y);
+          yi[k] = fmaf(a, t.y, yi[k] * t.x);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < R1; ++k) buf[k * (M + 1) + m] = yr[k];
+        wave_lds_sync();
+        float zr[S][M], zi[S][M];
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+#pragma unroll
+          for (int j = 0; j < M; ++j) zr[q][j] = buf[(m + M * q) * (M + 1) + j];
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < R1; ++k) buf[k * (M + 1) + m] = yi[k];
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+#pragma unroll
+          for (int j = 0; j < M; ++j) zi[q][j] = buf[(m + M * q) * (M + 1) + j];
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+          float fr[M], fi[M];
+          fft_regs<M, M, 1, 0, false, false>(zr[q], zi[q], fr, fi);
+#pragma unroll
+          for (int k = 0; k < M; ++k) {
+            const float2 t = sp[k * R1 + m + M * q];
+            const float a = fr[k];
+            fr[k] = fmaf(a, t.x, -fi[k] * t.y);
+            fi[k] = fmaf(a, t.y, fi[k] * t.x);
+          }
+          fft_regs<M, M, 1, 0, true, false>(fr, fi, zr[q], zi[q]);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+#pragma unroll
+          for (int j = 0; j < M; ++j) buf[(m + M * q) * (M + 1) + j] = zr[q][j];
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < R1; ++k) xr[k] = buf[k * (M + 1) + m];
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+#pragma unroll
+          for (int j = 0; j < M; ++j) buf[(m + M * q) * (M + 1) + j] = zi[q][j];
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < R1; ++k) xi[k] = buf[k * (M + 1) + m];
+#pragma unroll
+        for (int k = 1; k < R1; ++k) {
+          const float2 t = twl[k * M + m];
+          const float a = xr[k];
+          xr[k] = fmaf(a, t.x, xi[k] * t.y);
+          xi[k] = fmaf(-a, t.y, xi[k] * t.x);
+        }
+        fft_regs<R1, R1, 1, 0, true, false>(xr, xi, yr, yi);
+        if (scaled)
+#pragma unroll
+          for (int j = 0; j < R1 / 2; ++j) {
+            yr[j] = ldexpf(yr[j], e1);
+            yi[j] = ldexpf(yi[j], e2);
+          }
+        if (big1 == 0.f)  // (its partner's rounding errors)
+#pragma unroll
+          for (int j = 0; j < R1 / 2; ++j) yr[j] = 0.f;
+        if (big2 == 0.f)
+#pragma unroll
+          for (int j = 0; j < R1 / 2; ++j) yi[j] = 0.f;
+      }
+    }
+
+    if (TRANS) {
+      wave_lds_sync();
+      if (v < nv) {
+#pragma unroll
+        for (int j = 0; j < R1 / 2; ++j) {
+          buf[m + M * j] = yr[j];
+          buf2[m + M * j] = yi[j];
+        }
+      }
+      if (kAhead && tile + step < tile_end) load(tile + step, lane, wave);
+      __syncthreads();
+      float* dst = out + (size_t)view * nu * nv + v0 + tr;
+#pragma unroll 16
+      for (int j = 0; j < R1; ++j) {
+        const int u = tu + j * (M / 2);
+        const float au = fmaf(fp.b_u, (float)u, fp.a_u);
+        if (u < nu && tin) dst[(size_t)u * nv] = tbuf[j * (M / 2)] * cos_weight_of(fp.D, fmaf(au, au, bb));
+      }
+      if ((tile += step) >= tile_end) return;
+      __syncthreads();
+      continue;
+    }
+
+    float* const dst = out + (size_t)view * fp.rows * fp.pitch + kPadLo * fp.pitch + kPadLo;
+    const size_t plane = (size_t)fp.rows * fp.pitch;
+    if (v < nv) {
+      float* row = dst + (size_t)v * fp.pitch;
+#pragma unroll
+      for (int j = 0; j < R1 / 2; ++j) {
+        const int u = m + M * j;
+        if (u < nu) row[u] = yr[j];
+      }
+      if (v + 1 < nv) {
+        row += fp.pitch;
+#pragma unroll
+        for (int j = 0; j < R1 / 2; ++j) {
+          const int u = m + M * j;
+          if (u < nu) row[u] = yi[j];
+        }
+      }
+      // guard cells before and after these rows
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r = v + h;
+        if (r >= nv) break;
+        if (m < 1 + kPadHi && (!wrap || m == 0 || (r == nv - 1 && view == fp.n_views - 1)))
+          dst[(size_t)r * fp.pitch + (m == 0 ? -1 : nu + m - 1)] = 0.f;
+        if (!wrap) continue;
+        // the guard cells that alias sample (view, r, u), see fold_pads_kernel
+        if (m < kPadHi) {
+          const float y = h == 0 ? yr[0] : yi[0];
+          if (r >= 1) dst[(size_t)(r - 1) * fp.pitch + nu + m] = y;
+          if (view >= 1 && r <= kPadHi) (dst - plane)[(size_t)(nv + r - 1) * fp.pitch + nu + m] = y;
+        }
+        if (view >= 1 && r < kPadHi) {
+          float* above = dst - plane + (size_t)(nv + r) * fp.pitch;
+#pragma unroll
+          for (int j = 0; j < R1 / 2; ++j) {
+            const int u = m + M * j;
+            if (u < nu) above[u] = h == 0 ? yr[j] : yi[j];
+          }
+        }
+      }
+    }
+    // guard rows
+    if (v0 == 0)
+      for (int i = threadIdx.x; i < fp.pitch; i += blockDim.x) dst[i - fp.pitch - kPadLo] = 0.f;
+    if (v0 + rows_b >= nv)
+      for (int i = threadIdx.x; i < kPadHi * fp.pitch; i += blockDim.x) {
+        const int c = i % fp.pitch;
+        if (!wrap || c < kPadLo || view == fp.n_views - 1) dst[(size_t)nv * fp.pitch - kPadLo + i] = 0.f;
+      }
+    if (!kLoop || (tile += step) >= tile_end) return;
+    __syncthreads();
+  }
+}
+
+// Points of the row transforms, and lanes that hold a pair of rows.
+int filter_fft_points(int nu) {
+  int n = 128;
+  while (n < 2 * nu) n *= 2;
+  return n;
+}
+int filter_fft_lanes(int n) { return n >= 1024 ? 32 : (n == 128 ? 8 : 16); }
+
+template <bool TRANS>
+static hipError_t launch_filter_fft(const float* in, float* out, const float* taps, const float2* tables,
+                                    const FilterParams& fp, int wrap, hipStream_t s) {
+  if (fp.nu > 1024) return hipErrorInvalidValue;  // (check_geom)
+  const int n = filter_fft_points(fp.nu), m = filter_fft_lanes(n), per_wave = 128 / m;
+  int waves = n <= 1024 ? 4 : 8;
+  while (waves > 1 && (long)fp.n_views * ((fp.nv + per_wave * waves - 1) / (per_wave * waves)) < 512) waves /= 2;
+  const int rows_b = per_wave * waves, tiles = (fp.nv + rows_b - 1) / rows_b;
+  if ((long)tiles * fp.n_views > 0x3fffffffL) return hipErrorInvalidValue;
+  const size_t lds = sizeof(float) * ((n <= 1024 ? 4 : 2) * n + (size_t)(64 / m) * waves * fft_stride(n / m, m));
+  long blocks = (long)tiles * fp.n_views;
+  if (TRANS || n > 1024) blocks = std::min<long>(blocks, 256 * std::min<long>(160 * 1024 / lds, 16 / waves));
+#define MONTE_FFT(R, L)                                                                                        \
+  hipLaunchKernelGGL((filter_fft_kernel<R, L, TRANS>), dim3((unsigned)blocks), dim3(64 * waves), lds, s, in,   \
+                     out, taps, tables, tables + n, fp, tiles, wrap)
+  switch (n) {
+    case 128: MONTE_FFT(16, 8); break;
+    case 256: MONTE_FFT(16, 16); break;
+    case 512: MONTE_FFT(32, 16); break;
+    case 1024: MONTE_FFT(32, 32); break;
+    default:
+      if constexpr (TRANS) MONTE_FFT(64, 32);
+  }
+#undef MONTE_FFT
   return hipGetLastError();
 }
 
-hipError_t launch_fdk_filter_T(const float* filt_pad, float* proj, const float* taps, const FilterParams& fp,
-                               hipStream_t s) {
-  const size_t lds = filter_mfma_lds(fp.nu, true);
-  if (lds > 64 * 1024) return hipErrorInvalidValue;
-  dim3 grid((fp.nv + kFbm - 1) / kFbm, (fp.nu + kFbn - 1) / kFbn, fp.n_views);
-  hipLaunchKernelGGL(filter_T_mfma_kernel, grid, dim3(256), lds, s, filt_pad, proj, taps, fp);
-  return hipGetLastError();
+// Forward, rows of more than 512 samples stay products, at 5.2 ms for 1.5 (360 x 1024 x
+// 768): the filter's gain at a row's lowest frequencies, each of which has one factor in
+// FP32, is 1e-8 off by FFT, and sums over a volume, as the FP64 loss of a reconstruction's
+// residual, show it.  Products keep such a loss to 1e-9 (512^3 from 1024 x 768; 3e-8 by FFT);
+// up to 512 samples the scale's and the taps' rounding is as large.
+hipError_t launch_fdk_filter(const float* proj, float* filt_pad, const float* taps, const float2* tables,
+                             const FilterParams& fp, int wrap, hipStream_t s) {
+  if (fp.nu <= 512 && (!wrap || (fp.nu >= kPadHi && fp.nv > kPadHi)))
+    return launch_filter_fft<false>(proj, filt_pad, taps, tables, fp, wrap, s);
+  if (fp.nu <= 512) {  // guard cells past the next row or view
+    const hipError_t e = launch_filter_fft<false>(proj, filt_pad, taps, tables, fp, 0, s);
+    if (e != hipSuccess) return e;
+  } else {
+    const size_t lds = sizeof(float) * (2 * (size_t)kFkc * kFas + 2 * (size_t)fp.nu + kFkc + 2 * kFbn);
+    if (lds > 64 * 1024) return hipErrorInvalidValue;
+    const dim3 grid((fp.nv + kFbm - 1) / kFbm, (fp.nu + kFbn - 1) / kFbn, fp.n_views);
+    hipLaunchKernelGGL(filter_fwd_mfma_kernel, grid, dim3(256), lds, s, proj, filt_pad, taps, fp);
+  }
+  return launch_fill_pads(filt_pad, fp.n_views, fp.nu, fp.nv, fp.pitch, fp.rows, wrap, s);
+}
+
+hipError_t launch_fdk_filter_T(const float* filt_pad, float* proj, const float* taps, const float2* tables,
+                               const FilterParams& fp, hipStream_t s) {
+  return launch_filter_fft<true>(filt_pad, proj, taps, tables, fp, 0, s);
 }
 
 // -------------------------------------------------------------- pad copies
@@ -380,15 +755,6 @@ hipError_t launch_unpad_copy(const float* filt_pad, float* filt, int n_views, in
 }
 
 // ------------------------------------------------------- backprojection
-// Maps a hardware block index to a logical tile so that the blocks the
-// dispatcher sends to XCD x (blocks x, x+8, x+16, ...) cover one contiguous
-// range of logical tiles.  Tiles are numbered z-chunk slowest.
-__device__ inline int xcd_tile(int b, int nblocks) {
-  const int q = nblocks >> 3, r = nblocks & 7;
-  const int xcd = b & 7, j = b >> 3;
-  return xcd * q + (xcd < r ? xcd : r) + j;
-}
-
 
 // 1 / U and wn / dd to about an ulp: a hardware estimate and Newton steps, a
 // third of the instructions of the correctly rounded divisions.

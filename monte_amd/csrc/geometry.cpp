@@ -6,6 +6,7 @@
 // the presets differ only in these numbers (see BpView in internal.h).
 #include <algorithm>
 #include <cmath>
+#include <complex>
 
 #include "internal.h"
 
@@ -146,9 +147,9 @@ FilterParams compute_filter_params(const monte_geom& g) {
   return f;
 }
 
-void compute_filter_taps(const monte_geom& g, std::vector<float>& h) {
+static std::vector<double> filter_taps64(const monte_geom& g) {
   const int n = g.nu;
-  h.assign(2 * n - 1, 0.f);
+  std::vector<double> h(2 * n - 1);
   const bool shepp = g.preset == MONTE_PRESET_STANDARD && g.filter == MONTE_FILTER_SHEPP_LOGAN;
   for (int i = -(n - 1); i <= n - 1; ++i) {
     const int a = i < 0 ? -i : i;
@@ -162,7 +163,74 @@ void compute_filter_taps(const monte_geom& g, std::vector<float>& h) {
     } else {
       v = -1.0 / ((a * kPi) * (a * kPi));  // :60-61
     }
-    h[i + n - 1] = (float)v;
+    h[i + n - 1] = v;
+  }
+  return h;
+}
+
+void compute_filter_taps(const monte_geom& g, std::vector<float>& h) {
+  const std::vector<double> t = filter_taps64(g);
+  h.assign(t.begin(), t.end());
+}
+
+// What FP32 factors make of a sample that goes through a transform of n points in
+// registers and back (fft_regs): at each length a half of the terms are multiplied by a
+// factor whose square is not quite 1.
+static double regs_gain(int n) {
+  double g = 1.0;
+  for (int len = 8; len <= n; len *= 2)
+    for (int k = 0; k < len / 2; ++k) {
+      const double c = cos64(k * (64 / len)), s = cos64(k * (64 / len) - 16);
+      g += 0.5 * (c * c + s * s - 1.0) / (len / 2);
+    }
+  return g;
+}
+
+// The tables of the row transforms of `points` = R1 x lanes: twiddles
+// exp(-2 pi i k m / points) as [k < R1][m < lanes], then the spectrum of the taps'
+// running sum times the filter's scale / points (the inverse transform's).  The taps
+// h[-(nu - 1) .. nu - 1] get one more at lag points / 2 >= nu, which no sample of the
+// row is reached through, so that their sum is zero; their running sum's spectrum is
+// H(k) / (1 - exp(-2 pi i k / points)), and 0 at k = 0 where differences have none.
+//   The transforms' factors in FP32 are too small by 5e-8 to 1e-7 in all, the same in
+// every row; the spectrum makes up for it.
+void compute_filter_spectrum(const monte_geom& g, int points, int lanes, std::vector<float>& out) {
+  const int n = points;
+  std::vector<std::complex<double>> w(n), x(n);
+  for (int i = 0; i < n; ++i) w[i] = std::polar(1.0, -2.0 * kPi * i / n);
+  out.resize(4 * (size_t)n);
+  for (int k = 0; k < n / lanes; ++k)
+    for (int m = 0; m < lanes; ++m) {
+      out[2 * (k * lanes + m)] = (float)w[k * m % n].real();
+      out[2 * (k * lanes + m) + 1] = (float)w[k * m % n].imag();
+    }
+  const std::vector<double> h = filter_taps64(g);
+  double sum = 0.0;
+  for (double t : h) sum += t;
+  std::vector<double> c(n, 0.0);
+  for (int i = -(g.nu - 1); i < g.nu; ++i) c[(i + n) % n] = h[i + g.nu - 1];
+  c[n / 2] -= sum;
+  // radix 2, decimation in time
+  int bits = 0;
+  while ((1 << bits) < n) ++bits;
+  for (int i = 0; i < n; ++i) {
+    int j = 0;
+    for (int b = 0; b < bits; ++b) j |= ((i >> b) & 1) << (bits - 1 - b);
+    x[j] = c[i];
+  }
+  for (int len = 2; len <= n; len *= 2)
+    for (int i = 0; i < n; i += len)
+      for (int k = 0; k < len / 2; ++k) {
+        const std::complex<double> t = w[k * (n / len)] * x[i + k + len / 2];
+        x[i + k + len / 2] = x[i + k] - t;
+        x[i + k] += t;
+      }
+  const double scale = compute_filter_params(g).cs / (n * regs_gain(n / lanes) * regs_gain(lanes));
+  float* sp = out.data() + 2 * (size_t)n;
+  for (int k = 0; k < n; ++k) {
+    const std::complex<double> v = k ? scale * x[k].real() / (1.0 - w[k]) : 0.0;
+    sp[2 * k] = (float)v.real();
+    sp[2 * k + 1] = (float)v.imag();
   }
 }
 

@@ -105,6 +105,18 @@ BpGrid compute_bp_grid(const monte_geom& g);
 BpReach compute_bp_reach(const monte_geom& g, const BpGrid& grid);
 FilterParams compute_filter_params(const monte_geom& g);
 void compute_filter_taps(const monte_geom& g, std::vector<float>& h);  // h[0..2nu-2], centre nu-1
+// The factors cos(2 pi k / 64) of the filter's transforms
+constexpr float kCos64[17] = {
+    1.0f, 0.99518472667219693f, 0.98078528040323043f, 0.95694033573220882f, 0.92387953251128674f,
+    0.88192126434835505f, 0.83146961230254524f, 0.77301045336273699f, 0.70710678118654757f,
+    0.63439328416364549f, 0.55557023301960229f, 0.47139673682599781f, 0.38268343236508984f,
+    0.29028467725446233f, 0.19509032201612833f, 0.09801714032956077f, 0.0f};
+constexpr float cos64(int k) {
+  k &= 63;
+  return k <= 16 ? kCos64[k] : (k <= 32 ? -kCos64[32 - k] : (k <= 48 ? -kCos64[k - 32] : kCos64[64 - k]));
+}
+// Tables of the filter's row transforms: float2 twiddles [points], spectrum [points]
+void compute_filter_spectrum(const monte_geom& g, int points, int lanes, std::vector<float>& out);
 
 // ------------------------------------------------------------------- MC
 // Device attenuation tables of one job, per label and keV row:
@@ -255,7 +267,7 @@ struct monte_ctx {
 
   // FDK constants cached by geometry
   std::vector<double> const_key;
-  size_t taps_off = 0, views_off = 0;
+  size_t taps_off = 0, views_off = 0, fft_off = 0;
 
   // projector column lists cached by geometry: offsets, then the lists
   std::vector<double> plan_key;
@@ -301,8 +313,6 @@ void* noalloc_scratch(int device);
 // ---------------------------------------------------------- kernel launches
 // FDK (fdk.hip)
 hipError_t launch_fill(float* p, float v, size_t n, hipStream_t s);
-hipError_t launch_fdk_filter(const float* proj, float* filt_pad, const float* taps, const FilterParams& fp,
-                             hipStream_t s);
 hipError_t launch_pad_copy(const float* filt, float* filt_pad, int n_views, int nu, int nv, int pitch, int rows,
                            hipStream_t s);
 hipError_t launch_unpad_copy(const float* filt_pad, float* filt, int n_views, int nu, int nv, int pitch, int rows,
@@ -338,8 +348,14 @@ hipError_t launch_project(const float* volT, const BpView* views, int view0, int
 void projector_rows(const std::vector<BpView>& views, int view0, int n, const BpGrid& grid, int& lds_r0,
                     int& lds_rows);
 hipError_t launch_transpose_zx(const float* vol, float* volT, int nx, int ny, int nz, hipStream_t s);
-hipError_t launch_fdk_filter_T(const float* filt_pad, float* proj, const float* taps, const FilterParams& fp,
-                               hipStream_t s);
+// The filter with the guard cells (wrap: of the bp3d20 preset), and its transpose; tables of
+// compute_filter_spectrum.
+int filter_fft_points(int nu);
+int filter_fft_lanes(int points);
+hipError_t launch_fdk_filter(const float* proj, float* filt_pad, const float* taps, const float2* tables,
+                             const FilterParams& fp, int wrap, hipStream_t s);
+hipError_t launch_fdk_filter_T(const float* filt_pad, float* proj, const float* taps, const float2* tables,
+                               const FilterParams& fp, hipStream_t s);
 
 // MC (mc.hip)
 // The work queue is kMcQueues counters kMcQueueStride words apart, each

@@ -126,6 +126,85 @@ def test_filter_ragged_detectors(ctx, oracle, nu, nv):
     assert rel_max(t, t_ref) < TOL
 
 
+@pytest.mark.parametrize("views,nu,nv", [(1, 1, 9), (3, 4, 2), (7, 63, 31), (5, 64, 64), (3, 65, 9), (11, 128, 8),
+                                         (1, 129, 100), (9, 256, 63), (3, 257, 5), (13, 512, 33), (1, 513, 20),
+                                         (5, 1024, 37)])
+def test_filter_row_transforms(ctx, oracle, views, nu, nv):
+    """Rows at the ends of each transform length, odd numbers of rows and tiles; rows of noise, and rows whose mean dwarfs what the ramp leaves.
+    Tolerance: the weighted sample's rounding (6e-8 of up to 9 against outputs of about 1)
+    and as much again from the transform, on the largest of 1e4 samples."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk, fdk_backproject, fdk_filter, fdk_filter_adjoint
+
+    geom = G.small(n_views=views).replace(nu=nu, nv=nv, du=12.8 / nu, dv=12.8 / nv, u_off=0.03)
+    rng = np.random.default_rng(nu + nv)
+    og = oracle_geom(oracle, geom)
+    for mean in (0.0, 5.0):
+        proj = (rng.standard_normal(geom.proj_shape) + mean).astype(np.float32)
+        f = fdk_filter(_t(proj), geom, ctx).cpu().numpy()
+        f_ref = oracle.fdk_std_filter(og, oracle.fdk_std_weight(og, proj))
+        filt = (rng.standard_normal(geom.filt_shape) + mean).astype(np.float32)
+        t = fdk_filter_adjoint(_t(filt), geom, ctx).cpu().numpy()
+        t_ref = oracle.fdk_std_weight(og, oracle.fdk_std_filter_T(og, filt))
+        print(f"{nu} {nv} mean {mean}: {rel_max(f, f_ref):.2e} transposed {rel_max(t, t_ref):.2e}")
+        assert rel_max(f, f_ref) < 4e-6 and rel_max(t, t_ref) < 4e-6
+    # guard cells: the stages, which pad the stack by themselves, give the same volume (after a
+    # call that left other values where this one's guard cells are)
+    wide = geom.replace(nu=min(nu + 9, 1024), nv=nv + 5, u_off=0.0)
+    fdk(_t(np.full(wide.proj_shape, 1e6, np.float32)), wide, ctx)
+    vol = fdk(_t(proj), geom, ctx).cpu().numpy()
+    assert np.array_equal(vol, fdk_backproject(_t(f), geom, ctx).cpu().numpy())
+
+
+@pytest.mark.parametrize("views,side", [(1, 65), (3, 33), (5, 130), (9, 20), (4, 4), (5, 3), (3, 1)])
+def test_bp3d20_guard_cells(ctx, views, side):
+    """Guard cells hold the samples that the flat index reaches: as the stages have them."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk, fdk_backproject, fdk_filter
+
+    geom = G.bp3d20_65(n_views=views)
+    geom = geom.replace(nu=side, nv=side, du=geom.du * 60 / side, dv=geom.dv * 60 / side)  # (narrower than the volume)
+    proj = np.random.default_rng(side).standard_normal(geom.proj_shape).astype(np.float32)
+    wide = geom.replace(nu=side + 9, nv=side + 9)
+    fdk(_t(np.full(wide.proj_shape, 1e6, np.float32)), wide, ctx)
+    f = fdk_filter(_t(proj), geom, ctx)
+    vol = fdk(_t(proj), geom, ctx).cpu().numpy()
+    assert np.array_equal(vol, fdk_backproject(f, geom, ctx).cpu().numpy())
+
+
+@pytest.mark.parametrize("nu", [40, 100, 300, 512, 700])
+def test_filter_rows_do_not_mix(ctx, oracle, nu):
+    """Rows are transformed in pairs: a row's errors are of its own size, whatever its
+    neighbours hold (zeros, other sizes, the ends of the range, NaN and infinities)."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk_filter, fdk_filter_adjoint
+
+    scale = [1, 0, 0, 1e-3, 1e5, 1, 1e-30, 1, 1e34, 1, 1, 1e-36, 1e30, 1e34, 0, 0, 1, 100, np.nan, 1, 1, np.inf, 3]
+    geom = G.small(n_views=2).replace(nu=nu, nv=len(scale), du=12.8 / nu)
+    og = oracle_geom(oracle, geom)
+    rng = np.random.default_rng(nu)
+    rows = rng.standard_normal((2, len(scale), nu))
+    for v, sc in enumerate(scale):
+        if np.isfinite(sc):
+            rows[:, v] *= sc
+        else:
+            rows[:, v, nu // 3] = sc
+    filt = rows.astype(np.float32)
+    proj = np.ascontiguousarray(filt.transpose(0, 2, 1))
+    f = fdk_filter(_t(proj), geom, ctx).cpu().numpy()
+    t = fdk_filter_adjoint(_t(filt), geom, ctx).cpu().numpy().transpose(0, 2, 1)
+    f_ref = oracle.fdk_std_filter(og, oracle.fdk_std_weight(og, proj))
+    t_ref = oracle.fdk_std_weight(og, oracle.fdk_std_filter_T(og, filt)).transpose(0, 2, 1)
+    for v, sc in enumerate(scale):
+        for got, ref in ((f, f_ref), (t, t_ref)):
+            if not np.isfinite(sc):
+                assert not np.isfinite(got[:, v]).any(), v
+            elif sc == 0:
+                assert not got[:, v].any(), v
+            else:  # 1e-36: samples near the smallest normal number
+                assert rel_max(got[:, v], ref[:, v]) < (TOL if sc > 1e-33 else 1e-3), v
+
+
 def test_batch_equals_single(ctx):
     import torch
 
