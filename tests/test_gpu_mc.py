@@ -246,6 +246,45 @@ def test_counts_to_lineint_flat(ctx):
     assert rc == _lib.ERR_INVALID
 
 
+@pytest.mark.parametrize("kind", ["near_one", "intervals", "wide", "special"])
+def test_lineint_logarithm(ctx, kind):
+    """The conversion's logarithm over its ranges: around 1, at the ends of its table's intervals,
+    over the whole exponent range, and where it has none.  ln F - ln N in FP64 within 4e-16 of
+    each logarithm, then rounded to FP32 (6e-8)."""
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd.mc import counts_to_lineint_flat
+
+    geom = G.small(n_views=1).replace(nu=256, nv=15)
+    n = geom.nu * geom.nv
+    rng = np.random.default_rng(3)
+    u = rng.random(n)
+    if kind == "near_one":
+        flat, counts = 1 + u * 10.0 ** -rng.integers(0, 16, n), 1 + rng.random(n) * 10.0 ** -rng.integers(0, 16, n)
+    elif kind == "intervals":
+        edge = (1 + rng.integers(0, 129, n) / 128) * 2.0 ** rng.integers(0, 40, n)
+        flat, counts = np.nextafter(edge, edge * rng.choice([0.5, 2], n)), edge * 0.5
+    elif kind == "wide":
+        flat, counts = 10.0 ** rng.uniform(-307, 307, n), 10.0 ** rng.uniform(0, 307, n)
+    else:
+        flat = rng.choice([np.inf, 5e-324, 1e-310, 2.3e-308, 1.0, 0.0, -3.0, np.nan, 1e308, 7.0], n)
+        counts = rng.choice([np.inf, 0.0, -1.0, np.nan, 1.0, 5.0, 1e308], n)
+    flat, counts = flat.reshape(1, geom.nu, geom.nv), counts.reshape(1, geom.nu, geom.nv)
+    got = counts_to_lineint_flat(torch.from_numpy(counts).cuda(), geom, torch.from_numpy(flat).cuda(),
+                                 ctx).cpu().numpy().astype(np.float64)
+    with np.errstate(all="ignore"):
+        v = np.where(counts > flat, flat, counts)
+        v = np.where(v < 1.0, 1.0, v)
+        lf, lv = np.log(flat), np.log(v)
+        ref = np.where(flat > 0, lf - lv, 0.0)
+        ok = np.isfinite(ref)
+        assert np.array_equal(got[~ok], ref[~ok], equal_nan=True)
+        err, tol = np.abs(got - ref)[ok], (4e-16 * (np.abs(lf) + np.abs(lv)) + 1e-16 + 6.1e-8 * np.abs(ref))[ok]
+    assert np.all((err <= tol) | (ref[ok] == 0) & (got[ok] == 0))
+    assert np.all(got[(v == flat) & ok] == 0)
+
+
 def _box_chords(geom, lo, hi):
     """Closed-form chord lengths of every source -> pixel-centre ray through the box
     [lo, hi] (cm), standard preset: source at -sod (cos b, sin b, 0), pixel centre at
