@@ -172,6 +172,30 @@ def test_bp3d20_guard_cells(ctx, views, side):
     assert np.array_equal(vol, fdk_backproject(f, geom, ctx).cpu().numpy())
 
 
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("nz", [1, 3, 7])
+def test_volume_outside_region_is_cleared(ctx, shift, nz):
+    """A volume at any 4-byte address and of any size is zero outside the region, and nothing
+    around it is written."""
+    import ctypes as C
+
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd.fdk import _ptr, fdk
+
+    geom = G.bp3d20_65(n_views=2).replace(nx=9, ny=11, nz=nz, roi_x0=3, roi_x1=5)
+    proj = torch.randn(geom.proj_shape, device="cuda")
+    ref = fdk(proj, geom, ctx)
+    n = ref.numel()
+    buf = torch.full((n + 12,), 7.0, device="cuda")
+    g = geom.c()
+    ctx.call("monte_fdk", C.byref(g), _ptr(proj), _ptr(buf[4 + shift:]), 1)
+    assert torch.equal(buf[4 + shift:4 + shift + n].reshape(ref.shape), ref)
+    assert bool((buf[:4 + shift] == 7).all()) and bool((buf[4 + shift + n:] == 7).all())
+    assert not ref[..., :3].any() and not ref[..., 5:].any() and ref[..., 3:5].any()
+
+
 @pytest.mark.parametrize("nu", [40, 100, 300, 512, 700])
 def test_filter_rows_do_not_mix(ctx, oracle, nu):
     """Rows are transformed in pairs: a row's errors are of its own size, whatever its
