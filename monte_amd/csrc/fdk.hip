@@ -1151,12 +1151,16 @@ __global__ __launch_bounds__(1024) void backproject_kernel(const float* __restri
 
 // Volumes too small to fill the chip with tiles, and voxels so coarse on the
 // detector that a tile's patch does not fit in LDS: taps straight from the
-// padded views (four 4-byte gathers, 21.7 clocks a wave, where two 8-byte ones
-// cost 32.7).  A wave takes 64 columns in a row (x fastest) over ZC voxels, and
+// padded views, in two 8-byte gathers a voxel: a gather costs by the lines its lanes
+// reach, and four of 4 bytes took 443 us for 378 in the reference geometry's FDK, and
+// twice as long in volumes of 34^3 to 60^3 (158 : 73 us for 35 x 28 x 34 from 322 views).
+// A wave takes 64 columns in a row (x fastest) over ZC voxels, and
 // the block's waves share the views out, so a small volume's chain of views is
 // short (one voxel takes the latency of a view's set-up and gathers after
 // another); their sums are added in wave order, so the volume does not depend
 // on scheduling.
+typedef float Pair4 __attribute__((ext_vector_type(2), aligned(4)));  // two floats at any 4-byte address
+
 template <int ZC, bool ZEROS>
 __global__ __launch_bounds__(1024) void backproject_direct_kernel(const float* __restrict__ pad,
                                                                   const BpView* __restrict__ views, int view0,
@@ -1207,10 +1211,11 @@ __global__ __launch_bounds__(1024) void backproject_direct_kernel(const float* _
       const float b0 = m0 * fv, b1 = m1 * fv;
       const uint32_t at = off0 + (uint32_t)__mul24((int)(sc >> 32), g.pitch);
       sv += dv;
-      float val = (m0 - b0) * src[at];
-      val = fmaf(m1 - b1, src[at + 1], val);
-      val = fmaf(b0, src[at + (uint32_t)g.pitch], val);
-      val = fmaf(b1, src[at + (uint32_t)g.pitch + 1], val);
+      const Pair4 ta = *(const Pair4*)(src + at), tb = *(const Pair4*)(src + at + (uint32_t)g.pitch);
+      float val = (m0 - b0) * ta.x;
+      val = fmaf(m1 - b1, ta.y, val);
+      val = fmaf(b0, tb.x, val);
+      val = fmaf(b1, tb.y, val);
       acc[j] += val;
     }
   }
