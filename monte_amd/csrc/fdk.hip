@@ -1279,8 +1279,13 @@ struct BpPlan {
 // halves what the set-up costs a voxel), else of 8 or 4, whose views up to 4 groups
 // share; where 16 x 16 columns are too wide a patch, 8 x 8 of 4 times the
 // depth (99x72x92 on 373x75, 3 pixels a voxel: 0.92 ms with its adjoint straight
-// from memory).  117x83x109 from 61 views of 175x94 (252 tiles) took 143 us
-// straight from memory and 114 us by the kernel before these.
+// from memory).
+//   Orbits share a set-up and halve or quarter the tiles; shallow tiles pay more set-up
+// than they share: below 16 voxels (8 for quarter turns), single columns are taken, from
+// 40 views of 65^3 in 35 us for 45 and 193^3 in 216 for 263, from 122 views of 65^3 in
+// 72 for 97 and 241^3, 2.4 pixels a voxel, in 1.72 ms for 1.85 (but of 113^3, in 252 us
+// for 234).  Volumes that make fewer than 640 groups in tiles of 8 go straight from memory:
+// 57^3 from 61 views in 37 us for 42, 65^3 (900 groups) in 45 for 44.
 //
 // A region of fewer than 8 columns along x (the reference's 5 of 256) goes straight
 // from memory, whose waves take columns in a row: tiles of 8 x 8 would idle 24 lanes
@@ -1296,13 +1301,14 @@ static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
     for (int stack : {1, 4})
       for (int zc : {32, 16, 8, 4}) {
         if (zc == 32 && (orbit > 1 || stack > 1 || !r.zeros)) continue;
+        if (orbit > 1 && (stack > 1 || zc < (orbit == 4 ? 8 : 16))) continue;
         const int nx = orbit == 4 ? hx : g.x1 - g.x0, ny = orbit > 1 ? hy : g.ny;
         const int tx = stack == 1 ? 16 : 8, ty = 256 / (tx * stack);
         int rows, cols;
         patch_bounds(g, r, tx, ty, zc * stack, rows, cols);
         const long tiles = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((g.nz + zc * stack - 1) / (zc * stack));
         for (int groups : {1, 2, 4})
-          if (tiles * groups >= 512 && g.n_views >= 4 * groups && patch_fits(orbit, rows, cols, groups))
+          if (tiles * groups >= (zc < 16 && orbit == 1 ? 640 : 512) && g.n_views >= 4 * groups && patch_fits(orbit, rows, cols, groups))
             return {orbit, groups, zc, stack};
       }
   }
