@@ -142,12 +142,14 @@ typedef struct monte_tuning {
   int32_t mc_batch;          /* photon cycles per work unit of one 8x8 detector tile (about 64 * mc_batch
                                 histories per unit; views with fewer cycles group tiles).  monte_mc_batch
                                 and monte_mc_project halve it, down to 16, for launches of fewer than 32
-                                units per wave of the grid */
+                                units per wave of the grid, and down to 1 for fewer than 4 */
   int32_t mc_blocks_per_cu;  /* persistent grid = CUs * this */
-  int32_t bp_zchunk;         /* voxels along z per backprojection thread */
-  int32_t bp_tile_x, bp_tile_y; /* backprojection block tile (threads) */
+  int32_t bp_zchunk;         /* voxels along z per backprojection thread at most: 4, 8 or 16 (= the default:
+                                as many as the scan's tiles take, up to 32) */
+  int32_t bp_tile_x, bp_tile_y; /* columns of a backprojection tile, as far as its patches allow */
   int32_t bp_view_chunk;     /* views per backprojection launch */
-  int32_t pj_zchunk;         /* projector voxels per lane along z: 2, 4, 8, or 0 = the default (2) */
+  int32_t pj_zchunk;         /* 0 = by rows or by voxels, as the scan's sizes have it; 2, 4, 8: by voxels,
+                                so many per lane along z */
   int32_t mc_ray_brick;      /* > 0: a photon's first flight takes as Woodcock majorant the largest mu
                                 among the labels its source -> pixel line crosses (found per view and
                                 pixel on bricks of this many voxels a side); 0: the global majorant.
