@@ -5,9 +5,8 @@
 // Reference: recon/bp3d20_325.cpp:39-175 (weight :39-46, filter :51-81,
 // backprojection :91-175).  The reference runs these as scalar FP64 loops; here
 // each is one kernel:
-//   filter:  one block per (view, 16 detector columns); the weighted input
-//            tile is transposed through LDS and every thread keeps a 4 x NB
-//            register tile of outputs, so each LDS tap feeds 4 FMAs.
+//   filter:  a pair of detector rows is one complex transform, held by 8 to 32
+//            lanes; the weighted [u][v] tile is transposed through LDS.
 //   backprojection: one thread per voxel column (x,y), or per orbit of columns
 //            that a part of a turn maps onto each other, and ZC voxels along z.
 //            Along a column u, the distance weight and the v-slope are constant,
@@ -971,7 +970,8 @@ __global__ __launch_bounds__(1024) void backproject_kernel(const float* __restri
   const int wz = stack == 1 ? 0 : wave, wt = stack == 1 ? wave : 0;  // (its place along z and in the tile)
   const int xw = tx0 + wt % wx * 8, yw = ty0 + wt / wx * 8;
   const bool idle = xw >= xb || yw >= yb;  // (a wave past the edge only copies)
-  const int x = min(xw + lane % 8, xb - 1), y = min(yw + lane / 8, yb - 1);  // (past the end: repeats a column, never stored)
+  // (past the end: repeats a column, never stored)
+  const int x = min(xw + lane % 8, xb - 1), y = min(yw + lane / 8, yb - 1);
   const int zt = zc * ZC * stack, z0 = zt + wz * ZC;  // the tile's first voxel and the wave's
   // its groups of 16 start at zb; its first voxel's place from the middle of its group
   const int zb = ZC % kZBase == 0 ? z0 : (z0 / kZBase) * kZBase, joff = ZC % kZBase == 0 ? -kZMid : z0 - zb - kZMid;
@@ -1268,7 +1268,8 @@ static bool patch_fits(int orbit, int rows, int cols, int groups) {
 // Which kernel takes a backprojection: a property of the scan alone (sizes of
 // the default tiling), so the volume does not depend on the tuned tile shape.
 struct BpPlan {
-  int orbit;   // columns a thread owns: 4 or 2 where 1/4 or 1/2 of a turn maps the scan onto itself, 1, or 0: straight from memory
+  int orbit;   // columns a thread owns: 4 or 2 where 1/4 or 1/2 of a turn maps the scan onto itself, 1,
+               // or 0: straight from memory
   int groups;  // groups of 4 waves that share a tile's views out
   int zc;      // voxels per thread at most
   int stack;   // 1: a block's 4 waves lie side by side over its columns; 4: one above the other
@@ -1278,8 +1279,7 @@ struct BpPlan {
 // (2 per CU) at least: tiles of 16 voxels of z (32 for single columns, which
 // halves what the set-up costs a voxel), else of 8 or 4, whose views up to 4 groups
 // share; where 16 x 16 columns are too wide a patch, 8 x 8 of 4 times the
-// depth (99x72x92 on 373x75, 3 pixels a voxel: 0.92 ms with its adjoint straight
-// from memory).
+// depth.
 //   Orbits share a set-up and halve or quarter the tiles; shallow tiles pay more set-up
 // than they share: below 16 voxels (8 for quarter turns), single columns are taken, from
 // 40 views of 65^3 in 35 us for 45 and 193^3 in 216 for 263, from 122 views of 65^3 in
@@ -1289,7 +1289,8 @@ struct BpPlan {
 //
 // A region of fewer than 8 columns along x (the reference's 5 of 256) goes straight
 // from memory, whose waves take columns in a row: tiles of 8 x 8 would idle 24 lanes
-// of 64 (0.83 against 0.76 ms for the reference geometry's FDK).
+// of 64 (the reference geometry's FDK took 0.83 ms so, 0.76 straight from memory with
+// the filter and the gathers of then, and 0.38 now).
 static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
   // a group of 16 voxels has to stay within the 40 rows of group_v's clamp
   if (g.x1 - g.x0 < 8 || !(r.svk * std::fabs(g.gsz) / (r.sod - r.rad) <= 4.5)) return {0, 1, 8, 1};
@@ -1308,7 +1309,8 @@ static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
         patch_bounds(g, r, tx, ty, zc * stack, rows, cols);
         const long tiles = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((g.nz + zc * stack - 1) / (zc * stack));
         for (int groups : {1, 2, 4})
-          if (tiles * groups >= (zc < 16 && orbit == 1 ? 640 : 512) && g.n_views >= 4 * groups && patch_fits(orbit, rows, cols, groups))
+          if (tiles * groups >= (zc < 16 && orbit == 1 ? 640 : 512) && g.n_views >= 4 * groups &&
+              patch_fits(orbit, rows, cols, groups))
             return {orbit, groups, zc, stack};
       }
   }
@@ -1375,7 +1377,7 @@ hipError_t launch_backproject(const float* filt_pad, const BpView* views, int vi
     return sizeof(float) * (groups > 1 ? std::max(patch, (size_t)sums * 256) : patch);
   };
 #define MONTE_BP(ZC, NQ, ZEROS)                                                                                \
-  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256 * groups),                       \
+  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256 * groups), \
                      lds_of(PatchLayout<NQ>::kRS, NQ * ZC), s, filt_pad, views, view0, nviews_chunk,          \
                      grid, vol, accumulate, tile_x, tiles_x, tiles_y, rows, reach.turn, stack)
 #define MONTE_BP_Z(NQ, ZEROS)                                                                                    \
@@ -1492,7 +1494,9 @@ struct SlabRanges {
 };
 
 __device__ inline int bcast_i(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
-__device__ inline float bcast_f(float v, int src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); }
+__device__ inline float bcast_f(float v, int src) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
 __device__ inline double bcast_d(double v, int src) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), src);
