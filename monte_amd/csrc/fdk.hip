@@ -1280,6 +1280,9 @@ struct BpPlan {
 // halves what the set-up costs a voxel), else of 8 or 4, whose views up to 4 groups
 // share; where 16 x 16 columns are too wide a patch, 8 x 8 of 4 times the
 // depth.
+//   These stay while 16 voxels deep, or 8 with 2048 tiles: 61 views of 161^3, 3.4 columns a
+// voxel, take 381 us (487 straight from memory) at 0.9 rows a voxel, 432 (493) at 1.2; of
+// 113^3 in 900 tiles of 8 172 (152) at 1.6 rows, and in tiles of 4 243 (167) at 2.4.
 //   Orbits share a set-up and halve or quarter the tiles; shallow tiles pay more set-up
 // than they share: below 16 voxels (8 for quarter turns), single columns are taken, from
 // 40 views of 65^3 in 35 us for 45 and 193^3 in 216 for 263, from 122 views of 65^3 in
@@ -1308,6 +1311,7 @@ static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
         int rows, cols;
         patch_bounds(g, r, tx, ty, zc * stack, rows, cols);
         const long tiles = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((g.nz + zc * stack - 1) / (zc * stack));
+        if (stack > 1 && zc < 16 && (zc < 8 || tiles < 2048)) continue;
         for (int groups : {1, 2, 4})
           if (tiles * groups >= (zc < 16 && orbit == 1 ? 640 : 512) && g.n_views >= 4 * groups &&
               patch_fits(orbit, rows, cols, groups))

@@ -299,6 +299,7 @@ _BP_KINDS = {
     "one_stacked": dict(nx=100, ny=72, nz=90, n_views=21, nu=400, du=0.02),
     "half_stacked": dict(nx=100, ny=72, nz=93, n_views=22, nu=400, du=0.02),
     "quarter_stacked": dict(nx=101, ny=101, nz=131, n_views=24, nu=300, du=0.03),
+    "one_stacked_8": dict(nx=129, ny=129, nz=257, n_views=5, nu=300, du=0.02, nv=400, dv=0.015),
     "direct_few": dict(nx=33, ny=31, nz=45, n_views=9),
     "direct_coarse": dict(nx=130, ny=131, nz=140, n_views=3, vx=0.045, vy=0.045, vz=0.045, du=0.012, nu=500),
 }
