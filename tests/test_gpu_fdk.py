@@ -229,6 +229,41 @@ def test_filter_rows_do_not_mix(ctx, oracle, nu):
                 assert rel_max(got[:, v], ref[:, v]) < (TOL if sc > 1e-33 else 1e-3), v
 
 
+@pytest.mark.parametrize("nu", [40, 64, 300, 512, 700, 1024])
+def test_filter_rows_keep_their_own_precision(ctx, oracle, nu):
+    """A row's rms error is of its own size beside a row of the same transform that is 2 to 15 times
+    as large, or whose differences are (noise beside smooth rows, steps and single pixels).
+    Tolerance: a transform of N points and its inverse err by 0.6 eps sqrt(2 log2 N) rms, 1.7e-7 at
+    2048 points, and by sqrt(5 / 2) times as much where the neighbour is twice as large (scales are
+    powers of two); the weight's roundings are 1e-7 in all: 3e-7.  Forward rows are noise, whose
+    weighted samples' rounding the ramp does not enlarge."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk_filter, fdk_filter_adjoint
+
+    rng = np.random.default_rng(nu)
+    u = np.arange(nu)
+    noise = lambda s: s * rng.standard_normal(nu)  # noqa: E731
+    smooth, step, pixel = np.exp(-(((u - nu / 2) / (nu / 6)) ** 2)), (abs(u - nu / 2) < nu / 6) * 1.0, (u == nu // 3) * 1.0
+    rows = [noise(s) for r in (1, 2, 4, 8, 15) for s in (1, r, r, 1)]
+    n_noise = len(rows)
+    for other in (smooth, step, pixel):
+        rows += [other, noise(1), noise(1), other, other, noise(12), noise(1), 14 * other]
+    rows += [smooth, step, step, pixel, pixel, smooth]
+    rows = np.stack(rows).astype(np.float32)
+    geom = G.small(n_views=1).replace(nu=nu, nv=len(rows), du=12.8 / nu, dv=0.05)
+    og = oracle_geom(oracle, geom)
+    t = fdk_filter_adjoint(_t(rows[None]), geom, ctx).cpu().numpy()[0].T
+    t_ref = oracle.fdk_std_weight(og, oracle.fdk_std_filter_T(og, rows[None]))[0].T
+    proj = np.ascontiguousarray(rows[None].transpose(0, 2, 1))
+    f = fdk_filter(_t(proj), geom, ctx).cpu().numpy()[0]
+    f_ref = oracle.fdk_std_filter(og, oracle.fdk_std_weight(og, proj))[0]
+    et = [rel_l2(t[v], t_ref[v]) for v in range(len(rows)) if not np.array_equal(rows[v] != 0, pixel != 0)]
+    ef = [rel_l2(f[v], f_ref[v]) for v in range(n_noise)]
+    print(f"nu {nu}: transposed {max(et):.2e}, forward {max(ef):.2e}")
+    assert max(et) < 4e-7
+    assert max(ef) < (4e-7 if nu <= 512 else 8e-7)  # longer forward rows are sums of products, of error ~ sqrt(nu)
+
+
 def test_batch_equals_single(ctx):
     import torch
 
