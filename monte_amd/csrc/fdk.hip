@@ -16,6 +16,7 @@
 //            only the detector rows that slab projects to).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "internal.h"
 
@@ -2208,107 +2209,120 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
   const int chunks = (g.nz + 63) / 64, per_column = NQ * chunks;
 
   float accl[NQ][NR], accr[NQ][NR];
+  // careful: voxels that a row's tent leaves out are not multiplied
+  auto walk = [&](auto careful) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int p = 0; p < NR; ++p) accl[q][p] = accr[q][p] = 0.f;
+
+    for (int a = 0; a < NQ; ++a) {
+      const int ka = k + a * part;
+      const BpView& c = views[ka];
+      const size_t cell = (size_t)ka * n_strips + st;
+      const uint32_t beg = offs[cell], end = offs[cell + 1];
+      for (uint32_t b0 = beg; b0 < end; b0 += 64) {
+        const int ncols = (int)min(64u, end - b0);
+        // lane i prepares the i-th column: its weights and its line in fixed point
+        int cx = 0, cy = 0;
+        float wl = 0.f, wr = 0.f, d = 0.f;
+        long long q0 = 0;
+        uint32_t inv = 0;
+        int first = 0, last = -1;  // rows (from rbase) it reaches
+        if (lane < ncols) {
+          const uint32_t e = list[b0 + lane];
+          cx = (int)(e & 0xffffu);
+          cy = (int)(e >> 16);
+          const double X = voxel_x(g, cx), Y = voxel_y(g, cy);
+          const ColumnCore mine = column_core<true>(c, X, Y, (float)X, (float)Y, g);
+          // the centre of an odd volume is an orbit of one, taken NQ times
+          const float w = NQ > 1 && 2 * cx + 1 == g.nx && 2 * cy + 1 == g.ny ? mine.w / NQ : mine.w;
+          wr = w * mine.fu;
+          wl = w - wr;
+          const double A = fma(mine.kv, g.gz0, c.sv0) - (double)rbase, D = mine.kv * g.gsz, iD = recip64(D);
+          d = (float)D;
+          const double q = fmin(fmax((-1.0 - A) * iD, -1.0e8), 1.0e8);
+          q0 = __double2ll_rn(q * 4294967296.0);
+          inv = (uint32_t)__double2ll_rn(fmin(iD * 2147483648.0, 4294967295.0));
+          first = (int)floor(fmin(fmax(A - 1.0, -1.0e6), 1.0e6));
+          last = (int)ceil(fmin(fmax(fma((double)(g.nz - 1), D, A) + 1.0, -1.0e6), 1.0e6));
+        }
+        auto fetch = [&](int i, int slot) {
+          const int x = bcast_i(cx, i), y = bcast_i(cy, i);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's last reads are done
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) {
+            const int m = NQ == 2 ? 2 * q : (turn > 0 ? q : (4 - q) & 3);  // quarter turns (x, y) -> (n - 1 - y, x)
+            const int xq = m == 0 ? x : (m == 1 ? g.nx - 1 - y : (m == 2 ? g.nx - 1 - x : y));
+            const int yq = m == 0 ? y : (m == 1 ? x : (m == 2 ? g.ny - 1 - y : g.nx - 1 - x));
+            const char* col = (const char*)(volT + ((size_t)yq * g.nx + xq) * g.nz);
+            float* dst = cols + (slot * NQ + q) * slot_words + kRowPad;
+            for (int ch = 0; ch < chunks; ++ch)
+              if (ch * 64 + lane < g.nz) copy_to_lds(col + ch * 256, (uint32_t)lane * 4u, dst + ch * 64);
+          }
+        };
+        const int ahead = min(depth - 1, ncols);
+        for (int i = 0; i < ahead; ++i) fetch(i, i);
+        int slot = 0, fslot = ahead;
+        for (int i = 0; i < ncols; ++i) {
+          if (i + ahead < ncols) fetch(i + ahead, fslot);
+          if (++fslot == depth) fslot = 0;
+          wait_copies(min(ahead, ncols - 1 - i) * per_column);
+          const float wli = bcast_f(wl, i), wri = bcast_f(wr, i), di = bcast_f(d, i);
+          const long long q0i = bcast_ll(q0, i);
+          const uint32_t invi = (uint32_t)bcast_i((int)inv, i);
+          const int fi = bcast_i(first, i), la = bcast_i(last, i);
+          const float dm = di * -2.3283064365386963e-10f, d1 = di - 1.0f;  // 2^-32
+          const float* col = cols + slot * NQ * slot_words + kRowPad;
+#pragma unroll
+          for (int p = 0; p < NR; ++p) {
+            if (fi > 64 * p + 63 || la < 64 * p) continue;  // (uniform)
+            const uint64_t q = (uint64_t)invi * (uint32_t)(2 * lane + 128 * p) + (uint64_t)q0i;
+            const int z = clamp_i((int)(uint32_t)(q >> 32) + 1, -kRowPad, g.nz);
+            const float s0 = fmaf((float)(uint32_t)q, dm, d1);
+            float t[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) t[j] = fmaxf(1.0f - fabsf(fmaf((float)j, di, s0)), 0.f);
+#pragma unroll
+            for (int qq = 0; qq < NQ; ++qq) {
+              const float* v = col + qq * slot_words + z;
+              auto value = [&](int j) { return careful && t[j] == 0.f ? 0.f : v[j]; };
+              float sum = t[0] * value(0);
+#pragma unroll
+              for (int j = 1; j < J; ++j) sum = fmaf(t[j], value(j), sum);
+              accl[qq][p] = fmaf(wli, sum, accl[qq][p]);
+              accr[qq][p] = fmaf(wri, sum, accr[qq][p]);
+            }
+          }
+          if (++slot == depth) slot = 0;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch's copies
+      }
+      // column q of the next list belongs to the view of this list's column q + 1
+      if (NQ > 1) {
+#pragma unroll
+        for (int p = 0; p < NR; ++p) {
+          const float l0 = accl[0][p], r0 = accr[0][p];
+#pragma unroll
+          for (int q = 0; q + 1 < NQ; ++q) {
+            accl[q][p] = accl[q + 1][p];
+            accr[q][p] = accr[q + 1][p];
+          }
+          accl[NQ - 1][p] = l0;
+          accr[NQ - 1][p] = r0;
+        }
+      }
+    }
+  };
+  walk(std::false_type{});
+  // A voxel that is not finite reaches the rows it projects to, and no others: 0 times it is
+  // not 0.  Such strips are walked again.
+  bool finite = true;
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
 #pragma unroll
-    for (int p = 0; p < NR; ++p) accl[q][p] = accr[q][p] = 0.f;
-
-  for (int a = 0; a < NQ; ++a) {
-    const int ka = k + a * part;
-    const BpView& c = views[ka];
-    const size_t cell = (size_t)ka * n_strips + st;
-    const uint32_t beg = offs[cell], end = offs[cell + 1];
-    for (uint32_t b0 = beg; b0 < end; b0 += 64) {
-      const int ncols = (int)min(64u, end - b0);
-      // lane i prepares the i-th column: its weights and its line in fixed point
-      int cx = 0, cy = 0;
-      float wl = 0.f, wr = 0.f, d = 0.f;
-      long long q0 = 0;
-      uint32_t inv = 0;
-      int first = 0, last = -1;  // rows (from rbase) it reaches
-      if (lane < ncols) {
-        const uint32_t e = list[b0 + lane];
-        cx = (int)(e & 0xffffu);
-        cy = (int)(e >> 16);
-        const double X = voxel_x(g, cx), Y = voxel_y(g, cy);
-        const ColumnCore mine = column_core<true>(c, X, Y, (float)X, (float)Y, g);
-        // the centre of an odd volume is an orbit of one, taken NQ times
-        const float w = NQ > 1 && 2 * cx + 1 == g.nx && 2 * cy + 1 == g.ny ? mine.w / NQ : mine.w;
-        wr = w * mine.fu;
-        wl = w - wr;
-        const double A = fma(mine.kv, g.gz0, c.sv0) - (double)rbase, D = mine.kv * g.gsz, iD = recip64(D);
-        d = (float)D;
-        const double q = fmin(fmax((-1.0 - A) * iD, -1.0e8), 1.0e8);
-        q0 = __double2ll_rn(q * 4294967296.0);
-        inv = (uint32_t)__double2ll_rn(fmin(iD * 2147483648.0, 4294967295.0));
-        first = (int)floor(fmin(fmax(A - 1.0, -1.0e6), 1.0e6));
-        last = (int)ceil(fmin(fmax(fma((double)(g.nz - 1), D, A) + 1.0, -1.0e6), 1.0e6));
-      }
-      auto fetch = [&](int i, int slot) {
-        const int x = bcast_i(cx, i), y = bcast_i(cy, i);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's last reads are done
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          const int m = NQ == 2 ? 2 * q : (turn > 0 ? q : (4 - q) & 3);  // quarter turns (x, y) -> (n - 1 - y, x)
-          const int xq = m == 0 ? x : (m == 1 ? g.nx - 1 - y : (m == 2 ? g.nx - 1 - x : y));
-          const int yq = m == 0 ? y : (m == 1 ? x : (m == 2 ? g.ny - 1 - y : g.nx - 1 - x));
-          const char* col = (const char*)(volT + ((size_t)yq * g.nx + xq) * g.nz);
-          float* dst = cols + (slot * NQ + q) * slot_words + kRowPad;
-          for (int ch = 0; ch < chunks; ++ch)
-            if (ch * 64 + lane < g.nz) copy_to_lds(col + ch * 256, (uint32_t)lane * 4u, dst + ch * 64);
-        }
-      };
-      const int ahead = min(depth - 1, ncols);
-      for (int i = 0; i < ahead; ++i) fetch(i, i);
-      int slot = 0, fslot = ahead;
-      for (int i = 0; i < ncols; ++i) {
-        if (i + ahead < ncols) fetch(i + ahead, fslot);
-        if (++fslot == depth) fslot = 0;
-        wait_copies(min(ahead, ncols - 1 - i) * per_column);
-        const float wli = bcast_f(wl, i), wri = bcast_f(wr, i), di = bcast_f(d, i);
-        const long long q0i = bcast_ll(q0, i);
-        const uint32_t invi = (uint32_t)bcast_i((int)inv, i);
-        const int fi = bcast_i(first, i), la = bcast_i(last, i);
-        const float dm = di * -2.3283064365386963e-10f, d1 = di - 1.0f;  // 2^-32
-        const float* col = cols + slot * NQ * slot_words + kRowPad;
-#pragma unroll
-        for (int p = 0; p < NR; ++p) {
-          if (fi > 64 * p + 63 || la < 64 * p) continue;  // (uniform)
-          const uint64_t q = (uint64_t)invi * (uint32_t)(2 * lane + 128 * p) + (uint64_t)q0i;
-          const int z = clamp_i((int)(uint32_t)(q >> 32) + 1, -kRowPad, g.nz);
-          const float s0 = fmaf((float)(uint32_t)q, dm, d1);
-          float t[J];
-#pragma unroll
-          for (int j = 0; j < J; ++j) t[j] = fmaxf(1.0f - fabsf(fmaf((float)j, di, s0)), 0.f);
-#pragma unroll
-          for (int qq = 0; qq < NQ; ++qq) {
-            const float* v = col + qq * slot_words + z;
-            float sum = t[0] * v[0];
-#pragma unroll
-            for (int j = 1; j < J; ++j) sum = fmaf(t[j], v[j], sum);
-            accl[qq][p] = fmaf(wli, sum, accl[qq][p]);
-            accr[qq][p] = fmaf(wri, sum, accr[qq][p]);
-          }
-        }
-        if (++slot == depth) slot = 0;
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch's copies
-    }
-    // column q of the next list belongs to the view of this list's column q + 1
-    if (NQ > 1) {
-#pragma unroll
-      for (int p = 0; p < NR; ++p) {
-        const float l0 = accl[0][p], r0 = accr[0][p];
-#pragma unroll
-        for (int q = 0; q + 1 < NQ; ++q) {
-          accl[q][p] = accl[q + 1][p];
-          accr[q][p] = accr[q + 1][p];
-        }
-        accl[NQ - 1][p] = l0;
-        accr[NQ - 1][p] = r0;
-      }
-    }
-  }
+    for (int p = 0; p < NR; ++p) finite = finite && fabsf(accl[q][p]) + fabsf(accr[q][p]) < INFINITY;
+  if (__any(!finite)) walk(std::true_type{});
   // Two strips meet in a detector column: two addends onto zero, the same in
   // either order.  Guard cells are not used (standard preset).
 #pragma unroll

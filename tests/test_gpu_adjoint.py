@@ -191,6 +191,46 @@ def test_projector_by_rows_matches_oracle(ctx, oracle, name):
     assert np.array_equal(p, fdk_project(_t(y), g, ctx).cpu().numpy())
 
 
+@pytest.mark.parametrize("name", ["one", "half_odd", "quarter_odd", "three_voxels", "long"])
+def test_projector_by_rows_keeps_non_finite_voxels_to_their_rows(ctx, name):
+    """A NaN or an infinity in the volume reaches the cells that its voxel projects to, as by
+    voxels, and no cell beside them."""
+    from monte_amd.fdk import fdk_project
+
+    g = _by_rows_geometry(name)
+    rng = np.random.default_rng(17)
+    y = rng.standard_normal(g.vol_shape).astype(np.float32)
+    for bad in (np.nan, np.inf, -np.inf):
+        y[tuple(int(rng.integers(0, s)) for s in y.shape)] = bad
+    p = fdk_project(_t(y), g, ctx).cpu().numpy()
+    saved = ctx.tuning
+    try:
+        ctx.set_tuning(pj_zchunk=2)
+        p2 = fdk_project(_t(y), g, ctx).cpu().numpy()
+    finally:
+        ctx.set_tuning(**saved)
+    ok = np.isfinite(p2)
+    print(name, "cells that are not finite", int((~ok).sum()), "by rows", int((~np.isfinite(p)).sum()))
+    assert 0 < (~ok).sum() <= 3 * 4 * g.n_views
+    assert np.array_equal(np.isfinite(p), ok)
+    assert rel_max(p[ok], p2[ok]) < 3e-6
+
+
+def _by_rows_geometry(name):
+    import math
+
+    from monte_amd import geometry as G
+
+    kw = dict(_BY_ROWS[name])
+    back, step = kw.pop("back", False), kw.pop("step", 0.9)
+    v = 4.0 / max(kw["nx"], kw["ny"], 8)
+    nv = kw.pop("nv", int(kw["nz"] * step) + 14)
+    nu = kw.pop("nu", 60)
+    return G.Geometry(**{**dict(nu=nu, nv=nv, sod=40.0, sdd=80.0, du=10.2 / nu, dv=0.04, vx=v, vy=v,
+                                vz=step * 0.04 * 40.0 / 80.0, u_off=0.03, v_off=-0.02), **kw},
+                      dangle=-2.0 * math.pi / kw["n_views"] if back else None)
+
+
 def test_autograd_matches_fp64_finite_differences(ctx, oracle):
     """d/dp of L = sum(g * FDK(p)) at 33^3 / 64^2 / 30 views."""
     import torch
