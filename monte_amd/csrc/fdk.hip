@@ -2150,8 +2150,10 @@ hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& g
 // so they are the J consecutive voxels from z0 = floor((r - 1 - A) / D) + 1, J =
 // ceil(2 / D), at s0 = sv(z0) - r, s0 + D, ...  The sum is added to the lane's two
 // registers per row, for the column itself and for the one to its right.
-//   (r - 1 - A) / D is formed in 32.32 fixed point from the row's integer offset,
-// so z0 is its high word and s0 comes from the low one to 2^-22 rows.
+//   (r - 1 - A) / D is formed in 32.32 fixed point from the row's integer offset, and z0 is its
+// high word; s0 = A + z0 D - r in 32.32 as well, as the projector by voxels forms it, and the
+// tent of its upper 28 fraction bits in integers, to half an ulp of FP32.  (In FP32 from the
+// low word of the first, weights were 2.7e-8 to 4.7e-8 rms off, for 1.1e-8 to 1.8e-8 by voxels.)
 // A column's voxels come from memory straight into the wave's LDS, `depth` - 1
 // columns ahead, between zeros that the rows past its ends read.
 //   NQ > 1: as the backprojector, the NQ columns of an orbit share all of a row's
@@ -2162,6 +2164,19 @@ hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& g
 // lanes own voxels, two read-add-writes of LDS per voxel) took 9.97 ms at 325^3 ->
 // 360 views of 512^2.
 constexpr int kRowPad = 4;  // zeros before and after a column in LDS (>= J)
+constexpr float kTentUnit = 268435456.0f;  // 2^28: a whole row in the tents' fixed point
+
+__device__ inline int mad_i24(int a, int b, int c) {  // a b + c of 24-bit a and b (uniform)
+  int r;
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+  return r;
+}
+
+__device__ inline int median0(int a, int b) {  // of a, b and 0
+  int r;
+  asm("v_med3_i32 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 
 __device__ inline void wait_copies(int n) {  // until at most n copies to LDS are in flight
 #define MONTE_WAIT(N) asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory")
@@ -2225,9 +2240,10 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
         const int ncols = (int)min(64u, end - b0);
         // lane i prepares the i-th column: its weights and its line in fixed point
         int cx = 0, cy = 0;
-        float wl = 0.f, wr = 0.f, d = 0.f;
-        long long q0 = 0;
+        float wl = 0.f, wr = 0.f;
+        long long q0 = 0, s1 = 0;
         uint32_t inv = 0;
+        int dl = 0, dh = 0;  // D's fraction and whole part
         int first = 0, last = -1;  // rows (from rbase) it reaches
         if (lane < ncols) {
           const uint32_t e = list[b0 + lane];
@@ -2239,8 +2255,15 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
           const float w = NQ > 1 && 2 * cx + 1 == g.nx && 2 * cy + 1 == g.ny ? mine.w / NQ : mine.w;
           wr = w * mine.fu;
           wl = w - wr;
+          if (!careful) {  // the tents' scale
+            wr *= 1.0f / kTentUnit;
+            wl *= 1.0f / kTentUnit;
+          }
           const double A = fma(mine.kv, g.gz0, c.sv0) - (double)rbase, D = mine.kv * g.gsz, iD = recip64(D);
-          d = (float)D;
+          const long long df = __double2ll_rn(D * 4294967296.0);
+          dl = (int)(uint32_t)df;
+          dh = (int)((df - dl) >> 32);
+          s1 = __double2ll_rn((fmin(fmax(A, -1.0e6), 1.0e6) + 1.0) * 4294967296.0);
           const double q = fmin(fmax((-1.0 - A) * iD, -1.0e8), 1.0e8);
           q0 = __double2ll_rn(q * 4294967296.0);
           inv = (uint32_t)__double2ll_rn(fmin(iD * 2147483648.0, 4294967295.0));
@@ -2268,21 +2291,27 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
           if (i + ahead < ncols) fetch(i + ahead, fslot);
           if (++fslot == depth) fslot = 0;
           wait_copies(min(ahead, ncols - 1 - i) * per_column);
-          const float wli = bcast_f(wl, i), wri = bcast_f(wr, i), di = bcast_f(d, i);
-          const long long q0i = bcast_ll(q0, i);
+          const float wli = bcast_f(wl, i), wri = bcast_f(wr, i);
+          const long long q0i = bcast_ll(q0, i), s1i = bcast_ll(s1, i);
+          const int dli = bcast_i(dl, i), dhi = bcast_i(dh, i), step = dhi * (int)kTentUnit + (dli >> 4);
           const uint32_t invi = (uint32_t)bcast_i((int)inv, i);
           const int fi = bcast_i(first, i), la = bcast_i(last, i);
-          const float dm = di * -2.3283064365386963e-10f, d1 = di - 1.0f;  // 2^-32
           const float* col = cols + slot * NQ * slot_words + kRowPad;
 #pragma unroll
           for (int p = 0; p < NR; ++p) {
             if (fi > 64 * p + 63 || la < 64 * p) continue;  // (uniform)
             const uint64_t q = (uint64_t)invi * (uint32_t)(2 * lane + 128 * p) + (uint64_t)q0i;
             const int z = clamp_i((int)(uint32_t)(q >> 32) + 1, -kRowPad, g.nz);
-            const float s0 = fmaf((float)(uint32_t)q, dm, d1);
+            // sv(z) - r + 1, of which a tent's weight is the distance from the nearer of 0 and 2
+            const uint64_t f = (uint64_t)((long long)z * dli + s1i);
+            const int row = mad_i24(z, dhi, (int)(uint32_t)(f >> 32) - lane) - 64 * p;
+            const uint32_t at = __builtin_amdgcn_alignbit((uint32_t)row, (uint32_t)f, 4);
             float t[J];
 #pragma unroll
-            for (int j = 0; j < J; ++j) t[j] = fmaxf(1.0f - fabsf(fmaf((float)j, di, s0)), 0.f);
+            for (int j = 0; j < J; ++j) {
+              const uint32_t a = at + (uint32_t)(j * step);
+              t[j] = (float)median0((int)a, (int)((uint32_t)(2 * kTentUnit) - a)) * (careful ? 1.0f / kTentUnit : 1.0f);
+            }
 #pragma unroll
             for (int qq = 0; qq < NQ; ++qq) {
               const float* v = col + qq * slot_words + z;
