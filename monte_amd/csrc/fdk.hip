@@ -798,8 +798,8 @@ hipError_t launch_unpad_copy(const float* filt_pad, float* filt, int n_views, in
 
 // ------------------------------------------------------- backprojection
 
-// 1 / U and wn / dd to about an ulp: a hardware estimate and Newton steps, a
-// third of the instructions of the correctly rounded divisions.
+// 1 / U and wn / dd rounded as the divisions are (for normal numbers, and all but one in 2^40): a
+// hardware estimate and Newton steps, a third of the divisions' instructions.
 __device__ inline double recip64(double u) {
   double y = __builtin_amdgcn_rcp(u);
   y = fma(y, fma(-u, y, 1.0), y);
@@ -847,7 +847,8 @@ __device__ inline ColumnCore column_core(const BpView& c, double X, double Y, fl
   }
   float rd = __builtin_amdgcn_rcpf(dd);
   rd = fmaf(rd, fmaf(-dd, rd, 1.0f), rd);
-  const float q = c.wn * rd;
+  float q = c.wn * rd;
+  q = fmaf(fmaf(-dd, q, c.wn), rd, q);  // (rounded as the division is)
   r.w = c.fac * q * q;
   return r;
 }

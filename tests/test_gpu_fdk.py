@@ -264,6 +264,32 @@ def test_filter_rows_keep_their_own_precision(ctx, oracle, nu):
     assert max(ef) < (4e-7 if nu <= 512 else 8e-7)  # longer forward rows are sums of products, of error ~ sqrt(nu)
 
 
+def test_distance_weight_is_rounded_as_its_division(ctx):
+    """One view of ones, interior voxels: the weight (sod / U)^2 dangle itself, formed in FP32 from
+    a correctly rounded quotient.  The emulated sums round once more in FP64: equal but for a few."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk_backproject
+
+    geom = G.Geometry(nx=51, ny=66, nz=420, n_views=5, nu=96, nv=80, sod=30.0, sdd=60.0, du=0.1, dv=0.08, vx=0.04,
+                      vy=0.04, vz=2.6 / 420)
+    f4, f8 = np.float32, np.float64
+    g = geom.c()
+    for k in range(5):
+        f = np.zeros(geom.filt_shape, f4)
+        f[k] = 1.0
+        vol = fdk_backproject(_t(f), geom, ctx).cpu().numpy()
+        b = k * g.dangle
+        X = (-0.5 * 50 * 0.04 + np.arange(51) * 0.04).astype(f4).astype(f8)[None, :]
+        Y = (-0.5 * 65 * 0.04 + np.arange(66) * 0.04).astype(f4).astype(f8)[:, None]
+        inner = (f8(f4(np.sin(b))) * Y + 30.0).astype(f4).astype(f8)
+        dd = (f8(f4(np.cos(b))) * X + inner).astype(f4)
+        q = f4(30.0) / dd
+        w = f4(g.dangle) * q * q
+        same = vol[200:220] == w[None]
+        print(k, float(same.mean()))
+        assert same.mean() > 0.999
+
+
 def test_batch_equals_single(ctx):
     import torch
 
