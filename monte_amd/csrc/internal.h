@@ -311,6 +311,9 @@ int noalloc_setup(int device);  // with `device` current; 0 or a hipError_t
 void* noalloc_scratch(int device);
 
 // ---------------------------------------------------------- kernel launches
+// Blocks of `threads` that one launch may have: HIP takes fewer than 2^32 threads along an axis.
+constexpr uint64_t max_blocks(int threads) { return 0xffffffffull / (unsigned)threads; }
+
 // FDK (fdk.hip)
 hipError_t launch_fill(float* p, float v, size_t n, hipStream_t s);
 hipError_t launch_pad_copy(const float* filt, float* filt_pad, int n_views, int nu, int nv, int pitch, int rows,

@@ -1024,10 +1024,11 @@ __device__ inline int job_of_block(int n_jobs, uint32_t b, F begin) {
 // Flight boxes and brick sets of all jobs in one launch: they read the same
 // labels and do not depend on each other.  (A launch each per job, with the box
 // read back by the host in between, took 4.3 of 10 ms of 24 uneven jobs.)
-__global__ __launch_bounds__(256) void mc_prep_kernel(McPrep* __restrict__ preps, int n_jobs) {
-  const int j = job_of_block(n_jobs, blockIdx.x, [&](int i) { return preps[i].prep_begin; });
+__global__ __launch_bounds__(256) void mc_prep_kernel(McPrep* __restrict__ preps, int n_jobs, uint32_t block0) {
+  const uint32_t block = block0 + blockIdx.x;
+  const int j = job_of_block(n_jobs, block, [&](int i) { return preps[i].prep_begin; });
   McPrep& P = preps[j];
-  const uint32_t b = blockIdx.x - P.prep_begin;
+  const uint32_t b = block - P.prep_begin;
   if (b < P.box_blocks) {
     support_box(P, b);
     return;
@@ -1072,14 +1073,15 @@ __global__ void mc_boxes_kernel(const McPrep* __restrict__ preps, McJob* __restr
 // 325^3 / 512^2 / 360 views with the planes formed at every step, 3.2 ms so).
 template <bool PLANES>
 __global__ __launch_bounds__(kRayBlock) void ray_sets_kernel(const McPrep* __restrict__ preps, McJob* __restrict__ jobs,
-                                                             int n_jobs) {
+                                                             int n_jobs, uint32_t block0) {
   extern __shared__ double planes[];
-  const int j = job_of_block(n_jobs, blockIdx.x, [&](int i) { return preps[i].ray_begin; });
+  const uint32_t block = block0 + blockIdx.x;
+  const int j = job_of_block(n_jobs, block, [&](int i) { return preps[i].ray_begin; });
   const McPrep& P = preps[j];
   const RayGrid& R = P.ray;
   const int view_begin = jobs[j].view_begin;
   const int npix = R.nu * R.nv, per_view = (npix + kRayBlock - 1) / kRayBlock;
-  const uint32_t b = blockIdx.x - P.ray_begin;
+  const uint32_t b = block - P.ray_begin;
   const int kk = (int)(b / (uint32_t)per_view), pix = (int)(b - (uint32_t)kk * (uint32_t)per_view) * kRayBlock + (int)threadIdx.x;
   if (b == 0 && threadIdx.x == 0) set_job_box(P, jobs[j]);
   const double cb = P.cs64[2 * (view_begin + kk)], sb = P.cs64[2 * (view_begin + kk) + 1];
@@ -1170,19 +1172,24 @@ __global__ __launch_bounds__(kRayBlock) void ray_sets_kernel(const McPrep* __res
 
 hipError_t launch_mc_prep(McPrep* preps, int n_jobs, uint32_t prep_blocks, hipStream_t s) {
   if (n_jobs < 1 || prep_blocks == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(mc_prep_kernel, dim3(prep_blocks), dim3(256), 0, s, preps, n_jobs);
+  for (uint64_t b = 0; b < prep_blocks; b += max_blocks(256))  // the jobs' blocks together may pass a launch's limit
+    hipLaunchKernelGGL(mc_prep_kernel, dim3((unsigned)std::min(max_blocks(256), prep_blocks - b)), dim3(256), 0, s,
+                       preps, n_jobs, (uint32_t)b);
   return hipGetLastError();
 }
 
 hipError_t launch_ray_sets(const McPrep* preps, McJob* jobs, int n_jobs, uint32_t ray_blocks, uint64_t max_planes,
                            hipStream_t s) {
   if (n_jobs < 1 || ray_blocks == 0) return hipErrorInvalidValue;
-  // the planes of grids up to 4096 bricks along the axes together fit in 32 KB of LDS
-  if (max_planes <= 4096)
-    hipLaunchKernelGGL(ray_sets_kernel<true>, dim3(ray_blocks), dim3(kRayBlock), sizeof(double) * max_planes, s, preps,
-                       jobs, n_jobs);
-  else
-    hipLaunchKernelGGL(ray_sets_kernel<false>, dim3(ray_blocks), dim3(kRayBlock), 0, s, preps, jobs, n_jobs);
+  for (uint64_t b = 0; b < ray_blocks; b += max_blocks(kRayBlock)) {
+    const dim3 grid((unsigned)std::min(max_blocks(kRayBlock), ray_blocks - b));
+    // the planes of grids up to 4096 bricks along the axes together fit in 32 KB of LDS
+    if (max_planes <= 4096)
+      hipLaunchKernelGGL(ray_sets_kernel<true>, grid, dim3(kRayBlock), sizeof(double) * max_planes, s, preps, jobs,
+                         n_jobs, (uint32_t)b);
+    else
+      hipLaunchKernelGGL(ray_sets_kernel<false>, grid, dim3(kRayBlock), 0, s, preps, jobs, n_jobs, (uint32_t)b);
+  }
   return hipGetLastError();
 }
 

@@ -97,3 +97,34 @@ def test_smallest_jobs_match_oracle(ctx, oracle, batch_run):
             assert np.abs(z).max() < 3.0 and same > 0.95
         for k in ("tallied_primary", "tallied_scatter", "photo", "compton", "coherent"):
             assert abs(st[k] - st_ref[k]) <= max(10, 1e-3 * st_ref[k]), (i, k)
+
+
+def test_label_sets_past_one_launch(ctx):
+    """Ten jobs whose 4.7e9 first-flight label sets take more blocks than one launch may have (2^32
+    threads): the tallies of the same jobs one by one."""
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd import phantoms
+    from monte_amd.mc import McJobSpec, McSettings, device_labels, mc_batch
+
+    if torch.cuda.mem_get_info()[0] < 40e9:
+        pytest.skip("needs 20 GB of device memory")
+    geom = G.Geometry(n_views=300, nu=1024, nv=1536, nx=9, ny=9, nz=9, sod=20.0, sdd=40.0, du=0.01, dv=0.01, vx=1.0,
+                      vy=1.0, vz=1.0)
+    assert 10 * geom.n_views * geom.nu * geom.nv > 2**32
+    ph = phantoms.cube_phantom(9, 1.0, seed=3)
+    labels = device_labels(ph, "cuda")
+    tallies = [torch.zeros(geom.proj_shape, dtype=torch.float64, device="cuda") for _ in range(2)]
+
+    def jobs():
+        return [McJobSpec(ph, geom, McSettings(photons_per_view=2000, e_kev=60.0, job=j, seed=5), labels, *tallies)
+                for j in range(10)]
+
+    stats = mc_batch(jobs(), ctx=ctx)
+    assert all(s["histories"] == 2000 * 300 and s["interactions"] > 0 for s in stats)
+    single = [mc_batch([j], ctx=ctx)[0] for j in jobs()[:1] + jobs()[-1:]]
+    for a, b in zip((stats[0], stats[-1]), single):
+        assert {k: v for k, v in a.items() if k != "kernel_ms"} == {k: v for k, v in b.items() if k != "kernel_ms"}
+    total = float(tallies[0].sum() + tallies[1].sum())
+    assert total == sum(s["tallied_primary"] + s["tallied_scatter"] for s in stats + single)
