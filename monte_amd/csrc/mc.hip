@@ -1384,17 +1384,24 @@ hipError_t launch_primary_exact(const PrimaryGeom& P, const McPrep* prep, const 
                                 const double* bins, int n_bins, int n_labels, double weight, float* out,
                                 hipStream_t s) {
   const uint64_t rows8 = ((P.nv + kPrimV - 1) / kPrimV + 7) / 8;
-  const uint64_t blocks = 8 * rows8 * (uint64_t)P.n_views * ((P.nu + kPrimU - 1) / kPrimU);
-  if (blocks == 0) return hipSuccess;
-  if (blocks > 0x7fffffffull || n_labels < 0 || n_labels > kMaxLabels) return hipErrorInvalidValue;
+  const uint64_t per_view = 8 * rows8 * ((P.nu + kPrimU - 1) / kPrimU);
+  if (per_view == 0 || P.n_views <= 0) return hipSuccess;
+  if (n_labels < 0 || n_labels > kMaxLabels) return hipErrorInvalidValue;
   const uint64_t np = (uint64_t)P.n[0] + P.n[1] + P.n[2] + 3;
   const size_t lens = sizeof(double) * n_labels * kPrimU * kPrimV;
-  if (np <= 3900)  // with 16 labels' lengths, 63 KB of LDS
-    hipLaunchKernelGGL(primary_exact_kernel<true>, dim3((unsigned)blocks), dim3(kPrimU * kPrimV),
-                       lens + sizeof(double) * np, s, P, prep, cs64, labels, bins, n_bins, n_labels, weight, out);
-  else
-    hipLaunchKernelGGL(primary_exact_kernel<false>, dim3((unsigned)blocks), dim3(kPrimU * kPrimV), lens, s, P, prep,
-                       cs64, labels, bins, n_bins, n_labels, weight, out);
+  const int step = (int)std::min<uint64_t>(P.n_views, max_blocks(kPrimU * kPrimV) / per_view);  // views of a launch
+  for (int k = 0; k < P.n_views; k += step) {
+    PrimaryGeom Q = P;
+    Q.n_views = std::min(step, P.n_views - k);
+    const dim3 grid((unsigned)(per_view * Q.n_views));
+    float* o = out + (size_t)k * P.nu * P.nv;
+    if (np <= 3900)  // with 16 labels' lengths, 63 KB of LDS
+      hipLaunchKernelGGL(primary_exact_kernel<true>, grid, dim3(kPrimU * kPrimV), lens + sizeof(double) * np, s, Q, prep,
+                         cs64 + 2 * (size_t)k, labels, bins, n_bins, n_labels, weight, o);
+    else
+      hipLaunchKernelGGL(primary_exact_kernel<false>, grid, dim3(kPrimU * kPrimV), lens, s, Q, prep,
+                         cs64 + 2 * (size_t)k, labels, bins, n_bins, n_labels, weight, o);
+  }
   return hipGetLastError();
 }
 

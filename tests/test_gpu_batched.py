@@ -128,3 +128,5 @@ def test_label_sets_past_one_launch(ctx):
         assert {k: v for k, v in a.items() if k != "kernel_ms"} == {k: v for k, v in b.items() if k != "kernel_ms"}
     total = float(tallies[0].sum() + tallies[1].sum())
     assert total == sum(s["tallied_primary"] + s["tallied_scatter"] for s in stats + single)
+    del tallies
+    torch.cuda.empty_cache()

@@ -337,6 +337,27 @@ def test_primary_exact_box_closed_form(ctx):
     assert err.max() < 1e-5
 
 
+def test_primary_exact_views_past_one_launch(ctx):
+    """More views of one pixel than one launch holds (2^32 threads, eight tile rows a view): every
+    turn of 1000 views is the first."""
+    import math
+
+    import torch
+
+    from monte_amd import geometry as G
+    from monte_amd import phantoms
+    from monte_amd.mc import primary_exact
+
+    geom = G.small(n_views=1000).replace(nu=1, nv=1, dangle=2 * math.pi / 1000, u_off=0.7)
+    ph = phantoms.small_phantom()
+    ref = primary_exact(ph, geom, e_kev=60.0, ctx=ctx)
+    views = 2_200_000
+    assert views * 8 * 256 > 2**32
+    got = primary_exact(ph, geom.replace(n_views=views), e_kev=60.0, ctx=ctx).reshape(-1, 1000)
+    assert float(ref.max()) > 0
+    assert float((got - ref.reshape(1, 1000)).abs().max()) <= 1e-5 * float(ref.max())
+
+
 def test_woodcock_majorant_invariance(ctx):
     """A label that no voxel carries, made dense, raises the global Woodcock majorant
     (more virtual steps per history) without changing the physics: both runs
