@@ -1368,14 +1368,21 @@ __global__ __launch_bounds__(kPrimU * kPrimV) void primary_exact_kernel(PrimaryG
   if (any) {
     // bins: per spectral bin its weight and the attenuation of each label (one bin
     // of weight 1 when mono-energetic)
-    double num = 0.0, le = 0.0;
-    for (int e = 0; e < n_bins; ++e) {
-      const double* b = bins + (size_t)e * (n_labels + 1);
-      le = 0.0;
-      for (int l = 0; l < n_labels; ++l) le += lens[l * kBlock + tid] * b[1 + l];
-      if (weight > 0.0) num += b[0] * exp(-le);
-    }
-    result = weight > 0.0 ? -log(num / weight) : le;
+    auto combine = [&](bool opaque) {
+      double num = 0.0, le = 0.0;
+      for (int e = 0; e < n_bins; ++e) {
+        const double* b = bins + (size_t)e * (n_labels + 1);
+        le = 0.0;
+        for (int l = 0; l < n_labels; ++l) {
+          const double len = lens[l * kBlock + tid];
+          if (!opaque || len != 0.0) le += len * b[1 + l];
+        }
+        if (weight > 0.0) num += b[0] * exp(-le);
+      }
+      return weight > 0.0 ? -log(num / weight) : le;
+    };
+    result = combine(false);
+    if (result != result) result = combine(true);  // 0 of a label of infinite attenuation is nothing
   }
   out[((size_t)k * P.nu + iu) * P.nv + iv] = (float)result;
 }

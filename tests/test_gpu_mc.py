@@ -358,6 +358,25 @@ def test_primary_exact_views_past_one_launch(ctx):
     assert float((got - ref.reshape(1, 1000)).abs().max()) <= 1e-5 * float(ref.max())
 
 
+@pytest.mark.parametrize("spectral", [False, True])
+def test_primary_exact_opaque_label(ctx, spectral):
+    """A label of infinite density stops the rays that cross it and leaves the others as they are."""
+    from monte_amd import geometry as G
+    from monte_amd import phantoms, tables
+    from monte_amd.mc import primary_exact
+    from monte_amd.phantoms import LabelPhantom
+
+    geom = G.small(n_views=5)
+    ph = phantoms.small_phantom()
+    spec = tables.kramers_spectrum(120.0, 2.5) if spectral else None
+    run = lambda rods: primary_exact(LabelPhantom(ph.labels, ph.voxel, [ph.materials[0], ph.materials[1], rods], ph.origin),  # noqa: E731
+                                     geom, e_kev=60.0, spectrum=spec, ctx=ctx).cpu().numpy()
+    got, clear, solid = run((tables.CALCIUM, np.inf)), run((-1, 0.0)), run((tables.CALCIUM, 1.55))
+    crossed = solid != clear
+    assert 0.01 < crossed.mean() < 0.5
+    assert np.all(np.isposinf(got[crossed])) and np.array_equal(got[~crossed], clear[~crossed])
+
+
 def test_woodcock_majorant_invariance(ctx):
     """A label that no voxel carries, made dense, raises the global Woodcock majorant
     (more virtual steps per history) without changing the physics: both runs
