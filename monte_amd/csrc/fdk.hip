@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void fill_kernel(float* __restrict__ p, float 
 
 hipError_t launch_fill(float* p, float v, size_t n, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  const size_t blocks = std::min<size_t>((n + 1023) / 1024, 0x7fffffff);
+  const size_t blocks = std::min<size_t>((n + 1023) / 1024, max_blocks(256));  // (the rest by looping)
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, v, n);
   return hipGetLastError();
 }
@@ -623,6 +623,7 @@ static hipError_t launch_filter_fft(const float* in, float* out, const float* ta
   if ((long)tiles * fp.n_views > 0x3fffffffL) return hipErrorInvalidValue;
   const size_t lds = sizeof(float) * ((n <= 1024 ? 4 : 2) * n + (size_t)(64 / m) * waves * fft_stride(n / m, m));
   long blocks = (long)tiles * fp.n_views;
+  if (!TRANS && blocks > (long)max_blocks(64 * waves)) return hipErrorInvalidValue;
   if (TRANS || n > 1024) blocks = std::min<long>(blocks, 256 * std::min<long>(160 * 1024 / lds, 16 / waves));
 #define MONTE_FFT(R, L)                                                                                        \
   hipLaunchKernelGGL((filter_fft_kernel<R, L, TRANS>), dim3((unsigned)blocks), dim3(64 * waves), lds, s, in,   \
@@ -1204,9 +1205,9 @@ template <int ZC, bool ZEROS>
 __global__ __launch_bounds__(1024) void backproject_direct_kernel(const float* __restrict__ pad,
                                                                   const BpView* __restrict__ views, int view0,
                                                                   int nviews, BpGrid g, float* __restrict__ vol,
-                                                                  int accumulate, int col_blocks) {
+                                                                  int accumulate, int col_blocks, int zc0) {
   extern __shared__ float part[];  // [waves][ZC][64]
-  const int cb_i = blockIdx.x % col_blocks, zc = blockIdx.x / col_blocks;
+  const int cb_i = blockIdx.x % col_blocks, zc = zc0 + blockIdx.x / col_blocks;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int ncx = g.x1 - g.x0, ncol = ncx * g.ny;
   const int col = min(cb_i * 64 + lane, ncol - 1);
@@ -1385,15 +1386,19 @@ hipError_t launch_backproject(const float* filt_pad, const BpView* views, int vi
     constexpr int zd = 8;
     const long ncol = (long)ncx * grid.ny, cb = (ncol + 63) / 64;
     const int most = std::min(16, std::max(1, nviews_chunk / 2));
-    const long blocks = cb * ((grid.nz + zd - 1) / zd);
+    const int zchunks = (grid.nz + zd - 1) / zd;
     int waves = 1;
-    while (2 * waves <= most && blocks * waves < 4096) waves *= 2;
-    if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    while (2 * waves <= most && cb * zchunks * waves < 4096) waves *= 2;
+    const int step = (int)std::min<long>(zchunks, max_blocks(64 * waves) / cb);  // chunks of z of a launch
+    if (step == 0) return hipErrorInvalidValue;
 #define MONTE_BP(ZEROS)                                                                                        \
-  hipLaunchKernelGGL((backproject_direct_kernel<zd, ZEROS>), dim3((unsigned)blocks), dim3(64 * waves),         \
+  hipLaunchKernelGGL((backproject_direct_kernel<zd, ZEROS>), dim3((unsigned)(cb * n)), dim3(64 * waves),       \
                      sizeof(float) * waves * zd * 64, s, filt_pad, views, view0, nviews_chunk, grid, vol,      \
-                     accumulate, (int)cb)
-    if (reach.zeros) MONTE_BP(true); else MONTE_BP(false);
+                     accumulate, (int)cb, z)
+    for (int z = 0; z < zchunks; z += step) {
+      const int n = std::min(step, zchunks - z);
+      if (reach.zeros) MONTE_BP(true); else MONTE_BP(false);
+    }
 #undef MONTE_BP
     return hipGetLastError();
   }
@@ -1406,14 +1411,15 @@ hipError_t launch_backproject(const float* filt_pad, const BpView* views, int vi
   };
   int rows, cols;
   patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
-  if (!patch_fits(nq, rows, cols, groups)) {  // the tuned shape does not fit: the default does
+  const long most_blocks = (long)max_blocks(256 * groups);
+  if (!patch_fits(nq, rows, cols, groups) || blocks_of(tile_x, zc) > most_blocks) {  // not the tuned shape: the default
     tile_x = stack == 1 ? 16 : 8;
     zc = plan.zc;
     patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
   }
   const int tiles_x = (nx + tile_x - 1) / tile_x, tile_y = 256 / (tile_x * stack), tiles_y = (ny + tile_y - 1) / tile_y;
   const long nblocks = blocks_of(tile_x, zc);
-  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+  if (nblocks > most_blocks) return hipErrorInvalidValue;
   // the groups' patches, which the sums of a group go through at the end
   auto lds_of = [&](int row_words, int sums) {
     const size_t patch = (size_t)2 * rows * row_words * groups;
@@ -2130,7 +2136,7 @@ hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& g
                                uint32_t* list, bool write, hipStream_t s) {
   const long nblocks = (long)project_strips(grid) * n_views;
   if (nblocks <= 0) return hipSuccess;
-  if (nblocks > 0x7fffffffL || grid.nx > 65536 || grid.ny > 65536) return hipErrorInvalidValue;
+  if (nblocks > (long)max_blocks(64) || grid.nx > 65536 || grid.ny > 65536) return hipErrorInvalidValue;
   BpGrid g = grid;  // the first quadrant or half
   if (orbit == 4) g.x1 = (g.nx + 1) / 2;
   if (orbit > 1) g.ny = (g.ny + 1) / 2;
@@ -2417,7 +2423,7 @@ hipError_t launch_project_rows(const float* volT, const BpView* views, int view0
   const size_t slot = sizeof(float) * orbit * (2 * kRowPad + grid.nz);
   const int depth = (int)std::min<size_t>(6, std::max<size_t>(2, 12 * 1024 / slot));
   const long nblocks = (long)n_strips * chunks * 8 * ((base_views + 7) / 8);
-  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+  if (nblocks > (long)max_blocks(64)) return hipErrorInvalidValue;
 #define MONTE_PR(NQ, JJ, RR)                                                                                   \
   hipLaunchKernelGGL((project_rows_kernel<NQ, JJ, RR>), dim3((unsigned)nblocks), dim3(64), slot * depth, s,    \
                      volT, views, view0, n_strips, base_views, grid, filt_pad, row0, row_end, chunks, depth,   \
@@ -2447,7 +2453,7 @@ hipError_t launch_project(const float* volT, const BpView* views, int view0, int
   // (8 XCDs x the largest view share x strips; blocks past an XCD's share return)
   const long nblocks = (long)n_strips * 8 * ((nviews_chunk + 7) / 8);
   if (nblocks <= 0) return hipSuccess;
-  if (nblocks > 0x7fffffffL) return hipErrorInvalidValue;
+  if (nblocks > (long)max_blocks(64)) return hipErrorInvalidValue;
   if (lds_r0 < 0 || lds_rows < 1 || lds_r0 + lds_rows > grid.rows) return hipErrorInvalidValue;
   const size_t lds = sizeof(float) * ((size_t)lds_rows * kStripP + kTrash);
   if (lds > 64 * 1024) return hipErrorInvalidValue;

@@ -182,3 +182,19 @@ def test_invalid_arguments_are_reported(ctx):
     out = fdk(_t(np.ones(g.proj_shape, np.float32)), g, ctx)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
+
+
+def test_projector_refuses_more_strips_than_a_launch_holds(ctx):
+    """66000 views of 1016 columns: more waves than the 2^32 threads of one launch are an error."""
+    import torch
+
+    from monte_amd import _lib
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk_project
+
+    geom = G.small(n_views=66000).replace(nu=1016, nv=1, nx=2, ny=2, nz=2)
+    assert geom.n_views * (geom.nu + 4) * 64 > 2**32
+    with pytest.raises(_lib.MonteError):
+        fdk_project(_t(np.ones(geom.vol_shape, np.float32)), geom, ctx)
+    out = fdk_project(_t(np.ones(geom.vol_shape, np.float32)), geom.replace(n_views=8), ctx)
+    assert torch.isfinite(out).all() and bool((out != 0).any())
