@@ -958,7 +958,7 @@ __device__ inline void copy_to_lds(const char* row, uint32_t off, float* dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :
                : "s"(__builtin_amdgcn_readfirstlane((int)at)), "v"(off), "s"(row)
-               : "memory");
+               : "memory", "m0");
 }
 
 // min(max(x, lo), hi) in one instruction
