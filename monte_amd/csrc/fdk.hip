@@ -953,6 +953,8 @@ struct PatchLayout {
 // cannot tell the two patches apart and would wait for the copies of one
 // before it reads the other; there is no result register, and the caller waits
 // (vmcnt) and meets the other waves before anything reads the words.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (that M0 is a reserved register)
 __device__ inline void copy_to_lds(const char* row, uint32_t off, float* dst) {
   const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)dst;
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
@@ -960,6 +962,7 @@ __device__ inline void copy_to_lds(const char* row, uint32_t off, float* dst) {
                : "s"(__builtin_amdgcn_readfirstlane((int)at)), "v"(off), "s"(row)
                : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // min(max(x, lo), hi) in one instruction
 __device__ inline int clamp_i(int x, int lo, int hi) {
