@@ -1483,6 +1483,23 @@ int monte_fdk_graph(monte_ctx* c, const monte_geom* g, const float* proj, float*
   return MONTE_OK;
 }
 
+// -------------------------------------------------- routes (internal, for tests)
+// fdk_routes of a geometry; needs no device.  t null: the default tuning.
+int monte_internal_fdk_routes(const monte_geom* g, const monte_tuning* t, int32_t* out) {
+  if (!g || !out) return MONTE_ERR_INVALID;
+  const int rc = check_geom(nullptr, g, true);
+  if (rc) return rc;
+  const monte_tuning tune = t ? *t : default_tuning();
+  const BpGrid grid = compute_bp_grid(*g);
+  const int n = tune.bp_view_chunk > 0 ? std::min(tune.bp_view_chunk, g->n_views) : g->n_views;
+  std::vector<BpView> views;
+  compute_bp_views(*g, views);
+  int r0, rows;
+  projector_rows(views, 0, n, grid, r0, rows);
+  fdk_routes(grid, compute_bp_reach(*g, grid), n, r0, rows, tune, out);
+  return MONTE_OK;
+}
+
 // ------------------------------------------------------------ end to end
 int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, const monte_mc_cfg* cfg,
                    const monte_e2e_buffers* buf, int use_graph, monte_mc_stats* stats) {

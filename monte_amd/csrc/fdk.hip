@@ -1364,25 +1364,61 @@ static BpPlan bp_plan(const BpGrid& g, const BpReach& r) {
   return {0, 1, 8, 1};
 }
 
+// The kernel and tile shape of one launch of a backprojection; false: the call cannot run.
+struct BpLaunch {
+  BpPlan plan;
+  int zc, tile_x, tiles_x, tiles_y;
+  int rows, cols;  // of a patch
+  long blocks;     // (0: straight from memory)
+};
+static bool bp_launch(const BpGrid& grid, const BpReach& reach, int nviews_chunk, const monte_tuning& t, BpLaunch& L) {
+  // taps are addressed by 32-bit offsets with a 24-bit row multiply
+  if (grid.pitch >= (1 << 23) || (long long)grid.rows * grid.pitch * 4 >= (1LL << 32)) return false;
+  if (t.bp_tile_x > 0 && 256 % t.bp_tile_x) return false;
+  int zc = t.bp_zchunk > 0 ? t.bp_zchunk : 16;
+  if (zc != 4 && zc != 8 && zc != 16) return false;
+  L = BpLaunch{};
+  BpPlan& plan = L.plan;
+  plan = bp_plan(grid, reach);
+  if (plan.orbit > 1 && nviews_chunk != grid.n_views) {  // orbits need the whole turn
+    int rows, cols;
+    patch_bounds(grid, reach, 16, 16, plan.zc, rows, cols);
+    plan = {patch_fits<1>(rows, cols, 1) ? 1 : 0, 1, plan.zc, 1};
+  }
+  if (plan.orbit == 0) return true;
+  const int nq = plan.orbit, groups = plan.groups, stack = plan.stack;
+  zc = zc == 16 ? std::min(32, plan.zc) : std::min(zc, plan.zc);  // (the largest tuned chunk stands for 32 too)
+  const int nx = nq == 4 ? (grid.nx + 1) / 2 : grid.x1 - grid.x0, ny = nq > 1 ? (grid.ny + 1) / 2 : grid.ny;
+  // whole 8 x 8 sub-tiles, one per wave
+  int tile_x = stack == 1 ? std::min(32, std::max(8, (int)t.bp_tile_x)) : 8;
+  auto blocks_of = [&](int tx, int z) {
+    const int ty = 256 / (tx * stack);
+    return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((grid.nz + z * stack - 1) / (z * stack));
+  };
+  patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, L.rows, L.cols);
+  const long most_blocks = (long)max_blocks(256 * groups);
+  if (!patch_fits(nq, L.rows, L.cols, groups) || blocks_of(tile_x, zc) > most_blocks) {  // not the tuned shape: the default
+    tile_x = stack == 1 ? 16 : 8;
+    zc = plan.zc;
+    patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, L.rows, L.cols);
+  }
+  L.zc = zc;
+  L.tile_x = tile_x;
+  const int tile_y = 256 / (tile_x * stack);
+  L.tiles_x = (nx + tile_x - 1) / tile_x;
+  L.tiles_y = (ny + tile_y - 1) / tile_y;
+  L.blocks = blocks_of(tile_x, zc);
+  return L.blocks <= most_blocks;
+}
+
 hipError_t launch_backproject(const float* filt_pad, const BpView* views, int view0, int nviews_chunk,
                               const BpGrid& grid, const BpReach& reach, float* vol, int accumulate,
                               const monte_tuning& t, hipStream_t s) {
-  // taps are addressed by 32-bit offsets with a 24-bit row multiply
-  if (grid.pitch >= (1 << 23) || (long long)grid.rows * grid.pitch * 4 >= (1LL << 32)) return hipErrorInvalidValue;
-  if (t.bp_tile_x > 0 && 256 % t.bp_tile_x) return hipErrorInvalidValue;
-  int zc = t.bp_zchunk > 0 ? t.bp_zchunk : 16;
-  if (zc != 4 && zc != 8 && zc != 16) return hipErrorInvalidValue;
+  BpLaunch L;
+  if (!bp_launch(grid, reach, nviews_chunk, t, L)) return hipErrorInvalidValue;
   const int ncx = grid.x1 - grid.x0;
   if (ncx <= 0 || grid.ny <= 0 || grid.nz <= 0 || nviews_chunk <= 0) return hipSuccess;
-  BpPlan plan = bp_plan(grid, reach);
-  if (plan.orbit > 1 && nviews_chunk != grid.n_views) {  // orbits need the whole turn
-    int rows, cols;
-    const int tx = plan.stack == 1 ? 16 : 8;
-    patch_bounds(grid, reach, tx, 256 / (tx * plan.stack), plan.zc * plan.stack, rows, cols);
-    plan = {patch_fits<1>(rows, cols, 1) ? 1 : 0, 1, plan.zc, plan.stack};
-  }
-  const int nq = plan.orbit, groups = plan.groups, stack = plan.stack;
-  zc = zc == 16 ? std::min(32, plan.zc) : std::min(zc, plan.zc);  // (the largest tuned chunk stands for 32 too)
+  const int nq = L.plan.orbit, groups = L.plan.groups, stack = L.plan.stack, zc = L.zc, rows = L.rows;
   if (nq == 0) {
     // 8 voxels a lane (16 spill registers in the bp3d20 preset), and waves per block
     // until about 4 per SIMD are in flight
@@ -1405,33 +1441,15 @@ hipError_t launch_backproject(const float* filt_pad, const BpView* views, int vi
 #undef MONTE_BP
     return hipGetLastError();
   }
-  const int nx = nq == 4 ? (grid.nx + 1) / 2 : ncx, ny = nq > 1 ? (grid.ny + 1) / 2 : grid.ny;
-  // whole 8 x 8 sub-tiles, one per wave
-  int tile_x = stack == 1 ? std::min(32, std::max(8, (int)t.bp_tile_x)) : 8;
-  auto blocks_of = [&](int tx, int z) {
-    const int ty = 256 / (tx * stack);
-    return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((grid.nz + z * stack - 1) / (z * stack));
-  };
-  int rows, cols;
-  patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
-  const long most_blocks = (long)max_blocks(256 * groups);
-  if (!patch_fits(nq, rows, cols, groups) || blocks_of(tile_x, zc) > most_blocks) {  // not the tuned shape: the default
-    tile_x = stack == 1 ? 16 : 8;
-    zc = plan.zc;
-    patch_bounds(grid, reach, tile_x, 256 / (tile_x * stack), zc * stack, rows, cols);
-  }
-  const int tiles_x = (nx + tile_x - 1) / tile_x, tile_y = 256 / (tile_x * stack), tiles_y = (ny + tile_y - 1) / tile_y;
-  const long nblocks = blocks_of(tile_x, zc);
-  if (nblocks > most_blocks) return hipErrorInvalidValue;
   // the groups' patches, which the sums of a group go through at the end
   auto lds_of = [&](int row_words, int sums) {
     const size_t patch = (size_t)2 * rows * row_words * groups;
     return sizeof(float) * (groups > 1 ? std::max(patch, (size_t)sums * 256) : patch);
   };
 #define MONTE_BP(ZC, NQ, ZEROS)                                                                                \
-  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)nblocks), dim3(256 * groups), \
+  hipLaunchKernelGGL((backproject_kernel<ZC, NQ, ZEROS>), dim3((unsigned)L.blocks), dim3(256 * groups), \
                      lds_of(PatchLayout<NQ>::kRS, NQ * ZC), s, filt_pad, views, view0, nviews_chunk,          \
-                     grid, vol, accumulate, tile_x, tiles_x, tiles_y, rows, reach.turn, stack)
+                     grid, vol, accumulate, L.tile_x, L.tiles_x, L.tiles_y, rows, reach.turn, stack)
 #define MONTE_BP_Z(NQ, ZEROS)                                                                                    \
   switch (zc) {                                                                                                \
     case 4: MONTE_BP(4, NQ, ZEROS); break;                                                                            \
@@ -2408,31 +2426,60 @@ int project_orbit(const BpGrid& g, const BpReach& r, const monte_tuning& t) {
   return r.turn != 0 && waves >= 40000 ? 4 : (r.half && waves >= 6000 ? 2 : 1);
 }
 
+// Detector rows of a launch by rows, as blocks of 64 x nr rows, and the voxels a row takes of a column.
+struct RowLaunch {
+  int row0, row_end, chunks, nr, J;
+};
+static bool row_launch(const BpGrid& grid, const BpReach& reach, int lds_r0, int lds_rows, RowLaunch& L) {
+  // detector rows that the window of padded rows holds
+  L.row0 = std::max(lds_r0 - kPadLo, 0);
+  L.row_end = std::min(lds_r0 - kPadLo + lds_rows, grid.nv);
+  // a block fetches and sets up its columns once for all its rows: few chunks
+  const int rows64 = std::max(0, (L.row_end - L.row0 + 63) / 64);
+  L.chunks = (rows64 + 5) / 6;
+  L.nr = L.chunks ? (rows64 + L.chunks - 1) / L.chunks : 0;
+  const double lo = reach.svk * std::fabs(grid.gsz) / (reach.sod + reach.rad);
+  L.J = lo >= 1.0 ? 2 : 3;
+  return lo >= 2.0 / 3.0;  // (project_orbit)
+}
+
+void fdk_routes(const BpGrid& grid, const BpReach& reach, int nviews_chunk, int lds_r0, int lds_rows,
+                const monte_tuning& t, int32_t out[kRouteWords]) {
+  std::fill(out, out + kRouteWords, 0);
+  BpLaunch B;
+  out[0] = -1;
+  if (bp_launch(grid, reach, nviews_chunk, t, B)) {
+    const int32_t b[8] = {B.plan.orbit, B.plan.groups, B.zc, B.plan.stack, B.tile_x, B.rows, B.cols, (int32_t)B.blocks};
+    std::copy(b, b + 8, out);
+  }
+  RowLaunch L;
+  out[8] = project_orbit(grid, reach, t);
+  if (out[8] && row_launch(grid, reach, lds_r0, lds_rows, L)) {
+    out[9] = L.chunks;
+    out[10] = L.nr;
+    out[11] = L.J;
+  }
+}
+
 hipError_t launch_project_rows(const float* volT, const BpView* views, int view0, int nviews_chunk, const BpGrid& grid,
                                const BpReach& reach, int orbit, float* filt_pad, int lds_r0, int lds_rows,
                                const uint32_t* plan_offs, const uint32_t* plan_list, hipStream_t s) {
   if (nviews_chunk <= 0) return hipSuccess;
   if (orbit != 1 && nviews_chunk != grid.n_views) return hipErrorInvalidValue;
-  // detector rows that the window of padded rows holds
-  const int row0 = std::max(lds_r0 - kPadLo, 0), row_end = std::min(lds_r0 - kPadLo + lds_rows, grid.nv);
-  if (row_end <= row0) return hipSuccess;
-  const int base_views = nviews_chunk / orbit, n_strips = project_strips(grid);
-  // a block fetches and sets up its columns once for all its rows: few chunks
-  const int rows64 = (row_end - row0 + 63) / 64;
-  const int chunks = (rows64 + 5) / 6, nr = (rows64 + chunks - 1) / chunks;
-  const double lo = reach.svk * std::fabs(grid.gsz) / (reach.sod + reach.rad);
-  if (lo < 2.0 / 3.0) return hipErrorInvalidValue;  // (project_orbit)
-  const int J = lo >= 1.0 ? 2 : 3;
+  RowLaunch L;
+  if (!row_launch(grid, reach, lds_r0, lds_rows, L)) return hipErrorInvalidValue;
+  if (L.row_end <= L.row0) return hipSuccess;
+  const int base_views = nviews_chunk / orbit, n_strips = project_strips(grid), chunks = L.chunks, J = L.J;
   const size_t slot = sizeof(float) * orbit * (2 * kRowPad + grid.nz);
   const int depth = (int)std::min<size_t>(6, std::max<size_t>(2, 12 * 1024 / slot));
   const long nblocks = (long)n_strips * chunks * 8 * ((base_views + 7) / 8);
   if (nblocks > (long)max_blocks(64)) return hipErrorInvalidValue;
 #define MONTE_PR(NQ, JJ, RR)                                                                                   \
   hipLaunchKernelGGL((project_rows_kernel<NQ, JJ, RR>), dim3((unsigned)nblocks), dim3(64), slot * depth, s,    \
-                     volT, views, view0, n_strips, base_views, grid, filt_pad, row0, row_end, chunks, depth,   \
+                     volT, views, view0, n_strips, base_views, grid, filt_pad, L.row0, L.row_end, chunks, depth, \
                      plan_offs, plan_list, reach.turn)
 #define MONTE_PR_R(NQ, JJ)                                                                                     \
-  switch (nr) {                                                                                                \
+  switch (L.nr) {                                                                                              \
     case 1: MONTE_PR(NQ, JJ, 1); break;                                                                        \
     case 2: MONTE_PR(NQ, JJ, 2); break;                                                                        \
     case 3: MONTE_PR(NQ, JJ, 3); break;                                                                        \

@@ -315,6 +315,12 @@ void* noalloc_scratch(int device);
 constexpr uint64_t max_blocks(int threads) { return 0xffffffffull / (unsigned)threads; }
 
 // FDK (fdk.hip)
+// What a scan's backprojection and projection run, for tests: columns of an orbit (0: straight from
+// memory, -1: refused), groups, voxels a thread, stack, tile_x, patch rows and columns, blocks (low
+// 32 bits); the row projector's orbit (0: by voxels), blocks of rows, rows / 64 of a block, voxels a row.
+constexpr int kRouteWords = 12;
+void fdk_routes(const BpGrid& grid, const BpReach& reach, int nviews_chunk, int lds_r0, int lds_rows,
+                const monte_tuning& t, int32_t out[kRouteWords]);
 hipError_t launch_fill(float* p, float v, size_t n, hipStream_t s);
 hipError_t launch_pad_copy(const float* filt, float* filt_pad, int n_views, int nu, int nv, int pitch, int rows,
                            hipStream_t s);
