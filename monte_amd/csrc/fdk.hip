@@ -1538,14 +1538,15 @@ struct SlabRanges {
   double q0, q1, id0, id1;  // edge parameters and reciprocal denominators
   double o0, ios;           // voxel index = (t - o0) * ios along the slab
   int n;                    // voxels along the slab
-  bool whole;               // an edge runs parallel to the slabs: take every column
+  bool whole;               // an edge, or a direction between them, runs along the slabs: take every column
 
   __device__ void init(double s_lo, double s_hi, const BpView& c, bool x_slabs, const BpGrid& g) {
     q0 = (s_lo - c.su0) / c.suk;
     q1 = (s_hi - c.su0) / c.suk;
     const double a2 = x_slabs ? c.ay : c.ax, c2 = x_slabs ? c.cy : c.cx;
     const double d0 = a2 - q0 * c2, d1 = a2 - q1 * c2;
-    whole = fabs(d0) < 1e-12 || fabs(d1) < 1e-12;
+    // (of opposite signs: a direction between the edges, 45 degrees or more off the axis, runs along the slabs)
+    whole = fabs(d0) < 1e-12 || fabs(d1) < 1e-12 || (d0 < 0.0) != (d1 < 0.0);
     id0 = 1.0 / d0;
     id1 = 1.0 / d1;
     o0 = x_slabs ? g.gy0 : g.gx0;

@@ -201,3 +201,20 @@ def test_projector_in_chunks_of_views(ctx, oracle, name, chunks):
             assert rel_max(got, ref) < TOL and rel_l2(got, ref) < TOL
     finally:
         ctx.set_tuning(**saved)
+
+
+@pytest.mark.parametrize("views,nx,ny", [(8, 4, 4), (9, 31, 17), (30, 12, 40)])
+def test_projector_of_wide_fans(ctx, oracle, views, nx, ny):
+    """A volume close to the source's orbit under a detector of 80 degrees either side: strips whose rays
+    run along the slabs that the column lists are made of."""
+    from monte_amd import geometry as G
+    from monte_amd.fdk import fdk_project
+
+    v = 30.0 / max(nx, ny)
+    g = G.Geometry(n_views=views, nu=24, nv=13, nx=nx, ny=ny, nz=5, sod=24.0, sdd=33.0, du=17.0, dv=12.5, vx=v, vy=v,
+                   vz=2.3)
+    y = np.random.default_rng(views).standard_normal(g.vol_shape).astype(np.float32)
+    ref = oracle.fdk_std_backproject_T(oracle_geom(oracle, g), y)
+    got = fdk_project(_t(y), g, ctx).cpu().numpy()
+    print(views, rel_max(got, ref), rel_l2(got, ref))
+    assert rel_max(got, ref) < TOL and rel_l2(got, ref) < TOL
