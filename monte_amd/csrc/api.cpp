@@ -44,7 +44,7 @@ namespace {
 
 constexpr int kSlotFwd = 0, kSlotAdj = 1, kSlotMc = 2, kSlotConst = 3, kSlotStageA = 4, kSlotStageB = 5,
               kSlotTuneA = 6, kSlotTuneB = 7, kSlotVolT = 8,
-              kSlotPlan = 10, kSlotE2E = 11, kSlotRay = 12, kSlotE2ERay = 13;
+              kSlotPlan = 9, kSlotE2E = 10, kSlotRay = 11, kSlotE2ERay = 12;
 
 constexpr size_t kHostCounters = 2048;  // sets of counters copied to pinned host memory (160 KB)
 
@@ -1192,7 +1192,6 @@ int monte_primary_exact(monte_ctx* c, const monte_geom* g, const monte_phantom* 
     P.vox[a] = vox[a];
     P.n[a] = n[a];
     P.b0[a] = org[a] - 0.5 * n[a] * vox[a];
-    P.b1[a] = org[a] + 0.5 * n[a] * vox[a];
   }
   P.nu = g->nu; P.nv = g->nv; P.n_views = g->n_views;
   // the descriptor of the phantom's box, the FP64 view table and the bins, in the MC slot by one copy
@@ -1353,12 +1352,12 @@ int monte_autotune(monte_ctx* c, int what, const monte_geom* g, const monte_phan
   if (what & 2) {
     int rc = check_geom(c, g, true);
     if (rc) return rc;
-    // time a slice of views on scratch buffers
-    monte_geom tg = *g;
+    // every view on scratch buffers: orbits of columns need the whole scan
+    const monte_geom& tg = *g;
     const float* taps;
     const BpView* views;
     if ((rc = ensure_constants(c, tg, &taps, &views))) return rc;
-    const int nviews = g->n_views;  // the whole scan: orbits of four views need it
+    const int nviews = g->n_views;
     float* pad = (float*)workspace(c, kSlotFwd, padded_elems(tg) * sizeof(float));
     float* vol = (float*)workspace(c, kSlotTuneB, vol_elems(tg) * sizeof(float));
     if (!pad || !vol) return fail(c, MONTE_ERR_NOMEM, "tuning buffers");

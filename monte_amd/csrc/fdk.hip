@@ -263,11 +263,12 @@ __global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 
     const float2* __restrict__ twid, const float2* __restrict__ spec, FilterParams fp, int tiles, int wrap) {
   constexpr int N = R1 * M, P = 64 / M, S = R1 / M, kHalf = N / 2, kStride = fft_stride(R1, M);
   // tables in LDS (from L1, a block's twiddles and spectrum took as long as its transforms:
-  // 0.45 ms where it is 0.29), without the spectrum where 8 waves would not fit
+  // 0.45 ms where it is 0.29), without the spectrum where 8 waves would not fit (transposed rows
+  // of more than 512)
   constexpr bool kSpLds = N <= 1024;
-  // blocks take tiles in turn, loading the next one's samples while they write: 0.40 -> 0.27 ms
+  // the transpose's blocks take tiles in turn, loading the next one's samples while they write: 0.40 -> 0.27 ms
   // for the transpose at 360 x 512^2; forward, 0.29 -> 0.44 (more waits at barriers)
-  constexpr bool kLoop = TRANS || N > 1024, kAhead = TRANS && R1 <= 32;
+  constexpr bool kAhead = TRANS && R1 <= 32;
   extern __shared__ float sm[];
   const int waves = blockDim.x >> 6, rows_b = 2 * P * waves, rshift = 31 - __builtin_clz(rows_b);
   float2* const twl = (float2*)sm;
@@ -282,8 +283,10 @@ __global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 
       if (kSpLds) spl[i] = spec[i];
     }
   };
-  if (kLoop) tables();
-  if (TRANS) __syncthreads();
+  if (TRANS) {
+    tables();
+    __syncthreads();
+  }
   // XCD x takes an eighth of the tiles, as xcd_tile deals them: a view's lines meet in one L2
   const int xcd = blockIdx.x & 7, q8 = (tiles * fp.n_views) >> 3, r8 = (tiles * fp.n_views) & 7;
   const int tile0 = xcd * q8 + min(xcd, r8), tile_end = tile0 + q8 + (xcd < r8 ? 1 : 0);
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 
   if (kAhead) load(tile, lane0, wave0);
   for (;;) {
     int lane = lane0, wave = wave0;
-    if (kLoop) {  // opaque, or the loop's addresses and weights are kept in registers, and spilt
+    if (TRANS) {  // opaque, or the loop's addresses and weights are kept in registers, and spilt
       asm volatile("" : "+v"(lane));
       asm volatile("" : "+v"(wave));
     }
@@ -348,8 +351,10 @@ __global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 
       }
       wave_lds_sync();
     }
-    if (!kLoop) tables();
-    if (!TRANS) __syncthreads();
+    if (!TRANS) {
+      tables();
+      __syncthreads();
+    }
 
     float yr[R1], yi[R1];  // at the end, filtered samples m + M n1 in the first half
     if (v < nv) {
@@ -599,8 +604,7 @@ __global__ __launch_bounds__(R1 == 64 ? 512 : 256, R1 == 64 ? 2 : (R1 == 32 ? 3 
         const int c = i % fp.pitch;
         if (!wrap || c < kPadLo || view == fp.n_views - 1) dst[(size_t)nv * fp.pitch - kPadLo + i] = 0.f;
       }
-    if (!kLoop || (tile += step) >= tile_end) return;
-    __syncthreads();
+    return;
   }
 }
 
@@ -624,7 +628,7 @@ static hipError_t launch_filter_fft(const float* in, float* out, const float* ta
   const size_t lds = sizeof(float) * ((n <= 1024 ? 4 : 2) * n + (size_t)(64 / m) * waves * fft_stride(n / m, m));
   long blocks = (long)tiles * fp.n_views;
   if (!TRANS && blocks > (long)max_blocks(64 * waves)) return hipErrorInvalidValue;
-  if (TRANS || n > 1024) blocks = std::min<long>(blocks, 256 * std::min<long>(160 * 1024 / lds, 16 / waves));
+  if (TRANS) blocks = std::min<long>(blocks, 256 * std::min<long>(160 * 1024 / lds, 16 / waves));
 #define MONTE_FFT(R, L)                                                                                        \
   hipLaunchKernelGGL((filter_fft_kernel<R, L, TRANS>), dim3((unsigned)blocks), dim3(64 * waves), lds, s, in,   \
                      out, taps, tables, tables + n, fp, tiles, wrap)
@@ -855,9 +859,10 @@ __device__ inline ColumnCore column_core(const BpView& c, double X, double Y, fl
 }
 
 // The v coordinate of voxel z is formed from a base taken in the middle of its
-// 16-aligned group, whatever the thread's z-chunk, so every chunking and tile
+// 16-aligned group, whatever the thread's z-chunk, so every tuned z-chunk and tile
 // shape evaluates the same floating-point expression for each voxel and the
-// volume is bitwise independent of the launch tuning.
+// volume is bitwise independent of them.  (Launches of part of the views add the
+// same terms in another order, and take orbits apart.)
 constexpr int kZBase = 16;
 constexpr int kZMid = kZBase / 2;  // the base voxel of a group of 16: dsv's rounding is multiplied by 8 at most
 

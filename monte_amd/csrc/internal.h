@@ -201,7 +201,7 @@ static_assert(sizeof(McPrep) <= 256, "the static scratch of the allocation-free 
 // FP64 ray geometry of the exact primary estimator.
 struct PrimaryGeom {
   double sod, sdd, un0, u_step, vn0, v_step;
-  double b0[3], b1[3], vox[3];
+  double b0[3], vox[3];
   int n[3];
   int nu, nv, n_views;
 };
@@ -257,11 +257,10 @@ struct monte_ctx {
   //   2 MC descriptors                    3 FDK constants (taps + per-view coefficients)
   //   4..7 staging for host-pointer mode and tuning scratch
   //   8 z-fastest copy of the volume for the matched projector
-  //   9 unused
-  //  10 column lists of the matched projector (per geometry)
-  //  11 end-to-end step: MC descriptors and loss partial sums
-  //  12 first-flight label sets of MC launches   13 those of the end-to-end step
-  static constexpr int kSlots = 14;
+  //   9 column lists of the matched projector (per geometry)
+  //  10 end-to-end step: MC descriptors and loss partial sums
+  //  11 first-flight label sets of MC launches   12 those of the end-to-end step
+  static constexpr int kSlots = 13;
   void* ws[kSlots] = {};
   size_t ws_size[kSlots] = {};
 
