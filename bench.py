@@ -27,7 +27,9 @@ sys.path.insert(0, ROOT)
 
 PEAK_LANE_OPS = 256 * 64 * 2.4e9  # MI355X FP32 VALU: 256 CUs x 64 lanes x 2.4 GHz, one op per lane per clock
 PEAK_HBM = 8.0e12
-BP_OPS = 18       # FP32 VALU ops per backprojection voxel-update (algorithmic)
+# FP32 VALU ops per backprojection voxel-update: 5 of the taps, 10 of the sample's coordinates and 70 / 16
+# of the column's set-up, which the four columns of a quarter-turn orbit share
+BP_OPS = 5 + (10 + 70 / 16) / 4
 MC_OPS_STEP, MC_OPS_INT, MC_OPS_HIST = 40, 150, 60  # per Woodcock step, per interaction, per history
 
 
@@ -183,7 +185,8 @@ def main():
         "roofline_fdk_backproject": {
             "bound": "valu", "achieved": BP_OPS * updates / fdk_s / 1e12, "peak": PEAK_LANE_OPS / 1e12,
             "unit": "Tlane-op/s", "frac": BP_OPS * updates / fdk_s / PEAK_LANE_OPS,
-            "note": "whole FDK time (filter + backprojection) against the backprojection roof",
+            "note": "whole FDK time (filter + backprojection) against the backprojection roof; 8.6 lane-ops per "
+                    "update, the geometry shared by the four columns of an orbit",
         },
         "tuning": tuning,
         "tuning_default": tuning_default,

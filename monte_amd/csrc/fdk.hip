@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void filter_fwd_mfma_kernel(const float* __res
 // Rows that are not finite are summed directly.
 //   Bound by VALU instructions: 1600 of a wave's 2750 (two pairs of 512) are the four
 // transforms, 400 twiddles and spectrum, 450 the weighted tile.  360 views of 512^2 take
-// 0.285 ms and 0.271 transposed, for 0.94 and 0.87 as products with the taps' Toeplitz matrix
+// 0.287 ms and 0.265 transposed, for 0.94 and 0.87 as products with the taps' Toeplitz matrix
 // (103 TFLOP/s of fp32 matrix instructions, of 147 in a large product); 325^2 takes 0.17 ms
 // for 0.50, 1024 x 768 transposed 1.4 for 4.6.  Rows that just miss a power of two gain
 // least: 180 views of 600 x 512 transposed, with the copy in, 0.52 ms for 0.85.
@@ -2193,7 +2193,7 @@ hipError_t launch_project_plan(const BpView* views, int n_views, const BpGrid& g
 //   NQ > 1: as the backprojector, the NQ columns of an orbit share all of a row's
 // geometry; the wave forms the strip in all NQ views that are a part of a turn
 // apart, taking the lists of first columns of each in turn.
-// Per row and column: 12 / NQ VALU instructions of geometry, 2 J - 1 of sums and 2
+// Per row and column: (7 + 7 J / 2) / NQ VALU instructions of geometry, 2 J - 1 of sums and 2
 // multiply-adds, J reads of LDS.  The kernel this one replaces in these cases (below:
 // lanes own voxels, two read-add-writes of LDS per voxel) took 9.97 ms at 325^3 ->
 // 360 views of 512^2.
@@ -2406,21 +2406,21 @@ __global__ __launch_bounds__(64) void project_rows_kernel(const float* __restric
 // voxel kernel above.  The rule takes the standard preset's zero guard cells and the
 // automatic tuning, and these sizes (adjoint with its filter, ms, by rows : by
 // voxels):
-//  - between 0.8 and 1.9 rows a voxel.  Below, a row takes more than three voxels (0.076
-//    against 0.085 at 65^3, but 0.97 : 0.89 at 193^3, 0.77 rows a voxel), above most rows
-//    of a column see one voxel (0.46 : 0.37 at 97^3, 1.81 rows a voxel).  Launches of up to
-//    5000 waves wait for a wave's chain of read-add-writes by voxels, and gain up to 2.6
-//    rows a voxel (0.042 : 0.051 at 33^3 / 30 views, 0.068 : 0.076 at 49^3 / 36 views, 2 rows).
+//  - between 0.8 and 1.9 rows a voxel.  Below, a row takes more than three voxels (0.090
+//    against 0.085 at 65^3, 1.10 : 1.09 at 193^3, from 0.65 rows a voxel), above most rows
+//    of a column see one voxel (0.50 : 0.39 at 97^3, up to 2.3 rows a voxel).  Launches of up
+//    to 5000 waves wait for a wave's chain of read-add-writes by voxels, and gain up to 2.6
+//    rows a voxel (0.046 : 0.055 at 33^3 / 30 views, 0.072 : 0.078 at 49^3 / 36 views, 2.5 rows).
 //  - a column within 384 rows: more take a second wave that reads all columns again
-//    (1.69 : 2.57 at 225^3, 448 rows).
+//    (4.5 : 3.1 at 225^3, 434 rows).
 //  - a volume of up to 48 MB.  Larger ones leave no columns for the next view in the
-//    L2s: a launch reads the volume once per view, at 5.2 TB/s (137 MB x 360 views at
-//    325^3: 11.5 : 9.97, since the voxel kernel keeps columns).
-// Within them: 0.050 : 0.071 at 49^3 (36 views of 64^2), 0.117 : 0.172 at 65^3 (90 of
-// 96^2), 0.26 : 0.34 at 97^3 (90 of 160^2), 0.77 : 1.00 at 129^3 (180 of 192^2), 1.2 :
-// 1.54 at 161^3 (180 of 256^2), 2.75 : 3.00 at 225^3 (180 of 384^2).
-//   Orbits save geometry and take waves: of 4 from 10000 waves (2.75 : 3.10 with 2 at
-// 17000, 0.72 : 0.68 at 7200), of 2 from 3000 (0.117 : 0.131 with 1 at 4300, 0.054 : 0.050
+//    L2s: a launch reads the volume once per view, at 5.2 TB/s (325^3 / 360 views of 512^2, the
+//    projection alone, without the second wave: 11.5 : 9.97, since the voxel kernel keeps columns).
+// Within them: 0.051 : 0.072 at 49^3 (36 views of 64^2), 0.128 : 0.176 at 65^3 (90 of
+// 96^2), 0.29 : 0.34 at 97^3 (90 of 160^2), 0.82 : 1.00 at 129^3 (180 of 192^2), 1.24 :
+// 1.52 at 161^3 (180 of 256^2), 2.79 : 2.99 at 225^3 (180 of 384^2).
+//   Orbits save geometry and take waves: of 4 from 10000 waves (in FP32 weights 2.75 : 3.10 with
+// 2 at 17000, 0.72 : 0.68 at 7200), of 2 from 3000 (0.117 : 0.131 with 1 at 4300, 0.054 : 0.050
 // at 1150).
 int project_orbit(const BpGrid& g, const BpReach& r, const monte_tuning& t) {
   const double lo = r.svk * std::fabs(g.gsz) / (r.sod + r.rad), hi = r.svk * std::fabs(g.gsz) / (r.sod - r.rad);

@@ -456,9 +456,10 @@ __device__ inline uint32_t label_raw(uint32_t i, const JT& J) {
 // A parked branch runs once at least this many lanes wait for it (or nothing
 // else can run).  Interactions wait for 32 lanes: each batch costs a whole
 // Klein-Nishina rejection loop and a flight set-up, so fuller batches pay
-// (at 6 waves per SIMD, 16, 24 and 32 lanes took 96.7, 94.6 and 94.2 ms on the
-// full workload at 1e7 photons per view; on the current kernel 40 and 48 lanes
-// took 86.3 and 103.6 against 83.5 ms, the collided lanes then idling longer).
+// (16, 24, 32, 40 and 48 lanes took 71.6, 69.4, 69.0, 70.9 and 88.0 ms on the full
+// workload at 1e7 photons per view, the collided lanes idling longer past 32; 152.0,
+// 151.4, 150.8, 149.7 and 148.9 on the end-to-end scan at 5e6).  Refills of 8 and 24
+// lanes took 69.4 and 70.9 ms, 151.3 and 149.4.
 constexpr unsigned kInteractBatch = 32;
 constexpr unsigned kRefillBatch = 16;
 

@@ -133,10 +133,11 @@ def test_odd_volume_shapes(ctx, oracle, shape):
     assert abs(b1 - b2) <= 1e-5 * abs(b1)
 
 
-# Scans whose voxels step by 0.5 to 2.5 rows project by detector rows: 4, 3 or 2 voxels a row
-# (steps of at least 1/2, 2/3 and 1), one to five rows a lane and several row blocks, orbits of
-# 4, 2 or 1 columns with odd sides (middle rows, a centre column) and turns either way, columns
-# shorter and longer than a wave, volumes past the detector's edges.
+# Scans whose voxels step by 0.8 to 2.6 rows project by detector rows: 3 or 2 voxels a row (steps
+# below 1 and from there), one to six rows a lane in one block, orbits of 4, 2 or 1 columns with
+# odd sides (middle rows, a centre column) and turns either way, columns shorter and longer than a
+# wave, volumes past the detector's edges.  (4 to 6 rows a lane of orbits, and several blocks of
+# rows: test_gpu_fdk_routes.py.)
 _BY_ROWS = {
     "quarter_even": dict(nx=20, ny=20, nz=30, n_views=88, nu=470),
     "quarter_odd": dict(nx=21, ny=21, nz=65, n_views=84, nu=490, step=1.2),
