@@ -621,12 +621,22 @@ int read_counters(monte_ctx* c, const McPrepared& P, std::vector<McCounters>& cn
   return MONTE_OK;
 }
 
+// Free paths under an infinite majorant have no length, and no collision is accepted: such flights
+// would never end.  (Attenuations are products of densities and table values, both only >= 0.)
+int check_transport(monte_ctx* c, const std::vector<HostJob>& hj) {
+  for (const HostJob& h : hj)
+    for (int e = 0; e < kRows; ++e)
+      if (!std::isfinite(h.tables.mumax[e])) return fail(c, MONTE_ERR_INVALID, "a label's attenuation is not finite");
+  return MONTE_OK;
+}
+
 // Prepares and runs one launch in a device buffer: the context's MC workspace,
 // or `base` (at least mc_layout's total bytes) when the caller provides one.
 int run_mc(monte_ctx* c, std::vector<HostJob>& hj, int block, int blocks_per_cu, float* ms_out,
            std::vector<McCounters>* counters_out, char* base = nullptr, int ray_slot = kSlotRay) {
   McPrepared P;
-  int rc = prepare_mc(c, hj, block, blocks_per_cu, base, P, ray_slot);
+  int rc = check_transport(c, hj);
+  if (!rc) rc = prepare_mc(c, hj, block, blocks_per_cu, base, P, ray_slot);
   hipError_t le = hipSuccess;
   std::vector<McCounters> cnt;
   if (!rc) {
@@ -1525,7 +1535,7 @@ int monte_e2e_step(monte_ctx* c, const monte_geom* g, const monte_phantom* ph, c
     c->e2e_mc_key.clear();
     c->e2e_graph_key.clear();
     std::vector<HostJob> hj(1);
-    if ((rc = build_job(c, g, ph, cfg, hj[0], batch))) return rc;
+    if ((rc = build_job(c, g, ph, cfg, hj[0], batch)) || (rc = check_transport(c, hj))) return rc;
     hj[0].d.primary = b.primary;
     hj[0].d.scatter = b.scatter;
     const size_t need = mc_layout(hj, wants_sets(c, kSlotE2ERay), mc_slots(kSlotE2ERay)).total + kLossBlocks * sizeof(double);

@@ -198,3 +198,27 @@ def test_projector_refuses_more_strips_than_a_launch_holds(ctx):
         fdk_project(_t(np.ones(geom.vol_shape, np.float32)), geom, ctx)
     out = fdk_project(_t(np.ones(geom.vol_shape, np.float32)), geom.replace(n_views=8), ctx)
     assert torch.isfinite(out).all() and bool((out != 0).any())
+
+
+def test_transport_refuses_infinite_attenuation(ctx):
+    """Delta tracking has no free path under an infinite majorant: an error, not a flight without end."""
+    import torch
+
+    from monte_amd import _lib, phantoms
+    from monte_amd import geometry as G
+    from monte_amd.e2e import EndToEnd
+    from monte_amd.mc import McJobSpec, McSettings, mc_batch, mc_project, primary_exact
+    from monte_amd.phantoms import LabelPhantom
+
+    geom = G.small(n_views=4)
+    ok = phantoms.small_phantom()
+    bad = LabelPhantom(ok.labels, ok.voxel, [ok.materials[0], ok.materials[1], (0, np.inf)], ok.origin)
+    s = McSettings(photons_per_view=1000)
+    for call in (lambda: mc_project(bad, geom, s, ctx=ctx),
+                 lambda: mc_batch([McJobSpec(ok, geom, s), McJobSpec(bad, geom, s)], ctx=ctx),
+                 lambda: EndToEnd(bad, geom, s, torch.zeros(geom.vol_shape, device="cuda"), ctx=ctx).step(graph=False)):
+        with pytest.raises(_lib.MonteError) as e:
+            call()
+        assert e.value.code == _lib.ERR_INVALID
+    assert bool(torch.isinf(primary_exact(bad, geom, ctx=ctx)).any())  # the exact primary takes it
+    assert mc_project(ok, geom, s, ctx=ctx)[2]["histories"] == 4000
